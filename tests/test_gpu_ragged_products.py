@@ -77,3 +77,28 @@ def test_convolutions_over_channels_in_partial_tiles(n, c, m, h, w, kernel, tile
               f"naive;tile={tile};mapToThreads=64,8;mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;sharedDepth=7;prefetchShared=1")
     (want,) = tc_oracle.run(B.CONVOLUTION, "convolution", arrays)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,k,n", [(101, 128, 101), (130, 70, 129), (66, 33, 300), (67, 64, 5), (64, 96, 128)])
+@pytest.mark.parametrize("first,second", [("m, r_k", "r_k, {n} - n"), ("{m} - m, r_k", "r_k, n"), ("r_k, {m} - m", "{n} - n, r_k")])
+def test_reversed_subscripts_over_partial_tiles(m, k, n, first, second, half):
+    """The copy of the last tile begins in front of the tensor."""
+    dtype, ty, load = (np.float16, "float16", "float(%s)") if half else (np.float32, "float", "%s")
+    A, Bm = ints((m, k), m + k, dtype), ints((k, n), k + n, dtype)
+    want = A.astype(np.float32) @ Bm.astype(np.float32)
+    stored = [A, Bm]
+    if first.startswith("r_k"):
+        stored = [A.T, Bm.T]
+    dims = [[d.strip() for d in subs.split(",")] for subs in (first, second)]
+    for i, side in enumerate(dims):
+        for axis, sub in enumerate(side):
+            if sub.startswith("{"):
+                stored[i] = np.flip(stored[i], axis)
+    stored = [np.ascontiguousarray(a) for a in stored]
+    subs = [s.format(m=m - 1, n=n - 1) for s in (first, second)]
+    src = (f"def f({ty}(P, Q) A, {ty}(R, S) B) -> (O) {{ O(m, n) +=! {load % f'A({subs[0]})'} * {load % f'B({subs[1]})'}"
+           f" where m in 0:{m}, n in 0:{n}, r_k in 0:{k} }}")
+    for tile in ("64,64,32", "16,32,64"):
+        print(f"reversed {m}x{k}x{n} half={half} A({subs[0]}) B({subs[1]}) tile={tile}", flush=True)
+        assert np.array_equal(run(src, "f", stored, f"naive;tile={tile};mapToThreads=64,8;{TAIL}"), want)

@@ -1,4 +1,6 @@
 """Rules by which the mapper chooses a kernel's form, on the generated source (no GPU)."""
+import re
+
 import pytest
 
 import tensorcomprehensions_amd as tc
@@ -16,3 +18,21 @@ def test_loads_of_one_element_are_one_access(term, staged):
     src = "def f(float(N, K) I) -> (s) { s(n) +=! %s where k in 0:4096 }" % term
     text, _ = mapped(src, "f", [(64, 4100)], "naive;tile=1,0;mapToThreads=256;mapToBlocks=64;matchLibraryCalls=1;useSharedMemory=1")
     assert ("lds0_I" in text) == staged
+
+
+MATRIX = "mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1"
+
+
+@pytest.mark.parametrize("dtype", ["float", "float16"])
+@pytest.mark.parametrize("columns,vectors", [("n", True), ("100 - n", False)])
+def test_no_vector_of_a_copy_begins_in_front_of_its_tensor(dtype, columns, vectors):
+    """100 - n over tiles of 64 points: the second tile's copy starts 27 elements in front of the
+    row, and a vector of four would hold element 0 of the tensor as its last."""
+    load = "%s" if dtype == "float" else "float(%s)"
+    src = f"def f({dtype}(M, K) A, {dtype}(K, N) B) -> (O) {{ O(m, n) +=! {load % 'A(m, r_k)'} * {load % f'B(r_k, {columns})'} where n in 0:101 }}"
+    name = "float32" if dtype == "float" else "float16"
+    text, _ = tc.map_only(src, "f", [ShapeOnly((96, 128), name), ShapeOnly((128, 101), name)], f"naive;tile=64,64,32;{MATRIX}")
+    loads = re.findall(r"pk\d*_B_\[it_\] = (?:__tc::loadBounded|\*|pB\[).*", text)
+    assert loads and all(("x4" in line) == vectors for line in loads)
+    if not vectors:
+        assert all("__tc::tmax(0, " in line or "(unsigned)g1_ < 101u" in line for line in loads)
