@@ -1137,15 +1137,22 @@ bool isStream(const StagePlan& st) {
 // 256 blocks put 32 threads in each of 256 blocks, every one of which walks thousands of tiles).  It
 // gets all the threads of the block in lanes of four, one lane group each, and as many of the blocks
 // as that takes (a residual sum of 6.3 M floats under the naive options: 203 -> 12.5 us).
-HipMappingOptions streamMappingOptions(const HipMappingOptions& given) {
+// The sizes are nominal: a product beyond what the device takes (64 x 64 threads on two loops) is cut.
+uint64_t boundedProduct(const std::array<uint64_t, 3>& sizes, uint64_t most) {
+  uint64_t product = 1;
+  for (uint64_t s : sizes) product = s == 0 ? 0 : product > most / s ? most : product * s;
+  return product;
+}
+HipMappingOptions streamMappingOptions(const HipMappingOptions& given, const DeviceLimits& limits) {
   HipMappingOptions o = given;
-  const uint64_t threads = o.block[0] * o.block[1] * o.block[2];
+  const uint64_t threads = boundedProduct({{o.block[0], o.block[1], o.block[2]}}, limits.maxThreadsPerBlock);
   o.tile(std::vector<uint64_t>{4 * threads}).unroll(4).useSharedMemory(false);
-  o.mapToThreads(threads).mapToBlocks(o.grid[0] * o.grid[1] * o.grid[2]).vectorWidth(4).useReadOnlyCache(true);
+  o.mapToThreads(threads).mapToBlocks(boundedProduct({{o.grid[0], o.grid[1], o.grid[2]}}, std::numeric_limits<int32_t>::max()));
+  o.vectorWidth(4).useReadOnlyCache(true);
   return o;
 }
-bool leavesThreadsOfAStreamUnused(const HipMappingOptions& o, const StagePlan& st) {
-  const uint64_t threads = o.block[0] * o.block[1] * o.block[2];
+bool leavesThreadsOfAStreamUnused(const HipMappingOptions& o, const StagePlan& st, const DeviceLimits& limits) {
+  const uint64_t threads = boundedProduct({{o.block[0], o.block[1], o.block[2]}}, limits.maxThreadsPerBlock);
   uint64_t tile = o.generic.hasTiling && !o.generic.tiling.empty() ? o.generic.tiling[0] : 0;
   if (tile == 0) tile = static_cast<uint64_t>(st.vars[0].extent);
   return threads >= 64 && std::min<uint64_t>(o.block[0], tile / o.vectorWidthValue) < threads;
@@ -1249,7 +1256,7 @@ MappedProgram mapToHip(
   // The fill that precedes a divided sum: all dimensions merged, four elements per thread, 256
   // threads, as many blocks as that takes.
   HipMappingOptions fillOptions = fillMappingOptions(optionsIn);
-  HipMappingOptions streamOptions = streamMappingOptions(optionsIn);
+  HipMappingOptions streamOptions = streamMappingOptions(optionsIn, limits);
   std::vector<const HipMappingOptions*> kernelOptions;
   bool anyThreadReduction = false;
   std::vector<std::unique_ptr<Emitter>> bodies;
@@ -1266,7 +1273,7 @@ MappedProgram mapToHip(
       k.stages.push_back(std::move(b.st));
     }
     // (a definition of one dimension is mapped as its options say)
-    if (!fill && single && raw[groups[gi].stages[0]].first().lhsVars.size() > 1 && isStream(k.stages[0]) && leavesThreadsOfAStreamUnused(optionsIn, k.stages[0])) chosen = &streamOptions;
+    if (!fill && single && raw[groups[gi].stages[0]].first().lhsVars.size() > 1 && isStream(k.stages[0]) && leavesThreadsOfAStreamUnused(optionsIn, k.stages[0], limits)) chosen = &streamOptions;
     const HipMappingOptions& options = *chosen;
     kernelOptions.push_back(chosen);
     k.sharedDepth = single ? k.stages[0].numParallel : groups[gi].depth;

@@ -36,3 +36,14 @@ def test_no_vector_of_a_copy_begins_in_front_of_its_tensor(dtype, columns, vecto
     assert loads and all(("x4" in line) == vectors for line in loads)
     if not vectors:
         assert all("__tc::tmax(0, " in line or "(unsigned)g1_ < 101u" in line for line in loads)
+
+
+@pytest.mark.parametrize("threads,used", [("256,8", 1024), ("64,64", 1024), ("32,32,8", 1024), ("1024,1024", 1024), ("16,15", 240), ("4294967296,4294967296", 1024)])
+def test_streams_take_any_nominal_block(threads, used):
+    """Thread sizes for loops that merging removed are nominal: their product may pass the device's
+    limit (and 64 bits)."""
+    src = "def f(float(N, M) A, float(N, M) B) -> (O) { O(n, m) = A(n, m) + B(n, m) }"
+    for blocks in ("256,256", "4294967296,4294967296"):
+        _, launches = tc.map_only(src, "f", [ShapeOnly((512, 1000))] * 2, f"naive;tile=32,32;mapToThreads={threads};mapToBlocks={blocks}")
+        (grid, block), = launches
+        assert block == (used, 1, 1) and grid == (-(-512 * 1000 // (4 * used)), 1, 1)
