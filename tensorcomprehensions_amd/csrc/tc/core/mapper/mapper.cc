@@ -1136,19 +1136,24 @@ bool isStream(const StagePlan& st) {
 // three loops say little about the one loop that merging left (tile 32, 64 x 4 threads and 256 x
 // 256 blocks put 32 threads in each of 256 blocks, every one of which walks thousands of tiles).  It
 // gets all the threads of the block in lanes of four, one lane group each, and as many of the blocks
-// as that takes (a residual sum of 6.3 M floats under the naive options: 203 -> 12.5 us).
+// as that takes (a residual sum of 6.3 M floats under the naive options: 203 -> 12.5 us; lanes of four
+// where the extent is a multiple of four, else the threads step through the tile).  32-bit results
+// are stored with write-through (11.4 -> 9.5 us); lanes of one, two or eight bytes would each be a store
+// of their own on its way to memory (6.3 M halves 12.9 us against 5.4, doubles 37.7 against 22.0,
+// bytes 7.5 against 3.7), so results of other widths keep the given option.
 // The sizes are nominal: a product beyond what the device takes (64 x 64 threads on two loops) is cut.
 uint64_t boundedProduct(const std::array<uint64_t, 3>& sizes, uint64_t most) {
   uint64_t product = 1;
   for (uint64_t s : sizes) product = s == 0 ? 0 : product > most / s ? most : product * s;
   return product;
 }
-HipMappingOptions streamMappingOptions(const HipMappingOptions& given, const DeviceLimits& limits) {
+HipMappingOptions streamMappingOptions(const HipMappingOptions& given, const DeviceLimits& limits, bool words) {
   HipMappingOptions o = given;
   const uint64_t threads = boundedProduct({{o.block[0], o.block[1], o.block[2]}}, limits.maxThreadsPerBlock);
   o.tile(std::vector<uint64_t>{4 * threads}).unroll(4).useSharedMemory(false);
   o.mapToThreads(threads).mapToBlocks(boundedProduct({{o.grid[0], o.grid[1], o.grid[2]}}, std::numeric_limits<int32_t>::max()));
-  o.vectorWidth(4).useReadOnlyCache(true);
+  o.vectorWidth(4);
+  if (words) o.useReadOnlyCache(true);
   return o;
 }
 bool leavesThreadsOfAStreamUnused(const HipMappingOptions& o, const StagePlan& st, const DeviceLimits& limits) {
@@ -1256,7 +1261,7 @@ MappedProgram mapToHip(
   // The fill that precedes a divided sum: all dimensions merged, four elements per thread, 256
   // threads, as many blocks as that takes.
   HipMappingOptions fillOptions = fillMappingOptions(optionsIn);
-  HipMappingOptions streamOptions = streamMappingOptions(optionsIn, limits);
+  const HipMappingOptions streamOptions[2] = {streamMappingOptions(optionsIn, limits, false), streamMappingOptions(optionsIn, limits, true)};
   std::vector<const HipMappingOptions*> kernelOptions;
   bool anyThreadReduction = false;
   std::vector<std::unique_ptr<Emitter>> bodies;
@@ -1273,7 +1278,9 @@ MappedProgram mapToHip(
       k.stages.push_back(std::move(b.st));
     }
     // (a definition of one dimension is mapped as its options say)
-    if (!fill && single && raw[groups[gi].stages[0]].first().lhsVars.size() > 1 && isStream(k.stages[0]) && leavesThreadsOfAStreamUnused(optionsIn, k.stages[0], limits)) chosen = &streamOptions;
+    if (!fill && single && raw[groups[gi].stages[0]].first().lhsVars.size() > 1 && isStream(k.stages[0]) && leavesThreadsOfAStreamUnused(optionsIn, k.stages[0], limits)) {
+      chosen = &streamOptions[k.stages[0].views.at(k.stages[0].tensor).type.bits == 32];
+    }
     const HipMappingOptions& options = *chosen;
     kernelOptions.push_back(chosen);
     k.sharedDepth = single ? k.stages[0].numParallel : groups[gi].depth;

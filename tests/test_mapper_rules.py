@@ -47,3 +47,13 @@ def test_streams_take_any_nominal_block(threads, used):
         _, launches = tc.map_only(src, "f", [ShapeOnly((512, 1000))] * 2, f"naive;tile=32,32;mapToThreads={threads};mapToBlocks={blocks}")
         (grid, block), = launches
         assert block == (used, 1, 1) and grid == (-(-512 * 1000 // (4 * used)), 1, 1)
+
+
+@pytest.mark.parametrize("dtype,name,through", [("float", "float32", True), ("int32", "int32", True), ("float16", "float16", False),
+                                                ("double", "float64", False), ("int8", "int8", False)])
+def test_only_words_of_a_stream_are_written_through(dtype, name, through):
+    src = f"def f({dtype}(N, M) A, {dtype}(N, M) B) -> (O) {{ O(n, m) = A(n, m) + B(n, m) }}"
+    text, _ = tc.map_only(src, "f", [ShapeOnly((512, 1000), name)] * 2, "naive")
+    assert ("__tc::storeThrough(rsO_" in text) == through
+    text, _ = tc.map_only(src, "f", [ShapeOnly((512, 1000), name)] * 2, "naive;useReadOnlyCache=1")
+    assert "__tc::storeThrough(rsO_" in text                    # as the options say
