@@ -1132,6 +1132,13 @@ bool isStream(const StagePlan& st) {
   return ok;
 }
 
+// Product of thread or block sizes.  Those of a stream are nominal: a product beyond what the device
+// takes (64 x 64 threads on two loops) is cut.
+uint64_t boundedProduct(const std::array<uint64_t, 3>& sizes, uint64_t most) {
+  uint64_t product = 1;
+  for (uint64_t s : sizes) product = s == 0 ? 0 : product > most / s ? most : product * s;
+  return product;
+}
 // Options for a stream whose given options leave threads of the block unused: sizes for two or
 // three loops say little about the one loop that merging left (tile 32, 64 x 4 threads and 256 x
 // 256 blocks put 32 threads in each of 256 blocks, every one of which walks thousands of tiles).  It
@@ -1141,12 +1148,6 @@ bool isStream(const StagePlan& st) {
 // are stored with write-through (11.4 -> 9.5 us); lanes of one, two or eight bytes would each be a store
 // of their own on its way to memory (6.3 M halves 12.9 us against 5.4, doubles 37.7 against 22.0,
 // bytes 7.5 against 3.7), so results of other widths keep the given option.
-// The sizes are nominal: a product beyond what the device takes (64 x 64 threads on two loops) is cut.
-uint64_t boundedProduct(const std::array<uint64_t, 3>& sizes, uint64_t most) {
-  uint64_t product = 1;
-  for (uint64_t s : sizes) product = s == 0 ? 0 : product > most / s ? most : product * s;
-  return product;
-}
 HipMappingOptions streamMappingOptions(const HipMappingOptions& given, const DeviceLimits& limits, bool words) {
   HipMappingOptions o = given;
   const uint64_t threads = boundedProduct({{o.block[0], o.block[1], o.block[2]}}, limits.maxThreadsPerBlock);

@@ -57,3 +57,25 @@ def test_only_words_of_a_stream_are_written_through(dtype, name, through):
     assert ("__tc::storeThrough(rsO_" in text) == through
     text, _ = tc.map_only(src, "f", [ShapeOnly((512, 1000), name)] * 2, "naive;useReadOnlyCache=1")
     assert "__tc::storeThrough(rsO_" in text                    # as the options say
+
+
+PRODUCT = "def f(float(M, K) A, float(N, K) B) -> (O) { O(m, n) +=! A(m, r_k) * B(n, r_k) }"
+
+
+@pytest.mark.parametrize("extra,tiled", [
+    ("useSharedMemory=1;prefetchShared=1", True), ("prefetchShared=1", False), ("useSharedMemory=1;prefetchShared=1;maxSharedMemory=9000", False),
+    ("useSharedMemory=1;prefetchShared=1;sharedDepth=1", False),
+])
+def test_partial_reduction_tiles_need_copies_of_both_operands(extra, tiled):
+    text, _ = tc.map_only(PRODUCT, "f", [ShapeOnly((512, 1000)), ShapeOnly((512, 1000))],
+                          f"naive;tile=64,64,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;{extra}")
+    assert ("for (int t_r_k" in text) == tiled and "kok_ ?" not in text
+
+
+def test_a_copy_smaller_than_the_block_leaves_the_reduction_whole():
+    """16 filters of 16 channels are fewer elements than threads and are not staged."""
+    src = "def f(float(N, C, H, W) I, float(M, C, KH, KW) W1) -> (O) { O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw) }"
+    for threads, tiled in (("64,8", False), ("64,4", True)):
+        text, _ = tc.map_only(src, "f", [ShapeOnly((32, 114, 16, 16)), ShapeOnly((64, 114, 1, 1))],
+                              f"naive;tile=1,16,8,0,16;mapToThreads={threads};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+        assert ("for (int t_r_c" in text) == tiled
