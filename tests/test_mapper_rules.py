@@ -79,3 +79,20 @@ def test_a_copy_smaller_than_the_block_leaves_the_reduction_whole():
         text, _ = tc.map_only(src, "f", [ShapeOnly((32, 114, 16, 16)), ShapeOnly((64, 114, 1, 1))],
                               f"naive;tile=1,16,8,0,16;mapToThreads={threads};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
         assert ("for (int t_r_c" in text) == tiled
+
+
+HALF_PRODUCT = "def f(float16(M, K) A, float16(N, K) B) -> (O) { O(m, n) +=! float(A(m, r_k)) * float(B(n, r_k)) }"
+
+
+@pytest.mark.parametrize("k,threads,vector,shifted", [
+    (128, "64,8", 8, False),        # whole tiles
+    (160, "64,8", 8, False),        # the last tile half empty: whole vectors all the same
+    (164, "64,8", 4, False),        # rows of whole vectors of four
+    (163, "64,8", 4, True),         # vectors across the end of the tensor
+    (128, "64,16", 4, False),       # vectors of eight for half of the threads
+])
+def test_copies_of_halves(k, threads, vector, shifted):
+    text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((128, k), "float16"), ShapeOnly((128, k), "float16")],
+                          f"naive;tile=64,64,64;mapToThreads={threads};mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+    assert set(re.findall(r"pk\d*_[AB]_\[it_\] = \*\(const __tc::halfx(\d)u\*\)", text)) == {str(vector)}
+    assert ("= __tc::shiftDown(" in text) == shifted
