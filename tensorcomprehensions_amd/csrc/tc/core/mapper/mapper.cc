@@ -178,14 +178,18 @@ bool reductionMayEndInMidTile(const StagePlan& st, const std::string& k) {
 // still fit in LDS twice, two tiles at least and every wavefront with an output tile of its own.  Rows
 // of a copy are then 128 bytes, and the tile is not left on the instruction of half the rate
 // (4096^3, 128x256x32, second operand transposed 211 -> 157 us and plain 253 -> 158; 512x2048x768,
-// 64x64x32: 14.1 -> 11.5 and 20.8 -> 11.5).
-void deepenHalfTile(const StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits) {
+// 64x64x32: 14.1 -> 11.5 and 20.8 -> 11.5).  Not where the deeper tiles multiply an eighth more
+// points than the given ones and a block holds more than 64x64 outputs, which a deeper tile serves
+// least (1024x1024, 128x128x32, second operand transposed: depth 224 as 4 tiles of 64 5.8 us, as 7 of
+// 32 5.2; depth 288 6.2 and 5.9, before 6.9; 64x64x32 of depth 224 3.6 and 3.5).  The planning of the
+// copies returns to the given tile when they turn out not to fit twice.
+void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits) {
   if (!o.prefetchSharedValue || !o.useSharedMemoryValue || st.mfmaK.size() != 1 || !st.mfmaBatch.empty()) return;
   for (const auto& operand : st.stmts[0].rhs->args) {
     if (st.views.at(contractionOperand(operand)->name).type.bits != 16) return;
   }
-  const int64_t depth = 64;
-  if (v.tile != depth / 2 || v.extent < 2 * depth) return;
+  const int64_t depth = 64, given = v.tile;
+  if (given != depth / 2 || v.extent < 2 * depth) return;
   int64_t rows = 1, columns = 1;
   for (const auto& w : st.vars) {
     for (const auto& n : st.mfmaM) rows *= w.name == n ? w.tile : 1;
@@ -194,12 +198,14 @@ void deepenHalfTile(const StagePlan& st, LoopVar& v, const HipMappingOptions& o,
   int64_t lds = limits.ldsBytesPerBlock;
   if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
   if (rows * columns < 256 * waves || 2 * 2 * (rows + columns) * (depth + 8) > lds) return;
-  const int64_t given = v.tile;
+  if (rows * columns > 64 * 64 && 8 * depth * ceilDiv(v.extent, depth) > 9 * given * ceilDiv(v.extent, given)) return;
   v.tile = depth;
   v.numTiles = ceilDiv(v.extent, depth);
+  st.givenReductionTile = given;
   if (v.extent % depth != 0 && !reductionMayEndInMidTile(st, v.name)) {
     v.tile = given;
     v.numTiles = ceilDiv(v.extent, given);
+    st.givenReductionTile = 0;
   }
 }
 

@@ -96,3 +96,24 @@ def test_copies_of_halves(k, threads, vector, shifted):
                           f"naive;tile=64,64,64;mapToThreads={threads};mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
     assert set(re.findall(r"pk\d*_[AB]_\[it_\] = \*\(const __tc::halfx(\d)u\*\)", text)) == {str(vector)}
     assert ("= __tc::shiftDown(" in text) == shifted
+
+
+def depths(text):
+    return {int(d) for d in re.findall(r"t_r_k[^;]*\* (\d+)\)", text)}
+
+
+@pytest.mark.parametrize("tile,k,depth", [("128,128,32", 127, 32), ("128,128,32", 128, 64), ("128,128,32", 224, 32), ("128,128,32", 288, 64),
+                                          ("128,256,32", 160, 32), ("64,64,32", 160, 64), ("64,64,16", 128, 16), ("128,128,24", 240, 24)])
+def test_tiles_of_halves_that_are_deepened(tile, k, depth):
+    """To 64 points, from two tiles on, in large blocks up to an eighth of surplus points."""
+    text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((512, k), "float16")] * 2, f"naive;tile={tile};{MATRIX}")
+    assert depths(text) == {depth}
+
+
+def test_a_deepened_tile_is_given_up_where_its_copies_fit_only_once():
+    """Copies read through the transposing read have wider pitches than the rule counts on."""
+    src = "def f(float16(K, M) A, float16(K, N) B) -> (O) { O(m, n) +=! float(A(r_k, m)) * float(B(r_k, n)) }"
+    for limit, depth in ((38000, 32), (42000, 64)):
+        text, _ = tc.map_only(src, "f", [ShapeOnly((256, 512), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX};maxSharedMemory={limit}")
+        assert depths(text) == {depth}
+        assert text.count("lds0_A[") and f"lds0_A[{2 * depth * 80}]" in text  # two copies
