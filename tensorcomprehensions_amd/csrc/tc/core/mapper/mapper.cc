@@ -274,6 +274,7 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
   if (best < 0 || 4 * bestCost > 3 * given) return;
   st.vars[best].tile = bestTile;
   st.vars[best].numTiles = ceilDiv(st.vars[best].extent, bestTile);
+  st.fittedToDevice = true;
 }
 
 void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {

@@ -105,6 +105,9 @@ struct StagePlan {
   // Tile of the outermost reduction variable as the options give it, where the mapper took another
   // (0: as given).
   int64_t givenReductionTile = 0;
+  // A block-mapped variable has a smaller tile than the options give it, so that the blocks fill the
+  // device.
+  bool fittedToDevice = false;
   // The stage adds partial sums into its tensor with atomics: its first parallel variable numbers
   // slices of the reduction and is no subscript of the tensor.
   bool atomic = false;

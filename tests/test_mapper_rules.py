@@ -117,3 +117,29 @@ def test_a_deepened_tile_is_given_up_where_its_copies_fit_only_once():
         text, _ = tc.map_only(src, "f", [ShapeOnly((256, 512), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX};maxSharedMemory={limit}")
         assert depths(text) == {depth}
         assert text.count("lds0_A[") and f"lds0_A[{2 * depth * 80}]" in text  # two copies
+
+
+@pytest.mark.parametrize("m,n,k,tile,threads,tail,tiled", [
+    (512, 512, 200, "64,64,32", "64,8", ";prefetchShared=1", True),     # an eighth of surplus points under the pipeline
+    (512, 512, 100, "64,64,32", "64,8", ";prefetchShared=1", False),    # more than a fifth
+    (512, 512, 72, "64,64,32", "64,8", ";prefetchShared=1", False),     # three tiles
+    (512, 512, 200, "64,64,32", "64,8", "", False),                     # no overlap to gain
+    (512, 512, 1000, "64,64,32", "64,8", "", True),                     # whole, the copies do not fit
+    (512, 512, 130, "64,64,32", "64,8", ";prefetchShared=1", True),     # whole, the steps are masked
+    (512, 512, 33, "64,64,32", "64,8", ";prefetchShared=1", False),     # and half of them would be surplus
+    (512, 512, 1000, "32,32,32", "64,8", ";prefetchShared=1", False),   # wavefronts that only a whole reduction keeps busy
+    (512, 512, 1000, "32,32,32", "64,4", ";prefetchShared=1", True),
+    (512, 512, 400, "16,32,128", "64,8", ";prefetchShared=1", True),    # a tile's reduction shared by four wavefronts
+    (512, 512, 300, "16,32,128", "64,8", ";prefetchShared=1", False),
+    (512, 512, 250, "64,64,32", "64,8", ";maxSharedMemory=9000", True), # masked either way
+])
+def test_partial_reduction_tiles(m, n, k, tile, threads, tail, tiled):
+    text, _ = tc.map_only(PRODUCT, "f", [ShapeOnly((m, k)), ShapeOnly((n, k))],
+                          f"naive;tile={tile};mapToThreads={threads};mapToBlocks=256,256;useMfma=1;useSharedMemory=1{tail}")
+    assert ("for (int t_r_k" in text) == tiled
+
+
+@pytest.mark.parametrize("k", [33, 70, 100, 160])
+def test_partial_reduction_tiles_of_halves_stay(k):
+    text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((512, k), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX}")
+    assert "for (int t_r_k" in text
