@@ -732,7 +732,7 @@ void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
     std::map<std::string, std::string> produced; // canonical load -> cache name
     for (size_t i = 0; i < gens.size(); ++i) {
       if (sigs[i].empty() || sigs[i] != sigs[0]) continue;
-      if (gens[i].cacheSlots() > 256) continue;
+      if (gens[i].cacheSlots() > StageCodegen::kMaxCacheSlots) continue;
       for (const auto& l : loads[i]) {
         bool sharedLater = false;
         for (size_t j = 0; j < gens.size(); ++j) {
@@ -768,7 +768,7 @@ void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
         visitUnconditional(stmt.rhs, [&](const ExprRef& e) {
           if (e->kind != Expr::Load || kc.registerForwards.count(e->name)) return; // (already in a register)
           StageCodegen::AddressForm want = gens[j].addressForm(e, nullptr);
-          if (!want.valid || want.slots > 256) return;
+          if (!want.valid || want.slots > StageCodegen::kMaxCacheSlots) return;
           std::string mine = "p" + e->name + "[" + gens[j].flatIndex(e->name, e->args, "") + "]";
           if (gens[j].regCaches.count(mine)) return;
           for (size_t i = 0; i < j; ++i) {

@@ -143,3 +143,17 @@ def test_partial_reduction_tiles(m, n, k, tile, threads, tail, tiled):
 def test_partial_reduction_tiles_of_halves_stay(k):
     text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((512, k), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX}")
     assert "for (int t_r_k" in text
+
+
+@pytest.mark.parametrize("src,shape,options,staged", [
+    ("def f(float(N, K) I) -> (s) { s(n) +=! I(n, k) * I(n, k) }", (64, 4096), "tile=1,0;mapToThreads=256;matchLibraryCalls=1", False),
+    ("def f(float(N, K) I) -> (s) { s(n) +=! I(n, k) * I(n, k) }", (64, 4100), "tile=1,0;mapToThreads=256;matchLibraryCalls=1", True),
+    ("def f(float(N, K) I) -> (s) { s(n) +=! I(n, k) * I(n, k) }", (64, 2000), "tile=1,0;mapToThreads=256;matchLibraryCalls=1;vectorWidth=4", True),
+    ("def f(float(N, K) I) -> (s) { s(k) +=! I(n, k) * I(n, k) }", (128, 1000), "tile=32,32;mapToThreads=32", True),
+    # (the sum before it leaves the elements in registers)
+    ("def f(float(N, K) I) -> (t, s) { t(n) +=! I(n, k) s(n) +=! I(n, k) * I(n, k) }", (64, 4100),
+     "outerScheduleFusionStrategy=Max;tile=1,0;mapToThreads=256;matchLibraryCalls=1;usePrivateMemory=1;unroll=64", False),
+])
+def test_squares_are_staged_where_the_copies_read_better(src, shape, options, staged):
+    text, _ = mapped(src, "f", [shape], f"naive;{options};mapToBlocks=4096;useSharedMemory=1")
+    assert bool(re.search(r"lds\d_I", text)) == staged
