@@ -1,6 +1,6 @@
 // libtc_hip_testing.so: what the host-side tests and the sanitized drivers need beyond the product's
 // C ABI -- a synthetic genetic search, the whole tune() on a cost model (tc/autotuner/model_backend.h),
-// a sample options cache and its self-test.  Test infrastructure: nothing of the product links it.
+// a sample options cache and its self-test, the mapper under other devices' limits.  Test infrastructure: nothing of the product links it.
 #include "capi/tc_hip_testing.h"
 
 #include <cstdio>
@@ -33,6 +33,33 @@ double syntheticCost(const TuningConfiguration& c) {
   cost += o.useSharedMemoryValue ? 0 : 2;
   cost += o.vectorWidthValue == 4 ? 0 : 1;
   return cost;
+}
+
+// "<compute units>|<images>x<channels>x<height>x<width>|<options>": grid of a 3x3 convolution with 64 filters
+std::string convolutionGrid(const std::string& arg) {
+  const size_t p1 = arg.find('|'), p2 = arg.find('|', p1 + 1);
+  TC_CHECK(p1 != std::string::npos && p2 != std::string::npos) << "expected <compute units>|<sizes>|<options>";
+  const std::string text =
+      "def convolution(float(N, C, H, W) I, float(M, C, KH, KW) W1) -> (O) {"
+      " O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw) }";
+  int64_t image[4], filter[4] = {64, 0, 3, 3};
+  std::stringstream sizes(arg.substr(p1 + 1, p2 - p1 - 1));
+  for (int64_t& d : image) {
+    std::string s;
+    std::getline(sizes, s, 'x');
+    d = std::stoll(s);
+  }
+  filter[1] = image[1];
+  DLConstTensor a{nullptr, {kDLROCM, 0}, 4, {2, 32, 1}, image, nullptr, 0};
+  DLConstTensor b{nullptr, {kDLROCM, 0}, 4, {2, 32, 1}, filter, nullptr, 0};
+  auto f = tc::detail::translate(tc::detail::parse(text).at("convolution"), {&a, &b}, CompilerOptions());
+  mapper::DeviceLimits limits;
+  limits.ldsBytesPerBlock = 163840;
+  limits.computeUnits = std::stoll(arg.substr(0, p1));
+  auto program = mapper::mapToHip(f, HipMappingOptions::fromText(arg.substr(p2 + 1)), "convolution", limits);
+  std::ostringstream out;
+  for (int i = 0; i < 3; ++i) out << (i ? "x" : "") << program.kernels.at(0).grid[i];
+  return out.str();
 }
 
 std::string runSyntheticSearch(const std::map<std::string, std::string>& kv) {
@@ -143,7 +170,9 @@ std::string cacheSelfTest(const std::string& scratch) {
 extern "C" int tc_testing_query(const char* what, const char* arg, char** out) {
   try {
     std::string w = what ? what : "", a = arg ? arg : "", result;
-    if (w == "genetic_search") {
+    if (w == "convolution_grid") {
+      result = convolutionGrid(a);
+    } else if (w == "genetic_search") {
       result = runSyntheticSearch(parseSettings(a.c_str()));
     } else if (w == "tune_on_model") {
       // "<settings>|<entry point>|<shape>;<shape>...|<tc text>": the whole tune() on the host

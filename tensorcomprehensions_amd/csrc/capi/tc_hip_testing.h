@@ -5,7 +5,9 @@
 #ifdef __cplusplus
 extern "C" {
 #endif
-/*   "genetic_search", "seed=..;generations=..;pop_size=.." -> best synthetic cost per generation
+/*   "convolution_grid", "<compute units>|<images>x<channels>x<height>x<width>|<options>" -> grid the mapper gives
+ *       a 3x3 convolution with 64 filters on a device of so many compute units
+ *   "genetic_search", "seed=..;generations=..;pop_size=.." -> best synthetic cost per generation
  *   "tune_on_model", "<settings>|<entry point>|<shape>;<shape>...|<tc text>" -> the whole tune() against the
  *       cost model of tc/autotuner/model_backend.h: "best=<options>\ncost_ns=..\nnaive_ns=.."
  *   "options_cache_selftest", "<scratch file>" -> "name=value" lines: what a sample cache answers (sizes,

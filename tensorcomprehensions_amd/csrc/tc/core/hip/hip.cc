@@ -10,13 +10,16 @@ HipGPUInfo::HipGPUInfo() {
   for (int i = 0; i < n; ++i) {
     char name[256] = {0}, arch[64] = {0};
     size_t lds = 65536;
+    int units = 256;
     if (tchip_device_name(i, name, sizeof(name)) != 0 || tchip_device_arch(i, arch, sizeof(arch)) != 0) {
       break;
     }
     tchip_device_lds_bytes(i, &lds);
+    tchip_device_compute_units(i, &units);
     names_.push_back(name);
     archs_.push_back(arch);
     lds_.push_back(lds);
+    units_.push_back(units);
   }
 }
 
@@ -43,6 +46,10 @@ std::string HipGPUInfo::GetArch(int id) const {
 size_t HipGPUInfo::SharedMemorySize() const {
   if (lds_.empty()) return 163840;
   return lds_.at(CurrentGPUId());
+}
+int HipGPUInfo::ComputeUnits() const {
+  if (units_.empty()) return 256;
+  return units_.at(CurrentGPUId());
 }
 
 } // namespace tc

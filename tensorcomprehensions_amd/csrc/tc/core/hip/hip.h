@@ -29,12 +29,14 @@ class HipGPUInfo {
   int CurrentGPUId() const;
   std::string GetGPUName(int id = -1) const;  // "" when no device is present
   std::string GetArch(int id = -1) const;     // "gfx950" when no device is present
-  size_t SharedMemorySize() const;            // LDS per workgroup; 65536 when no device is present
+  size_t SharedMemorySize() const;            // LDS per workgroup; 163840 when no device is present
+  int ComputeUnits() const;                   // of the device or partition; 256 when no device is present
 
  private:
   HipGPUInfo();
   std::vector<std::string> names_, archs_;
   std::vector<size_t> lds_;
+  std::vector<int> units_;
 };
 
 struct WithHipDevice {

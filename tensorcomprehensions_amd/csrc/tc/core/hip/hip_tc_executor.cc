@@ -53,6 +53,7 @@ HipCompilationResult HipBackend::compileWithTcMapper(
     const HipMappingOptions& options) {
   mapper::DeviceLimits limits;
   limits.ldsBytesPerBlock = static_cast<int64_t>(HipGPUInfo::GPUInfo().SharedMemorySize());
+  limits.computeUnits = HipGPUInfo::GPUInfo().ComputeUnits();
   HipCompilationResult r;
   r.specializedName = specializedKernelName(tcName, function);
   r.program = mapper::mapToHip(function, options, r.specializedName, limits);

@@ -211,15 +211,16 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
 
 // A matrix-core stage over reduction tiles whose blocks leave compute units idle: one block-mapped
 // variable gets the smaller tile that shortens the longest-running compute unit by a quarter or more,
-// if there is one.  A compute unit's time is its rounds of blocks times the output tiles of the busiest
+// if there is one (compute units are those of the device, or of its partition).  A compute unit's time
+// is its rounds of blocks times the output tiles of the busiest
 // wavefront and about two more for a block's staging (3x3 convolution of 16x64x57x57, 64 filters,
 // blocks of 32 filters x 11 rows, 8 channels a step: 160 blocks of 10 tiles 55.5 us, 256 blocks of 7
 // (7 rows) 46.0, 320 blocks of 6 in two rounds (6 rows) 63.9; 32x64x30x30: 128 blocks of 7 tiles 41.3,
 // 256 of 4 24.0; 1x1 over 32x128x16x16: 96 blocks of 4 tiles 13.3, 192 of 2 9.5).  Floats and
 // more than two output variables only (convolutions): products keep the rectangles of output tiles they
-// were given.
-void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves) {
-  constexpr int64_t kComputeUnits = 256, kStaging = 2;
+// were given.  mapToBlocks sizes that hold exactly the given tiles keep those tiles.
+void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
+  constexpr int64_t kStaging = 2;
   if (k.stages.size() != 1 || !o.prefetchSharedValue || !o.useSharedMemoryValue || !st.mfmaBatch.empty() || st.mfmaM.size() + st.mfmaN.size() < 3) return;
   for (const auto& operand : st.stmts[0].rhs->args) {
     if (st.views.at(contractionOperand(operand)->name).type.bits != 32) return;
@@ -246,11 +247,11 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
       for (const auto& n : st.mfmaN) columns *= w.name == n ? w.tile : 1;
     }
     const int64_t tiles = ceilDiv(rows, 16) * ceilDiv(columns, 16);
-    return tiles < waves ? 0 : ceilDiv(blocks, kComputeUnits) * (ceilDiv(tiles, waves) + kStaging);
+    return tiles < waves ? 0 : ceilDiv(blocks, computeUnits) * (ceilDiv(tiles, waves) + kStaging);
   };
   int64_t blocks = 0;
   const int64_t given = cost(blocks);
-  if (given == 0 || blocks >= kComputeUnits) return;
+  if (given == 0 || blocks >= computeUnits) return;
   int best = -1;
   int64_t bestTile = 0, bestCost = given;
   for (int i = 0; i < st.numParallel; ++i) {
@@ -320,7 +321,7 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
       v.tile = (t <= 0 || t > v.extent) ? v.extent : t;
       v.numTiles = ceilDiv(v.extent, v.tile);
     }
-    if (st.mfma) fillComputeUnits(k, st, o, waves);
+    if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
     // blocks: outermost shared parallel variables, x first
     int axis = 0;
     for (int i = 0; i < st.numParallel && i < k.sharedDepth && axis < static_cast<int>(o.grid.size()); ++i) {

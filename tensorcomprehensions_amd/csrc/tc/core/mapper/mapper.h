@@ -125,6 +125,7 @@ struct KernelPlan {
 struct DeviceLimits {
   int64_t ldsBytesPerBlock = 65536;
   int64_t maxThreadsPerBlock = 1024;
+  int64_t computeUnits = 256;
   int wavefront = 64;
 };
 

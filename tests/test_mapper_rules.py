@@ -5,6 +5,7 @@ import pytest
 
 import tensorcomprehensions_amd as tc
 from tensorcomprehensions_amd import ShapeOnly
+from tests.scaffolding import scaffold_query
 
 
 def mapped(src, entry, shapes, options):
@@ -157,3 +158,27 @@ def test_partial_reduction_tiles_of_halves_stay(k):
 def test_squares_are_staged_where_the_copies_read_better(src, shape, options, staged):
     text, _ = mapped(src, "f", [shape], f"naive;{options};mapToBlocks=4096;useSharedMemory=1")
     assert bool(re.search(r"lds\d_I", text)) == staged
+
+
+BANDS = "naive;tile=1,32,11,0,8;mapToThreads=64,8;useMfma=1;useSharedMemory=1;sharedDepth=7;prefetchShared=1"
+
+
+@pytest.mark.parametrize("units,sizes,blocks,grid", [
+    (256, "16x64x57x57", "256,256,256", "16x8x2"),      # 160 blocks of 11 rows leave units idle: 256 of 7
+    (128, "16x64x57x57", "256,256,256", "16x5x2"),      # more blocks than units
+    (256, "1x64x57x57", "256,256,256", "2x55x1"),
+    (32, "1x64x57x57", "256,256,256", "2x14x1"),
+    (256, "1x64x57x57", "2,5", "2x5x1"),                # as many blocks as the given tiles make: they stay
+    (256, "32x64x30x30", "256,256,256", "32x3x2"),      # no smaller tile that is a quarter faster
+    (256, "1x64x57x57", "64,64", "2x55x1"),
+])
+def test_convolutions_get_tiles_that_fill_the_device(units, sizes, blocks, grid):
+    assert scaffold_query("convolution_grid", f"{units}|{sizes}|{BANDS};mapToBlocks={blocks}") == grid
+
+
+def test_tiles_that_stay_as_given():
+    for options in (BANDS.replace(";prefetchShared=1", ""), BANDS.replace("useSharedMemory=1;", ""), BANDS.replace(",0,8", ",0,0"),
+                    BANDS.replace("1,32,11", "1,16,1")):    # fewer output tiles than wavefronts
+        rows = 55 if "1,16,1" in options else 5
+        got = scaffold_query("convolution_grid", f"256|1x64x57x57|{options};mapToBlocks=256,256,256")
+        assert f"{rows}" in got.split("x")
