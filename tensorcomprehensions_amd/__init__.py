@@ -95,6 +95,17 @@ class _NoPlan:
 
 
 _NO_PLAN = _NoPlan()
+_reported = False
+
+
+def _report_general_path(error):
+    """Once per process: the extension is missing, or was built for another PyTorch."""
+    global _reported
+    if not _reported:
+        _reported = True
+        import warnings
+        warnings.warn(f"calls on PyTorch tensors take the general path, 4 to 6 us slower per tensor: {error}; "
+                      "build the extension with `make -C tensorcomprehensions_amd/csrc`", RuntimeWarning, stacklevel=4)
 
 
 def _plan(executor):
@@ -108,9 +119,14 @@ def _plan(executor):
             return _NO_PLAN                     # (it may be loaded later)
         try:
             from ._torch_call import Plan
-            plan = Plan(executor._h.value, TcError)
-        except (ImportError, ValueError):
+        except ImportError as error:
             plan = _NO_PLAN
+            _report_general_path(error)
+        else:
+            try:
+                plan = Plan(executor._h.value, TcError)
+            except ValueError:                  # tensors of a type that ATen does not have
+                plan = _NO_PLAN
         executor._native = plan
     return plan
 
