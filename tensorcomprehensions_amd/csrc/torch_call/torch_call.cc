@@ -105,15 +105,27 @@ bool items(PyObject* sequence, PyObject**& first, Py_ssize_t& count) {
 
 using Pointers = std::array<void*, kMaxTensors>;
 
+// Row-major strides in every dimension, those of one element included: is_contiguous() takes any
+// stride there, compilation does not, and a defined comprehension compiles on strides it has not seen.
+bool hasCanonicalStrides(const at::Tensor& t) {
+  const auto sizes = t.sizes(), strides = t.strides();
+  int64_t expect = 1;
+  for (size_t d = sizes.size(); d-- > 0;) {
+    if (strides[d] != expect) return false;
+    expect *= sizes[d];
+  }
+  return true;
+}
+
 // data pointers of the tensors when all of them match
-bool collect(PyObject* sequence, const std::vector<TensorMeta>& metas, c10::DeviceIndex& device, Pointers& pointers) {
+bool collect(PyObject* sequence, const std::vector<TensorMeta>& metas, c10::DeviceIndex& device, Pointers& pointers, bool canonical = false) {
   PyObject** first;
   Py_ssize_t count;
   if (!items(sequence, first, count) || static_cast<size_t>(count) != metas.size()) return false;
   for (Py_ssize_t i = 0; i < count; ++i) {
     if (!THPVariable_Check(first[i])) return false;
     const at::Tensor& t = THPVariable_Unpack(first[i]);
-    if (!matches(t, metas[i], device)) return false;
+    if (!matches(t, metas[i], device) || (canonical && !hasCanonicalStrides(t))) return false;
     pointers[i] = t.data_ptr();
   }
   return true;
@@ -180,7 +192,7 @@ PyObject* planCall(PyObject* self, PyObject* inputs) {
   if (plan->inputs->empty()) Py_RETURN_NONE;
   c10::DeviceIndex device = -1;
   Pointers in, out;
-  if (!collect(inputs, *plan->inputs, device, in)) Py_RETURN_NONE;
+  if (!collect(inputs, *plan->inputs, device, in, true)) Py_RETURN_NONE;
   std::vector<at::Tensor> results;
   results.reserve(plan->outputs->size());
   for (size_t i = 0; i < plan->outputs->size(); ++i) {

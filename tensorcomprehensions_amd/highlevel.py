@@ -110,7 +110,8 @@ class TC:
             if options is None:
                 raise _tc.TcError(f"no mapping options available for {entry_point} at these sizes")
             ex = self._executors[key] = _tc.compile(self.tc, entry_point, list(inputs), options)
-        self._latest[entry_point] = ex
+        # (bool and uint8 tensors look alike to the executor; their options need not be the same)
+        self._latest[entry_point] = None if any(t[1] in ("torch.bool", "torch.uint8") for t in key[1:]) else ex
         return ex(*inputs, outputs=outputs, unchecked=unchecked)
 
 

@@ -100,3 +100,28 @@ def test_a_cleared_executor_reports_it():
     ex.clear_runtime_compiled_function()
     with pytest.raises(tc.TcError, match="No rtcFun_ attached"):
         ex(A, B)
+
+
+def test_defined_methods_answer_the_same_whatever_was_called_before():
+    """Strides and types that options and compilation have not seen go through them, also right after
+    a call that differs in nothing else."""
+    src = "def f(float(N, M) A) -> (C) { C(n, m) = A(n, m) + 1 }"
+    column, row = torch.arange(5.0, device="cuda").reshape(5, 1), torch.arange(5.0, device="cuda").reshape(1, 5)
+    for before in ([], [column]):
+        T = tc.define(src, tc.make_naive_options_factory())
+        for A in before:
+            assert torch.equal(T.f(A), A + 1)
+        with pytest.raises(tc.TcError, match="invalid strides"):
+            T.f(row.t())                                # (5, 1) with strides (1, 5)
+    asked = []
+
+    def factory(text, entry, *inputs):
+        asked.append([str(t.dtype) for t in inputs])
+        return tc.MappingOptions("naive")
+
+    T = tc.define(MASK, factory)
+    A = torch.arange(8, device="cuda", dtype=torch.float32)
+    B = (A % 2) == 0
+    for mask in (B, B.to(torch.uint8), B):
+        assert torch.equal(T.mask(A, mask), torch.where(B, A, torch.zeros_like(A)))
+    assert [a[1] for a in asked] == ["torch.bool", "torch.uint8"]
