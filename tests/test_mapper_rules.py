@@ -182,3 +182,18 @@ def test_tiles_that_stay_as_given():
         rows = 55 if "1,16,1" in options else 5
         got = scaffold_query("convolution_grid", f"256|1x64x57x57|{options};mapToBlocks=256,256,256")
         assert f"{rows}" in got.split("x")
+
+
+@pytest.mark.parametrize("width,tile,waves,blocked", [
+    (30, "1,16,7,0,8", 8, False),       # 13 tiles in one row as 16 places
+    (30, "1,16,7,0,8", 4, False),
+    (18, "1,16,14,0,8", 4, True),       # 14 as 16 in rows of four
+    (18, "1,16,14,0,8", 8, False),      # in rows of two
+    (34, "1,16,4,0,8", 8, True),        # 8 as 8
+    (18, "1,32,7,0,8", 4, True),        # 2 x 7 as four rectangles of 2 x 2
+])
+def test_rectangles_of_output_tiles_overhang_only_so_far(width, tile, waves, blocked):
+    src = "def f(float(N, C, H, W) I, float(M, C, KH, KW) W1) -> (O) { O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw) }"
+    text, _ = mapped(src, "f", [(256, 64, width, width), (96, 64, 3, 3)],
+                     f"naive;tile={tile};mapToThreads=64,{waves};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+    assert bool(re.search(r"float ra_\[\d+\]\[", text)) == blocked
