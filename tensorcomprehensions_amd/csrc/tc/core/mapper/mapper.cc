@@ -336,8 +336,10 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) {
       // one wavefront per 16x16 output tile; the block holds as many wavefronts as the block
       // option has threads.  Only the outermost reduction variable may be tiled (a tile that does
-      // not divide the extent needs operands whose surplus points can be told apart): operands are then staged in LDS one reduction tile at a time while the
-      // accumulators of a wavefront's output tiles stay in registers.
+      // not divide the extent needs operands whose surplus points can be told apart, and is kept
+      // where it pays, which the planning of the copies decides): operands are then staged in LDS
+      // one reduction tile at a time while the accumulators of a wavefront's output tiles stay in
+      // registers.
       bool firstReduction = true;
       for (auto& v : st.vars) {
         if (!v.reduction) continue;

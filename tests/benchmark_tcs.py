@@ -404,7 +404,7 @@ LARGE_CONTRACTIONS = {
 }
 
 LARGE_CONTRACTIONS.update({
-    # float16 operands on v_mfma_f32_16x16x16_f16 (the roofline of these two is the 2.5 PFLOP/s half peak)
+    # float16 operands on v_mfma_f32_16x16x32_f16 (the roofline of these two is the 2.5 PFLOP/s half peak)
     "half_tmm_4096": ("half_tmm", [("half", (4096, 4096)), ("half", (4096, 4096))],
                       "naive;tile=128,256,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;"
                       "prefetchShared=1", 4096),

@@ -13,9 +13,9 @@ pytestmark = pytest.mark.gpu
 
 # A(k, m): rows along the output variable in the first operand as well
 TRANSPOSED_A = "def half_tam(float16(K, M) A, float16(K, N) B) -> (C) { C(m, n) +=! float(A(r_k, m)) * float(B(r_k, n)) }"
-# operands that start inside their tensors, and a subscript that is no single variable
-SHIFTED = "def half_shift(float16(M, KP) A, float16(KP, N) B) -> (C) { C(m, n) +=! float(A(m, r_k + 3)) * float(B(r_k, n)) where r_k in 0:%d }"
-
+# operands that start inside their tensors: subscripts of one variable and a constant, or its mirror image
+SHIFTED = ("def half_shift(float16(M, KP) A, float16(KQ, N) B) -> (C) { C(m, n) +=! float(A(%s)) * float(B(%s))"
+           " where r_k in 0:%d, m in 0:%d, n in 0:%d }")
 
 def ints(shape, seed):
     return np.random.Generator(np.random.Philox(seed)).integers(-4, 5, size=shape).astype(np.float16)
@@ -60,12 +60,22 @@ def test_products_are_exact(m, k, n, tile, waves, wide):
             assert ("__tc::readTransposed(&" in text) == (entry != "half_tmm")
 
 
-def test_offset_subscripts_keep_the_general_reads():
-    k = 128
-    A, Bm = ints((64, k + 3), 1), ints((k + 3, 64), 2)
-    got, text = run(SHIFTED % k, "half_shift", [A, Bm],
+@pytest.mark.parametrize("a,b,m,k,n,vectors", [
+    ("m, r_k + 3", "r_k, n", 64, 128, 64, True),
+    ("m, r_k", "r_k + 1, n + 2", 64, 128, 64, True),
+    ("m + 1, r_k + 3", "r_k + 3, n + 5", 65, 131, 67, True),    # rows that end in mid-vector
+    ("m + 2, r_k", "r_k, 66 - n", 66, 130, 67, False),          # a mirrored subscript keeps the general reads
+    ("65 - m, r_k + 1", "r_k + 1, 98 - n", 66, 160, 99, False),
+])
+def test_offsets_move_the_copies_and_not_their_reads(a, b, m, k, n, vectors):
+    A, Bm = ints((m + 2, k + 3), 1), ints((k + 3, n + 5), 2)
+    index = {"m": np.arange(m), "r_k": np.arange(k), "n": np.arange(n)}
+    rows = [[eval(sub, {}, index) for sub in subs.split(",")] for subs in (a, b)]  # the subscripts, on all points
+    want = A[np.ix_(*rows[0])].astype(np.float32) @ Bm[np.ix_(*rows[1])].astype(np.float32)
+    got, text = run(SHIFTED % (a, b, k, m, n), "half_shift", [A, Bm],
                     "naive;tile=64,64,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
-    assert np.array_equal(got, A[:, 3:].astype(np.float32) @ Bm[:k].astype(np.float32))
+    assert np.array_equal(got, want)
+    assert ("__tc::readTransposed(&lds0_B[" in text) == vectors
 
 
 def test_a_tensor_that_is_both_operands():

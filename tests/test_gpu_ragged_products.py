@@ -102,3 +102,48 @@ def test_reversed_subscripts_over_partial_tiles(m, k, n, first, second, half):
     for tile in ("64,64,32", "16,32,64"):
         print(f"reversed {m}x{k}x{n} half={half} A({subs[0]}) B({subs[1]}) tile={tile}", flush=True)
         assert np.array_equal(run(src, "f", stored, f"naive;tile={tile};mapToThreads=64,8;{TAIL}"), want)
+
+
+@pytest.mark.parametrize("extra", ["", "useSharedMemory=1", "useSharedMemory=1;prefetchShared=1;maxSharedMemory=9000", "useSharedMemory=1;sharedDepth=1",
+                                   "useSharedMemory=1;prefetchShared=1"])
+@pytest.mark.parametrize("m,k,n", [(70, 100, 66), (33, 250, 130), (130, 72, 65)])
+def test_reductions_in_tiles_and_in_one_piece(m, k, n, extra):
+    """Both sides of the rule that keeps a partial reduction tile or drops it, operands staged or not."""
+    A, Bm = ints((m, k), m + k), ints((k, n), k + n)
+    want = A @ Bm
+    for tile, waves in (("64,64,32", 8), ("32,32,32", 8), ("16,32,64", 4)):
+        options = f"naive;tile={tile};mapToThreads=64,{waves};mapToBlocks=256,256;useMfma=1;{extra}"
+        print(f"product {m}x{k}x{n} {options}", flush=True)
+        assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), want)
+        assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), want)
+
+
+@pytest.mark.parametrize("n,c,m,side,kernel,tile,waves", [
+    (2, 13, 32, 30, 3, "1,16,7,0,8", 8), (2, 16, 32, 30, 3, "1,16,7,0,8", 4), (2, 12, 20, 18, 3, "1,32,7,0,8", 4), (3, 24, 16, 16, 1, "1,16,14,0,16", 8),
+])
+def test_convolutions_of_one_row_of_output_tiles(n, c, m, side, kernel, tile, waves):
+    """Thirteen or fourteen output tiles on four or eight wavefronts."""
+    arrays = [ints((n, c, side, side), 3), ints((m, c, kernel, kernel), 4), ints((m,), 5)]
+    got = run(B.CONVOLUTION, "convolution", arrays,
+              f"naive;tile={tile};mapToThreads=64,{waves};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;sharedDepth=7;prefetchShared=1")
+    (want,) = tc_oracle.run(B.CONVOLUTION, "convolution", arrays)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,k,n", [(300, 1000, 260), (130, 513, 200), (96, 160, 128), (257, 2048, 129)])
+def test_errors_on_deviates_stay_within_those_of_float_sums(m, k, n, half):
+    """Products are exact in float (halves) or rounded once, and k of them are added in float: every
+    element within (k + 1) u sum |a b|, u = 2^-24, and the norm of the errors within sqrt(k) u of the
+    result's, about twice what rounding k sums at random leaves."""
+    rng = np.random.Generator(np.random.Philox(k))
+    dtype = np.float16 if half else np.float32
+    A, Bm = rng.standard_normal((m, k)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
+    want = A.astype(np.float64) @ Bm.astype(np.float64)
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(A.astype(np.float64)) @ np.abs(Bm.astype(np.float64)))
+    for tile in (HALF_TILES if half else TILES):
+        options = f"naive;tile={tile};mapToThreads=64,8;{TAIL}"
+        print(f"deviates {m}x{k}x{n} half={half} tile={tile}", flush=True)
+        got = run(B.HALF_MATMUL if half else B.MATMUL, "half_matmul" if half else "matmul", [A, Bm], options).astype(np.float64)
+        assert (np.abs(got - want) <= bound).all()
+        assert np.linalg.norm(got - want) <= np.sqrt(k) * 2.0 ** -24 * np.linalg.norm(want)

@@ -197,3 +197,13 @@ def test_rectangles_of_output_tiles_overhang_only_so_far(width, tile, waves, blo
     text, _ = mapped(src, "f", [(256, 64, width, width), (96, 64, 3, 3)],
                      f"naive;tile={tile};mapToThreads=64,{waves};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
     assert bool(re.search(r"float ra_\[\d+\]\[", text)) == blocked
+
+
+def test_sizes_that_keep_a_stream_and_a_half_tile_as_given():
+    src = "def f(float(N, M) A, float(N, M) B) -> (O) { O(n, m) = A(n, m) + B(n, m) }"
+    for options, launch in (("tile=256;mapToThreads=256;mapToBlocks=64", ((64, 1, 1), (256, 1, 1))),
+                            ("tile=512;mapToThreads=256;mapToBlocks=64;vectorWidth=2", ((64, 1, 1), (256, 1, 1))),
+                            ("tile=32;mapToThreads=32;mapToBlocks=64", ((64, 1, 1), (32, 1, 1)))):
+        assert tc.map_only(src, "f", [ShapeOnly((512, 1000))] * 2, f"naive;{options}")[1] == [launch]
+    text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((512, 512), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX.replace(';prefetchShared=1', '')}")
+    assert depths(text) == {32}
