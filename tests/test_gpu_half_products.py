@@ -44,6 +44,7 @@ def run(src, entry, arrays, options):
     (256, 192, 512, "128,256,32", 8, True),
     (64, 96, 64, "64,64,24", 8, False),         # 24 does not divide 64
     (64, 320, 64, "32,32,32", 8, False),        # fewer output tiles than wavefronts
+    (144, 160, 160, "48,80,32", 4, False),      # no rectangles: the given tile, one output tile at a time
 ])
 def test_products_are_exact(m, k, n, tile, waves, wide):
     A, Bm = ints((m, k), m + k), ints((k, n), k + n)

@@ -207,3 +207,10 @@ def test_sizes_that_keep_a_stream_and_a_half_tile_as_given():
         assert tc.map_only(src, "f", [ShapeOnly((512, 1000))] * 2, f"naive;{options}")[1] == [launch]
     text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((512, 512), "float16")] * 2, f"naive;tile=64,64,32;{MATRIX.replace(';prefetchShared=1', '')}")
     assert depths(text) == {32}
+
+
+def test_a_deepened_tile_that_does_not_pay_leaves_the_given_one():
+    """15 output tiles on four wavefronts form no rectangles: 160 points stay five tiles of 32."""
+    text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((480, 160), "float16")] * 2,
+                          f"naive;tile=48,80,32;{MATRIX.replace('64,8', '64,4')}")
+    assert depths(text) == {32} and "for (int t_r_k" in text
