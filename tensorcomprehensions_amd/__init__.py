@@ -12,7 +12,8 @@ The functions mirror the reference's ATen entry points one-to-one
     autotune(tc, entry_point, inputs, base_options, **settings) -> [MappingOptions]
 
 torch is used for device memory and the current stream only; all work happens in
-libtc_hip.so through its C ABI.  There is no CPU or eager fallback.
+libtc_hip.so through its C ABI, for calls on torch tensors by way of the extension
+_torch_call.so (csrc/torch_call).  There is no CPU or eager fallback.
 """
 from collections import namedtuple
 import ctypes
