@@ -278,6 +278,72 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
   st.fittedToDevice = true;
 }
 
+// Products of float16 matrices O(m, n) +=! A * B whose outputs fill the device in blocks of 256 x 256 go to
+// __tc::largeHalfProduct (hip_libraries.h), whichever side of the operands the reduction is on: a block multiplies
+// more per value it reads from LDS than one of the given tiles.  Where the blocks leave compute units idle
+// the given tiles stay; so they do in other than 8 wavefronts, on other grids than one block a tile, without
+// shared memory or prefetchShared, where maxSharedMemory is below the 128 KB of the copies, for rows that are no whole
+// number of 16-byte vectors, and for reductions of fewer than 256 points.
+// Rounds of blocks x outputs of a block are compared.  Per output the large blocks take 0.5 to 0.7 of the time of
+// 128x256 ones and 0.4 to 0.6 of 128x128 ones, so they may compute a third more outputs, and twice as many where they occupy
+// 7/16 of the compute units (48 products of 800 to 4096 rows and columns, depths 256 to 4096, given / large: as many 1.3 to
+// 1.9, a third more 1.7 and 1.9, twice as many 1.01 to 1.32 from 112 blocks and 0.82 to 0.97 of 80 to 91, four times 0.5 to 0.65).
+constexpr int64_t kLargeHalfBlock = 256, kLargeHalfLds = 2 * 2 * 256 * 64 * 2;
+void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits, bool wide) {
+  if (k.stages.size() != 1 || wide || waves != 8 || !o.prefetchSharedValue || !o.useSharedMemoryValue || st.atomic) return;
+  int64_t lds = limits.ldsBytesPerBlock;
+  if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
+  if (lds < kLargeHalfLds || st.stmts.size() != 1 || !st.stmts[0].init || st.vars.size() != 3 || st.numParallel != 2 || st.lhsSubs.size() != 2) return;
+  const LoopVar &m = st.vars[0], &n = st.vars[1], &r = st.vars[2];
+  for (const auto& v : st.vars) {
+    if (v.min != 0) return;
+  }
+  auto isVar = [](const ExprRef& e, const LoopVar& v) { return e->kind == Expr::Var && e->name == v.name; };
+  auto isMatrix = [&](const std::string& tensor, int64_t rows, int64_t columns) {
+    const auto& view = st.views.at(tensor);
+    return view.extents.size() == 2 && view.extents[0] == rows && view.extents[1] == columns &&
+        rows * columns * view.type.bytes() < (int64_t(1) << 31);
+  };
+  if (!isVar(st.lhsSubs[0], m) || !isVar(st.lhsSubs[1], n) || !isMatrix(st.tensor, m.extent, n.extent)) return;
+  std::string tensors[2];  // of the m and of the n side
+  bool innermost[2];       // the reduction is the last subscript
+  for (const auto& operand : st.stmts[0].rhs->args) {
+    const ExprRef load = contractionOperand(operand);
+    if (st.views.at(load->name).type.bits != 16 || load->args.size() != 2) return;
+    bool found = false;
+    for (int side = 0; side < 2; ++side) {
+      const LoopVar& v = side == 0 ? m : n;
+      for (int last = 0; last < 2; ++last) {
+        const LoopVar &outer = last ? v : r, &inner = last ? r : v;
+        if (!isVar(load->args[0], outer) || !isVar(load->args[1], inner)) continue;
+        if (!isMatrix(load->name, outer.extent, inner.extent) || inner.extent % 8 != 0 || !tensors[side].empty()) return;
+        tensors[side] = load->name;
+        innermost[side] = last == 1;
+        found = true;
+      }
+    }
+    if (!found) return;
+  }
+  if (r.extent < 256) return;
+  const int64_t numTiles[2] = {m.numTiles, n.numTiles};
+  size_t axis = 0;
+  for (int64_t tiles : numTiles) {
+    if (tiles == 1) continue;
+    if (axis >= o.grid.size() || tiles > static_cast<int64_t>(o.grid[axis])) return;
+    ++axis;
+  }
+  const int64_t blocks = ceilDiv(m.extent, kLargeHalfBlock) * ceilDiv(n.extent, kLargeHalfBlock);
+  const int64_t given = ceilDiv(m.numTiles * n.numTiles, limits.computeUnits) * m.tile * n.tile;
+  const int64_t large = ceilDiv(blocks, limits.computeUnits) * kLargeHalfBlock * kLargeHalfBlock;
+  if (3 * large > 4 * given && (large > 2 * given || 16 * blocks < 7 * limits.computeUnits)) return;
+  std::ostringstream ss;
+  ss << (innermost[0] ? "true" : "false") << ", " << (innermost[1] ? "true" : "false") << ", " << m.extent << ", " << n.extent << ", " << r.extent
+     << ">(p" << st.tensor << ", p" << tensors[0] << ", p" << tensors[1];
+  st.largeHalfProduct = ss.str();
+  k.grid = {{blocks, 1, 1}};
+  k.block = {{64, waves, 1}};
+}
+
 void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
   const HipMappingOptions& o = kc.opts;
   KernelPlan& k = kc.k;
@@ -321,6 +387,8 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
       v.tile = (t <= 0 || t > v.extent) ? v.extent : t;
       v.numTiles = ceilDiv(v.extent, v.tile);
     }
+    if (st.mfma) takeLargeHalfProduct(k, st, o, waves, limits, kc.wide);
+    if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
     // blocks: outermost shared parallel variables, x first
     int axis = 0;
@@ -515,6 +583,15 @@ std::string kernelSignature(const ir::Function& f, const std::string& name, int6
 
 void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
   KernelPlan& k = kc.k;
+  if (!k.stages[0].largeHalfProduct.empty()) {
+    em.open(kernelSignature(kc.f, k.name, kc.NT()));
+    for (const auto& p : kc.f.params) em.line("(void)" + p.first + ";");
+    em.line("__shared__ __attribute__((aligned(1024))) char tiles_[" + std::to_string(kLargeHalfLds) + "];");
+    em.line("__tc::largeHalfProduct<" + k.stages[0].largeHalfProduct + ", (__tc::ldschar*)tiles_);");
+    em.close();
+    k.ldsBytes = kLargeHalfLds;
+    return;
+  }
   std::vector<StageCodegen> gens;
   gens.reserve(k.stages.size());
   int64_t ldsBudget = limits.ldsBytesPerBlock;
@@ -1357,9 +1434,12 @@ MappedProgram mapToHip(
     emitKernel(kc, limits, *bodies.back());
   }
   src << "// generated by the TC HIP mapper for gfx950; function " << f.name << "\n";
-  bool halfProducts = false;
-  for (const auto& b : bodies) halfProducts |= b->out.str().find("__tc::multiplyHalves(") != std::string::npos;
-  src << hip::deviceLibrary(anyThreadReduction, halfProducts);
+  bool halfProducts = false, largeHalfProducts = false;
+  for (const auto& b : bodies) {
+    halfProducts |= b->out.str().find("__tc::multiplyHalves(") != std::string::npos;
+    largeHalfProducts |= b->out.str().find("__tc::largeHalfProduct<") != std::string::npos;
+  }
+  src << hip::deviceLibrary(anyThreadReduction, halfProducts, largeHalfProducts);
   for (const auto& b : bodies) src << "\n" << b->out.str();
   prog.source = src.str();
   return prog;

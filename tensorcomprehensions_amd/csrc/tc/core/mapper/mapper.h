@@ -108,6 +108,9 @@ struct StagePlan {
   // A block-mapped variable has a smaller tile than the options give it, so that the blocks fill the
   // device.
   bool fittedToDevice = false;
+  // A product of halves with many outputs, computed by __tc::largeHalfProduct (its template arguments;
+  // empty: not this stage).
+  std::string largeHalfProduct;
   // The stage adds partial sums into its tensor with atomics: its first parallel variable numbers
   // slices of the reduction and is no subscript of the tensor.
   bool atomic = false;

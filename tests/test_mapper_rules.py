@@ -214,3 +214,43 @@ def test_a_deepened_tile_that_does_not_pay_leaves_the_given_one():
     text, _ = tc.map_only(HALF_PRODUCT, "f", [ShapeOnly((480, 160), "float16")] * 2,
                           f"naive;tile=48,80,32;{MATRIX.replace('64,8', '64,4')}")
     assert depths(text) == {32} and "for (int t_r_k" in text
+
+
+ANY_HALF_PRODUCT = "def f(float16(%s) A, float16(%s) B) -> (O) { O(m, n) +=! float(A(%s)) * float(B(%s)) }"
+
+
+@pytest.mark.parametrize("m,n,k,tile,changes,large", [
+    (4096, 4096, 4096, "128,256,32", "", True),
+    (2512, 3432, 256, "128,256,32", "", True),                  # as many outputs a round
+    (1808, 3688, 384, "128,128,64", "", True),                  # 120 blocks compute twice as many
+    (1784, 3256, 256, "128,128,64", "", False),                 # 91 blocks do
+    (4096, 4096, 248, "128,256,32", "", False),                 # a short reduction
+    (4096, 4096, 4092, "128,256,32", "", False),                # rows that are no whole vectors
+    (4095, 4096, 4096, "128,256,32", "", True),                 # (rows of the output may be any number)
+    (4096, 4095, 4096, "128,256,32", "", False),                # rows of B
+    (4096, 4096, 4096, "128,256,32", "maxSharedMemory=131071", False),
+    (4096, 4096, 4096, "128,256,32", "prefetchShared=0", False),
+    (4096, 4096, 4096, "128,256,32", "mapToThreads=64,4", False),
+    (4096, 4096, 4096, "128,256,32", "mapToBlocks=16,16", False),
+    (4096, 4096, 4096, "128,256,32", "reductionBlocks=2", False),
+])
+def test_large_half_products(m, n, k, tile, changes, large):
+    text, launches = tc.map_only(ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n"), "f", [ShapeOnly((m, k), "float16"), ShapeOnly((k, n), "float16")],
+                                 f"naive;tile={tile};{MATRIX};{changes}")
+    assert ("__tc::largeHalfProduct<true, false, " in text) == large
+    if large:
+        assert launches == [((-(-m // 256) * -(-n // 256), 1, 1), (64, 8, 1))]
+
+
+@pytest.mark.parametrize("src,dtype", [
+    (ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n"), "float16"),
+    (ANY_HALF_PRODUCT.replace("+=!", "+=") % ("M, K", "K, N", "m, r_k", "r_k, n"), "float16"),                     # adds to what is there
+    ((ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n")).replace(" }", " O(m, n) = fmax(O(m, n), 0) }"), "float16"),
+    ((ANY_HALF_PRODUCT % ("M, K", "L, N", "m, r_k + 8", "r_k, n")).replace(" }", " where r_k in 0:4096 }"), "float16"),  # rows not read whole
+    ((ANY_HALF_PRODUCT % ("M, K", "K, N", "4095 - m, r_k", "r_k, n")).replace(" }", " where m in 0:4096 }"), "float16"),
+    ("def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }", "float32"),
+])
+def test_other_products_keep_their_tiles(src, dtype):
+    plain = src == ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n")
+    text, _ = tc.map_only(src, "f", [ShapeOnly((4096, 4104 if "+ 8" in src else 4096), dtype), ShapeOnly((4096, 4096), dtype)], f"naive;tile=128,256,32;{MATRIX}")
+    assert ("__tc::largeHalfProduct<" in text) == plain
