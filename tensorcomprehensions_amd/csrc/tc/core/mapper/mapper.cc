@@ -391,13 +391,18 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
     // blocks: outermost shared parallel variables, x first
-    int axis = 0;
+    int axis = 0, position = -1;
     for (int i = 0; i < st.numParallel && i < k.sharedDepth && axis < static_cast<int>(o.grid.size()); ++i) {
       LoopVar& v = st.vars[i];
       // a variable with a single tile has nothing to distribute and does not use up an axis
+      if (!v.vectorLane) ++position;
       if (v.vectorLane || v.numTiles == 1) continue;
       v.blockAxis = axis;
-      v.gridExtent = std::min<int64_t>(static_cast<int64_t>(o.grid[axis]), v.numTiles);
+      // The block size of a variable is the one of its place among the options' sizes as well as that of the axis it
+      // moves up to (one image of 11 groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).
+      uint64_t blocks = o.grid[axis];
+      if (position < static_cast<int>(o.grid.size())) blocks = std::max<uint64_t>(blocks, o.grid[position]);
+      v.gridExtent = std::min<int64_t>(static_cast<int64_t>(std::min<uint64_t>(blocks, std::numeric_limits<int32_t>::max())), v.numTiles);
       gridUse[axis] = std::max(gridUse[axis], v.gridExtent);
       ++axis;
     }

@@ -254,3 +254,17 @@ def test_other_products_keep_their_tiles(src, dtype):
     plain = src == ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n")
     text, _ = tc.map_only(src, "f", [ShapeOnly((4096, 4104 if "+ 8" in src else 4096), dtype), ShapeOnly((4096, 4096), dtype)], f"naive;tile=128,256,32;{MATRIX}")
     assert ("__tc::largeHalfProduct<" in text) == plain
+
+
+@pytest.mark.parametrize("shape,blocks,grid", [
+    ((1, 11, 16), "1,11", (11, 1, 1)),           # a variable of one tile uses up no axis, and no block size either
+    ((1, 11, 16), "4,3", (4, 1, 1)),
+    ((1, 1, 16), "1,1,5", (5, 1, 1)),
+    ((3, 1, 16), "2,1,5", (2, 5, 1)),
+    ((3, 5, 7), "2,4,6", (2, 4, 6)),             # none: as given
+    ((1, 5, 7), "9,2,3", (5, 3, 1)),
+])
+def test_block_sizes_keep_their_variables(shape, blocks, grid):
+    src = "def f(float(N, G, H) A, float(H, K) W) -> (O) { O(n, g, h) +=! A(n, g, h) * W(h, r_k) }"
+    _, launches = mapped(src, "f", [shape, (shape[2], 8)], f"naive;tile=1,1,1;mapToThreads=1;mapToBlocks={blocks};collapseContiguous=0")
+    assert launches[0][0] == grid
