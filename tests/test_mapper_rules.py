@@ -257,8 +257,8 @@ def test_other_products_keep_their_tiles(src, dtype):
 
 
 @pytest.mark.parametrize("shape,blocks,grid", [
-    ((1, 11, 16), "1,11", (11, 1, 1)),           # a variable of one tile uses up no axis, and no block size either
-    ((1, 11, 16), "4,3", (4, 1, 1)),
+    ((1, 11, 16), "1,11", (11, 11, 1)),          # a variable of one tile uses up no axis, and no block size either
+    ((1, 11, 16), "4,3", (4, 3, 1)),
     ((1, 1, 16), "1,1,5", (5, 1, 1)),
     ((3, 1, 16), "2,1,5", (2, 5, 1)),
     ((3, 5, 7), "2,4,6", (2, 4, 6)),             # none: as given
