@@ -19,7 +19,7 @@ def test_quotients_are_those_of_the_division(divisor, by_reciprocal):
     x[:12] = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), 1e-45, -1e-45, 3e-45, 3.4028235e38, -3.4028235e38, 1.1754944e-38, 1.0])
     src = f"def quotient(float(N) A) -> (O) {{ O(n) = A(n) / {divisor} }}"
     ex = tc.compile(src, "quotient", [x], "naive;tile=256;mapToThreads=256;mapToBlocks=65536")
-    assert ("__tc::divideBy<" in ex.compiled_source.split('extern "C"')[-1]) == by_reciprocal
+    assert ("/ __tc::Whole<" in ex.compiled_source.split('extern "C"')[-1]) == by_reciprocal
     out = tc.prepare_outputs(src, "quotient", [x])
     tc.run(ex, [x], out)
     c = eval(divisor, {}, {"N": 1})
@@ -36,7 +36,7 @@ def test_sizes_divide_by_their_reciprocal():
     src = "def mean(float(M, N) X) -> (mean) { mean(m) +=! X(m, r_n) / N }"
     X = torch.randn(64, 3448, device="cuda")
     ex = tc.compile(src, "mean", [X], "naive;tile=1;mapToThreads=256;mapToBlocks=64;matchLibraryCalls=1")
-    assert "__tc::divideBy<3448>(" in ex.compiled_source
+    assert "/ __tc::Whole<3448>()" in ex.compiled_source
     out = tc.prepare_outputs(src, "mean", [X])
     tc.run(ex, [X], out)
     # (a float sum of n terms is within n * 2^-24 of the sum of their magnitudes)
