@@ -210,35 +210,47 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
   }
 }
 
-// A matrix-core stage over reduction tiles whose blocks leave compute units idle: one block-mapped
-// variable gets the smaller tile that shortens the longest-running compute unit by a quarter or more,
-// if there is one (compute units are those of the device, or of its partition).  A compute unit's time
-// is its rounds of blocks times the output tiles of the busiest
-// wavefront and about two more for a block's staging (3x3 convolution of 16x64x57x57, 64 filters,
-// blocks of 32 filters x 11 rows, 8 channels a step: 160 blocks of 10 tiles 55.5 us, 256 blocks of 7
-// (7 rows) 46.0, 320 blocks of 6 in two rounds (6 rows) 63.9; 32x64x30x30: 128 blocks of 7 tiles 41.3,
-// 256 of 4 24.0; 1x1 over 32x128x16x16: 96 blocks of 4 tiles 13.3, 192 of 2 9.5).  Floats and
-// more than two output variables only (convolutions): products keep the rectangles of output tiles they
-// were given.  mapToBlocks sizes that hold exactly the given tiles keep those tiles.
+// A matrix-core stage whose blocks leave compute units idle: a block-mapped variable gets the smaller tile
+// that shortens the longest-running compute unit by a quarter or more, if there is one, and then another one (compute units
+// are those of the device, or of its partition).  A compute unit's time is its rounds of blocks times the output tiles
+// of the busiest wavefront, or its share of one where wavefronts divide the reduction, and about two more for a block's staging.
+//   Convolutions: any smaller number of rows, whole sixteens of filters (3x3 of 16x64x57x57, 64 filters: 160 blocks of 10
+// tiles a wavefront 55.5 us, 256 of 7 46.0, 320 of 6 in two rounds 63.9; 13x83x7x38, 38 filters: 26 blocks of 32 filters x 5 rows
+// 28.0 us, 130 of one row 12.0; 1x1 of 4x118x30x38, 21 filters: 8 blocks of 15 rows 20.0, 120 of one 4.2).  Floats only.
+//   Products of eight reduction tiles and more: sides of half the length, which keep rectangles of output tiles
+// (215x1188x1305: 84 blocks of 64x64 24.2 us, 164 of 64x32 14.8, 287 of 32x32 21.9; 430x1367x1095 27.2 and 18.1; halves
+// 322x2061x993 17.9 and 13.6; where the halves make two rounds there is nothing to gain: 691x1840x792, 143 blocks, 35.7, 36.1).
+// mapToBlocks sizes that hold exactly the given tiles keep those tiles, as maxSharedMemory keeps those of products.
 void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
-  constexpr int64_t kStaging = 2;
-  if (k.stages.size() != 1 || !o.prefetchSharedValue || !o.useSharedMemoryValue || !st.mfmaBatch.empty() || st.mfmaM.size() + st.mfmaN.size() < 3) return;
-  for (const auto& operand : st.stmts[0].rhs->args) {
-    if (st.views.at(contractionOperand(operand)->name).type.bits != 32) return;
-  }
+  constexpr int64_t kStaging = 2, kLongReduction = 8;
+  if (k.stages.size() != 1 || !o.prefetchSharedValue || !o.useSharedMemoryValue || !st.mfmaBatch.empty()) return;
+  const bool product = st.mfmaM.size() + st.mfmaN.size() == 2;
+  bool halves = false;
+  for (const auto& operand : st.stmts[0].rhs->args) halves |= st.views.at(contractionOperand(operand)->name).type.bits != 32;
+  if (product ? o.hasMaxSharedMemory : halves) return;
+  int64_t points = 1; // of a reduction tile
+  int position = 0;
   for (const auto& v : st.vars) {
-    if (!v.reduction) continue;
-    if (v.numTiles == 1 || (v.extent % v.tile != 0 && !reductionMayEndInMidTile(st, v.name))) return;
-    break;
+    if (v.reduction && v.name == st.mfmaK[0]) {
+      // (a reduction the options do not tile has its operands staged whole)
+      const bool given = o.generic.hasTiling && position < static_cast<int>(o.generic.tiling.size()) && o.generic.tiling[position] > 0;
+      if (!given) return;
+      const bool tiled = v.numTiles > 1 && (v.extent % v.tile == 0 || reductionMayEndInMidTile(st, v.name));
+      if (product && (!tiled || v.numTiles < kLongReduction)) return;
+      points *= tiled ? v.tile : v.extent;
+    } else if (v.reduction) {
+      points *= v.extent;
+    }
+    if (!v.vectorLane) ++position;
   }
-  auto isMapped = [&](int i) { return i < k.sharedDepth && !st.vars[i].vectorLane && st.vars[i].numTiles > 1; };
-  // 0: not a form this speaks of
+  auto mayBeSplit = [&](int i) { return i < k.sharedDepth && !st.vars[i].vectorLane; };
+  // in units of 1 / waves of an output tile; 0: not a form this speaks of
   auto cost = [&](int64_t& blocks) -> int64_t {
     blocks = 1;
     size_t axis = 0;
     for (int i = 0; i < st.numParallel; ++i) {
       if (st.vars[i].numTiles == 1) continue;
-      if (!isMapped(i) || axis >= o.grid.size() || st.vars[i].numTiles > static_cast<int64_t>(o.grid[axis])) return 0;
+      if (!mayBeSplit(i) || axis >= o.grid.size() || st.vars[i].numTiles > static_cast<int64_t>(o.grid[axis])) return 0;
       blocks *= st.vars[i].numTiles;
       ++axis;
     }
@@ -248,35 +260,43 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
       for (const auto& n : st.mfmaN) columns *= w.name == n ? w.tile : 1;
     }
     const int64_t tiles = ceilDiv(rows, 16) * ceilDiv(columns, 16);
-    return tiles < waves ? 0 : ceilDiv(blocks, computeUnits) * (ceilDiv(tiles, waves) + kStaging);
+    if (product && tiles < waves) return 0;
+    const int64_t shared = std::max<int64_t>(1, std::min(waves / tiles, points / 4 / StageCodegen::kMinStepsPerSplit));
+    const int64_t work = tiles >= waves ? waves * ceilDiv(tiles, waves) : ceilDiv(waves, shared);
+    return ceilDiv(blocks, computeUnits) * (work + kStaging * waves);
   };
-  int64_t blocks = 0;
-  const int64_t given = cost(blocks);
-  if (given == 0 || blocks >= computeUnits) return;
-  int best = -1;
-  int64_t bestTile = 0, bestCost = given;
-  for (int i = 0; i < st.numParallel; ++i) {
-    LoopVar& v = st.vars[i];
-    if (!isMapped(i)) continue;
-    const int64_t tile = v.tile, numTiles = v.numTiles, step = tile % 16 == 0 ? 16 : 1;
-    for (int64_t t = tile - step; t > 0; t -= step) {
-      v.tile = t;
-      v.numTiles = ceilDiv(v.extent, t);
-      int64_t unused = 0;
-      const int64_t c = cost(unused);
-      if (c > 0 && (c < bestCost || (c == bestCost && best == i))) { // (as long, of less work: the smaller tile)
-        best = i;
-        bestTile = t;
-        bestCost = c;
-      }
-    }
+  auto setTile = [&](LoopVar& v, int64_t tile) {
     v.tile = tile;
-    v.numTiles = numTiles;
+    v.numTiles = ceilDiv(v.extent, tile);
+  };
+  for (int round = 0; round < 2; ++round) {
+    int64_t blocks = 0;
+    const int64_t given = cost(blocks);
+    if (given == 0 || blocks >= computeUnits) return;
+    int best = -1;
+    int64_t bestTile = 0, bestCost = given;
+    for (int i = 0; i < st.numParallel; ++i) {
+      if (!mayBeSplit(i)) continue;
+      LoopVar& v = st.vars[i];
+      const int64_t tile = v.tile, step = product ? tile / 2 : tile > 16 ? 16 : 1;
+      if (product && tile % 32 != 0) continue;
+      for (int64_t t = product ? tile / 2 : (tile - 1) / step * step; t > 0; t -= step) {
+        setTile(v, t);
+        int64_t unused = 0;
+        const int64_t c = cost(unused);
+        // (as long, of less work: the smaller tile; of a product's two sides the second)
+        if (c > 0 && (c < bestCost || (c == bestCost && best >= 0 && (best == i || product)))) {
+          best = i;
+          bestTile = t;
+          bestCost = c;
+        }
+      }
+      setTile(v, tile);
+    }
+    if (best < 0 || 4 * bestCost > 3 * given) return;
+    setTile(st.vars[best], bestTile);
+    st.fittedToDevice = true;
   }
-  if (best < 0 || 4 * bestCost > 3 * given) return;
-  st.vars[best].tile = bestTile;
-  st.vars[best].numTiles = ceilDiv(st.vars[best].extent, bestTile);
-  st.fittedToDevice = true;
 }
 
 // Products of float16 matrices O(m, n) +=! A * B whose outputs fill the device in blocks of 256 x 256 go to

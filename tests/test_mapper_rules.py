@@ -268,3 +268,36 @@ def test_block_sizes_keep_their_variables(shape, blocks, grid):
     src = "def f(float(N, G, H) A, float(H, K) W) -> (O) { O(n, g, h) +=! A(n, g, h) * W(h, r_k) }"
     _, launches = mapped(src, "f", [shape, (shape[2], 8)], f"naive;tile=1,1,1;mapToThreads=1;mapToBlocks={blocks};collapseContiguous=0")
     assert launches[0][0] == grid
+
+
+FLOAT_PRODUCT = "def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }"
+
+
+@pytest.mark.parametrize("m,k,n,tile,changes,grid", [
+    (215, 1188, 1305, "64,64,32", "", (4, 41)),             # 84 blocks of 64x64: columns are halved
+    (430, 1367, 1095, "64,64,32", "", (7, 35)),
+    (691, 1840, 792, "64,64,32", "", (11, 13)),             # 275 would run in two rounds
+    (215, 224, 1305, "64,64,32", "", (4, 21)),              # a short reduction
+    (215, 1188, 1305, "64,64,32", "maxSharedMemory=65536", (4, 21)),
+    (215, 1188, 1305, "64,64,32", "prefetchShared=0", (4, 21)),
+    (215, 1188, 1305, "64,64,32", "mapToBlocks=4,21", (4, 21)),
+    (254, 1500, 292, "16,32,128", "", (16, 10)),            # wavefronts already share a tile
+])
+def test_products_halve_a_side_to_fill_the_device(m, k, n, tile, changes, grid):
+    _, launches = mapped(FLOAT_PRODUCT, "f", [(m, k), (k, n)], f"naive;tile={tile};{MATRIX};{changes}")
+    assert sorted(launches[0][0][:2]) == sorted(grid)
+
+
+@pytest.mark.parametrize("sizes,kernel,tile,blocks", [
+    ((13, 83, 38, 7, 38), 3, "1,32,5,0,8", 13 * 2 * 5),     # one row a block: wavefronts share the reduction of six tiles
+    ((4, 118, 21, 30, 38), 1, "1,32,15,0,8", 4 * 30),       # a reduction whose given tile is dropped
+    ((4, 118, 21, 30, 38), 1, "1,32,15,0,0", 4 * 2),        # one that is given whole
+    ((1, 64, 64, 57, 57), 3, "1,32,11,0,8", 2 * 55),
+])
+def test_convolutions_get_small_tiles_where_units_are_idle(sizes, kernel, tile, blocks):
+    n, c, m, h, w = sizes
+    src = "def f(float(N, C, H, W) I, float(M, C, KH, KW) W1) -> (O) { O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw) }"
+    _, launches = mapped(src, "f", [(n, c, h, w), (m, c, kernel, kernel)],
+                         f"naive;tile={tile};mapToThreads=64,8;mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+    grid = launches[0][0]
+    assert grid[0] * grid[1] * grid[2] == blocks
