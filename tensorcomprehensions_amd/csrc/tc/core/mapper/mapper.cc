@@ -365,6 +365,109 @@ void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions&
   k.block = {{64, waves, 1}};
 }
 
+// A contraction whose threads keep whole sums (no matrix cores, no LDS, one axis of threads) under tile sizes that were made
+// for other extents.  Returns the innermost variable where it takes a block axis behind those of the options.
+//   A variable without a block axis is not walked tile by tile where all its points fit the registers: every walk
+// reads the operands that do not depend on it again (tensordot of 7x404x9x4x9x21 in tiles of two of the 4: 12.6 -> 5.7 us).
+//   Blocks with fewer than six wavefronts a compute unit get less work each, until there are sixteen: a block's loads wait for
+// each other and there is nobody to fill in.  First the points a thread takes of the innermost variable go to blocks
+// of their own, then the largest tile of the others is halved; more blocks along a variable than the options allow
+// it there are not (tensordot 4x17x8x4x47x25, 12 blocks of 256 threads and 80 sums each, 29.7 us; 180 blocks of 8 sums
+// 3.9; 10x285x12x2x29x31, 360 blocks 45.7, 1440 32.3; 7x33x12x2x39x56 83.6 and 7.7).  Beyond that there is nothing to gain:
+// 16x286x3x2x25x30, 576 blocks of nine wavefronts a unit, 16.1 us, in 1728 shorter pieces of its rows 20.6.
+const LoopVar* spreadContraction(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits) {
+  constexpr int64_t kFewWaves = 6, kWavesPerUnit = 16, kMostSums = 64;
+  if (k.stages.size() != 1 || st.mfma || st.atomic || o.useSharedMemoryValue || !o.generic.hasTiling || k.sharedDepth < st.numParallel) return nullptr;
+  if (st.stmts.empty() || st.stmts[0].redVars.empty() || o.generic.matchLibraryCallsValue) return nullptr;
+  for (size_t a = 1; a < o.block.size(); ++a) {
+    if (o.block[a] != 1) return nullptr;
+  }
+  std::vector<LoopVar*> vars; // parallel, the lanes of a vector left out
+  int64_t lanes = 1;
+  for (int i = 0; i < st.numParallel; ++i) {
+    if (st.vars[i].vectorLane) lanes *= st.vars[i].extent;
+    else vars.push_back(&st.vars[i]);
+  }
+  if (vars.size() < 2) return nullptr;
+  LoopVar& inner = *vars.back();
+  const int64_t unroll = o.generic.hasUnroll ? static_cast<int64_t>(o.generic.unrollValue) : 1;
+  const int64_t threads = std::min<int64_t>(static_cast<int64_t>(o.block[0]), inner.tile);
+  auto setTile = [](LoopVar& v, int64_t tile) {
+    v.tile = tile;
+    v.numTiles = ceilDiv(v.extent, tile);
+  };
+  auto isDistributed = [&](const LoopVar& v) {
+    size_t axis = 0;
+    for (const LoopVar* w : vars) {
+      if (w->numTiles == 1) continue;
+      if (w == &v) return axis < o.grid.size();
+      ++axis;
+    }
+    return false;
+  };
+  // 0: more tiles than blocks, which are then the ones asked for
+  auto blocks = [&]() -> int64_t {
+    int64_t n = 1;
+    size_t axis = 0;
+    for (size_t i = 0; i < vars.size(); ++i) {
+      if (vars[i]->numTiles == 1 || (vars[i] == &inner && axis >= o.grid.size())) {
+        n *= vars[i]->numTiles;
+        continue;
+      }
+      if (axis >= o.grid.size()) continue;
+      uint64_t most = o.grid[axis];
+      if (i < o.grid.size()) most = std::max<uint64_t>(most, o.grid[i]);
+      if (static_cast<uint64_t>(vars[i]->numTiles) > most) return 0;
+      n *= vars[i]->numTiles;
+      ++axis;
+    }
+    return n;
+  };
+  auto sums = [&]() {
+    int64_t n = lanes * ceilDiv(inner.tile, threads);
+    for (const LoopVar* v : vars) n *= v == &inner ? 1 : v->tile;
+    return n;
+  };
+  if (blocks() == 0) return nullptr;
+  auto waves = [&]() { return blocks() * ceilDiv(threads, limits.wavefront); };
+  const bool isShort = waves() < kFewWaves * limits.computeUnits;
+  auto largestOuter = [&]() {
+    LoopVar* best = nullptr;
+    for (LoopVar* v : vars) {
+      if (v != &inner && v->tile > 1 && (v->numTiles == 1 ? v->tile > 2 : isDistributed(*v)) && (!best || v->tile > best->tile)) best = v;
+    }
+    return best;
+  };
+  const bool hadAxis = inner.numTiles > 1;
+  if (isShort && (!hadAxis || isDistributed(inner))) {
+    int distributed = 0;
+    for (const LoopVar* v : vars) distributed += v != &inner && v->numTiles > 1 && isDistributed(*v);
+    const int64_t given = inner.tile, most = ceilDiv(given, threads);
+    const int64_t per = std::max<int64_t>(1, most / ceilDiv(kWavesPerUnit * limits.computeUnits, waves()));
+    if (distributed < 3 && per < most) {
+      setTile(inner, per * threads);
+      if (blocks() == 0) setTile(inner, given);
+    }
+  }
+  for (LoopVar* v : vars) {
+    if (v == &inner || v->numTiles == 1 || isDistributed(*v)) continue;
+    const int64_t tile = v->tile;
+    setTile(*v, v->extent);
+    if (sums() > std::min(kMostSums, unroll)) setTile(*v, tile);
+  }
+  while (isShort && waves() < kWavesPerUnit * limits.computeUnits) {
+    LoopVar* v = largestOuter();
+    if (!v) break;
+    const int64_t tile = v->tile, numTiles = v->numTiles;
+    setTile(*v, ceilDiv(v->tile, 2));
+    if (blocks() == 0 || (numTiles == 1 && !isDistributed(*v))) {
+      setTile(*v, tile);
+      break;
+    }
+  }
+  return inner.numTiles > 1 && !hadAxis ? &inner : nullptr;
+}
+
 void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
   const HipMappingOptions& o = kc.opts;
   KernelPlan& k = kc.k;
@@ -411,13 +514,21 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) takeLargeHalfProduct(k, st, o, waves, limits, kc.wide);
     if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
+    const LoopVar* spread = spreadContraction(k, st, o, limits);
     // blocks: outermost shared parallel variables, x first
     int axis = 0, position = -1;
-    for (int i = 0; i < st.numParallel && i < k.sharedDepth && axis < static_cast<int>(o.grid.size()); ++i) {
+    for (int i = 0; i < st.numParallel && i < k.sharedDepth && axis < 3; ++i) {
       LoopVar& v = st.vars[i];
       // a variable with a single tile has nothing to distribute and does not use up an axis
       if (!v.vectorLane) ++position;
       if (v.vectorLane || v.numTiles == 1) continue;
+      if (axis >= static_cast<int>(o.grid.size())) {
+        if (&v != spread) continue;
+        v.blockAxis = axis;
+        v.gridExtent = v.numTiles;
+        gridUse[axis] = std::max(gridUse[axis], v.gridExtent);
+        break;
+      }
       v.blockAxis = axis;
       // The block size of a variable is the one of its place among the options' sizes as well as that of the axis it
       // moves up to (one image of 11 groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).

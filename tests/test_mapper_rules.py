@@ -301,3 +301,28 @@ def test_convolutions_get_small_tiles_where_units_are_idle(sizes, kernel, tile, 
                          f"naive;tile={tile};mapToThreads=64,8;mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
     grid = launches[0][0]
     assert grid[0] * grid[1] * grid[2] == blocks
+
+
+TENSORDOT = "def f(float(N, C1, C2, H, W) A, float(N, C2, C3, H, W) B) -> (O) { O(n, c1, c3, h, w) +=! A(n, c1, r_c2, h, w) * B(n, r_c2, c3, h, w) }"
+STREAM = "naive;tile=1,8,2,0;mapToThreads=256;mapToBlocks=32,64;unroll=128;vectorWidth=4;useReadOnlyCache=1"
+
+
+@pytest.mark.parametrize("sizes,changes,grid,sums", [
+    ((32, 512, 8, 2, 28, 28), "", (32, 64, 1), 64),                 # blocks enough: as given
+    ((16, 286, 3, 2, 25, 30), "", (16, 36, 1), 48),                 # nine wavefronts a compute unit
+    ((4, 17, 8, 4, 47, 25), "", (4, 9, 5), 8),                      # 47 x 25 points to five blocks, then two of the 17
+    ((4, 17, 8, 4, 47, 25), "useSharedMemory=1", (4, 3, 1), 80),
+    ((4, 17, 8, 4, 47, 25), "mapToThreads=128,2", (4, 3, 1), None),
+    ((4, 17, 8, 4, 47, 25), "mapToBlocks=4,2", (4, 2, 1), 80),      # fewer blocks than tiles: the ones asked for
+    ((4, 17, 8, 4, 47, 25), "mapToBlocks=4,3", (4, 3, 5), 32),      # no more blocks along c1
+    ((1, 93, 3, 3, 25, 25), "", (47, 2, 3), 4),                     # (with one n, c3 has a block axis)
+    ((32, 512, 8, 4, 28, 28), "", (32, 64, 1), 64),                 # 128 sums would not fit
+    ((32, 512, 8, 3, 7, 7), "", (32, 64, 1), 24),                   # all of c3 at once
+    ((32, 512, 8, 3, 7, 7), "unroll=16", (32, 64, 1), 16),          # ... where the loops may be unrolled
+])
+def test_tiles_made_for_other_sizes(sizes, changes, grid, sums):
+    n, c1, c2, c3, h, w = sizes
+    text, launches = mapped(TENSORDOT, "f", [(n, c1, c2, h, w), (n, c2, c3, h, w)], f"{STREAM};{changes}")
+    assert launches[0][0] == grid
+    if sums is not None:
+        assert f"float acc_[{sums}];" in text
