@@ -217,8 +217,9 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
 //   Convolutions: any smaller number of rows, whole sixteens of filters (3x3 of 16x64x57x57, 64 filters: 160 blocks of 10
 // tiles a wavefront 55.5 us, 256 of 7 46.0, 320 of 6 in two rounds 63.9; 13x83x7x38, 38 filters: 26 blocks of 32 filters x 5 rows
 // 28.0 us, 130 of one row 12.0; 1x1 of 4x118x30x38, 21 filters: 8 blocks of 15 rows 20.0, 120 of one 4.2).  Floats only.
-//   Products of eight reduction tiles and more: sides of half the length, which keep rectangles of output tiles
-// (215x1188x1305: 84 blocks of 64x64 24.2 us, 164 of 64x32 14.8, 287 of 32x32 21.9; 430x1367x1095 27.2 and 18.1; halves
+//   Products of eight reduction tiles and more: sides of half the length and more whose output tiles divide into rectangles for the
+// wavefronts (halves: of half the length), already for a fifth (881x655x2389: 133 blocks of 128x128 47.8 us, 210 of 128x80 38.3, 228 of 80x128
+// 35.9; 1500x800x1700: 168 blocks 56.8, 224 of 96x128 46.8; 215x1188x1305: 84 blocks of 64x64 24.2 us, 164 of 64x32 14.8, 287 of 32x32 21.9; 430x1367x1095 27.2 and 18.1; halves
 // 322x2061x993 17.9 and 13.6; where the halves make two rounds there is nothing to gain: 691x1840x792, 143 blocks, 35.7, 36.1).
 // mapToBlocks sizes that hold exactly the given tiles keep those tiles, as maxSharedMemory keeps those of products.
 void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
@@ -244,6 +245,12 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     if (!v.vectorLane) ++position;
   }
   auto mayBeSplit = [&](int i) { return i < k.sharedDepth && !st.vars[i].vectorLane; };
+  auto inRectangles = [&](int64_t rowTiles, int64_t columnTiles) {
+    for (int64_t wm = 1; wm <= waves; ++wm) {
+      if (waves % wm == 0 && rowTiles % wm == 0 && columnTiles % (waves / wm) == 0) return true;
+    }
+    return false;
+  };
   // in units of 1 / waves of an output tile; 0: not a form this speaks of
   auto cost = [&](int64_t& blocks) -> int64_t {
     blocks = 1;
@@ -260,7 +267,7 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
       for (const auto& n : st.mfmaN) columns *= w.name == n ? w.tile : 1;
     }
     const int64_t tiles = ceilDiv(rows, 16) * ceilDiv(columns, 16);
-    if (product && tiles < waves) return 0;
+    if (product && (tiles < waves || !inRectangles(ceilDiv(rows, 16), ceilDiv(columns, 16)))) return 0;
     const int64_t shared = std::max<int64_t>(1, std::min(waves / tiles, points / 4 / StageCodegen::kMinStepsPerSplit));
     const int64_t work = tiles >= waves ? waves * ceilDiv(tiles, waves) : ceilDiv(waves, shared);
     return ceilDiv(blocks, computeUnits) * (work + kStaging * waves);
@@ -274,26 +281,27 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     const int64_t given = cost(blocks);
     if (given == 0 || blocks >= computeUnits) return;
     int best = -1;
-    int64_t bestTile = 0, bestCost = given;
+    int64_t bestTile = 0, bestCost = given, bestBlocks = 0;
     for (int i = 0; i < st.numParallel; ++i) {
       if (!mayBeSplit(i)) continue;
       LoopVar& v = st.vars[i];
-      const int64_t tile = v.tile, step = product ? tile / 2 : tile > 16 ? 16 : 1;
-      if (product && tile % 32 != 0) continue;
-      for (int64_t t = product ? tile / 2 : (tile - 1) / step * step; t > 0; t -= step) {
+      const int64_t tile = v.tile, step = product && halves ? tile / 2 : product || tile > 16 ? 16 : 1;
+      if (product && tile % (halves ? 32 : 16) != 0) continue;
+      for (int64_t t = (tile - 1) / step * step; t > 0 && (!product || 2 * t >= tile); t -= step) {
         setTile(v, t);
-        int64_t unused = 0;
-        const int64_t c = cost(unused);
-        // (as long, of less work: the smaller tile; of a product's two sides the second)
-        if (c > 0 && (c < bestCost || (c == bestCost && best >= 0 && (best == i || product)))) {
+        int64_t n = 0;
+        const int64_t c = cost(n);
+        // (as long, of less work: the smaller tile; of a product's two sides the second, if not a long one of clearly fewer blocks)
+        if (c > 0 && (c < bestCost || (c == bestCost && best >= 0 && (best == i || (product && (tile <= 64 || halves || 20 * n >= 19 * bestBlocks)))))) {
           best = i;
           bestTile = t;
           bestCost = c;
+          bestBlocks = n;
         }
       }
       setTile(v, tile);
     }
-    if (best < 0 || 4 * bestCost > 3 * given) return;
+    if (best < 0 || (product && !halves ? 5 * bestCost > 4 * given : 4 * bestCost > 3 * given)) return;
     setTile(st.vars[best], bestTile);
     st.fittedToDevice = true;
   }

@@ -147,3 +147,15 @@ def test_errors_on_deviates_stay_within_those_of_float_sums(m, k, n, half):
         got = run(B.HALF_MATMUL if half else B.MATMUL, "half_matmul" if half else "matmul", [A, Bm], options).astype(np.float64)
         assert (np.abs(got - want) <= bound).all()
         assert np.linalg.norm(got - want) <= np.sqrt(k) * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("m,k,n", [(881, 130, 2389), (1479, 221, 1728), (1730, 171, 1478), (764, 258, 3237), (1500, 160, 1700), (2040, 128, 1100), (150, 200, 140)])
+def test_products_with_shortened_sides(m, k, n, waves):
+    """Blocks of 80 to 112 rows or columns (128 given), where those of the given tiles leave compute units idle."""
+    print(f"product {m}x{k}x{n} waves={waves}", flush=True)
+    A, Bm = ints((m, k), m + k, np.float32), ints((k, n), k + n, np.float32)
+    want = A @ Bm
+    options = f"naive;tile=128,128,16;mapToThreads=64,{waves};{TAIL}"
+    assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), want)
+    assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), want)

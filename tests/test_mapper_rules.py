@@ -326,3 +326,17 @@ def test_tiles_made_for_other_sizes(sizes, changes, grid, sums):
     assert launches[0][0] == grid
     if sums is not None:
         assert f"float acc_[{sums}];" in text
+
+
+@pytest.mark.parametrize("m,k,n,tile,changes,grid", [
+    (881, 655, 2389, "128,128,16", "", (12, 19, 1)),            # 80 x 128: five tiles a wavefront for eight
+    (1500, 800, 1700, "128,128,16", "", (12, 18, 1)),           # 128 x 96, a fifth less
+    (1500, 112, 1700, "128,128,16", "", (12, 14, 1)),           # seven reduction tiles: as given
+    (2048, 512, 2048, "128,128,16", "", (16, 16, 1)),           # blocks enough
+    (881, 655, 2389, "128,128,16", "mapToThreads=64,4", (12, 19, 1)),
+    (881, 655, 2389, "128,128,16", "mapToBlocks=7,19", (7, 19, 1)),
+])
+def test_products_shorten_a_side_to_fill_the_device(m, k, n, tile, changes, grid):
+    text, launches = mapped("def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }", "f", [(m, k), (k, n)],
+                            f"naive;tile={tile};{MATRIX};{changes}")
+    assert launches[0][0] == grid
