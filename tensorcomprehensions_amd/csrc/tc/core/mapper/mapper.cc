@@ -221,9 +221,12 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
 // wavefronts (halves: of half the length), already for a fifth (881x655x2389: 133 blocks of 128x128 47.8 us, 210 of 128x80 38.3, 228 of 80x128
 // 35.9; 1500x800x1700: 168 blocks 56.8, 224 of 96x128 46.8; 215x1188x1305: 84 blocks of 64x64 24.2 us, 164 of 64x32 14.8, 287 of 32x32 21.9; 430x1367x1095 27.2 and 18.1; halves
 // 322x2061x993 17.9 and 13.6; where the halves make two rounds there is nothing to gain: 691x1840x792, 143 blocks, 35.7, 36.1).
+//   Products whose blocks make a second round for a few: a side up to half as long again under which there is one, where the
+// estimate says two thirds (2100x900x2100: 289 blocks of 128x128 117.7 us, 255 of 144x128 85.2; 1100x2000x1100: 324 of 64x64 72.6,
+// 216 of 96x64 61.7; 1400x600x1100, three quarters: 396 of 64x64 25.8, 198 of 128x64 26.9).
 // mapToBlocks sizes that hold exactly the given tiles keep those tiles, as maxSharedMemory keeps those of products.
 void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
-  constexpr int64_t kStaging = 2, kLongReduction = 8;
+  constexpr int64_t kStaging = 2, kLongReduction = 8, kLongSidesLds = 64 << 10;
   if (k.stages.size() != 1 || !o.prefetchSharedValue || !o.useSharedMemoryValue || !st.mfmaBatch.empty()) return;
   const bool product = st.mfmaM.size() + st.mfmaN.size() == 2;
   bool halves = false;
@@ -276,6 +279,35 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     v.tile = tile;
     v.numTiles = ceilDiv(v.extent, tile);
   };
+  int64_t blocks = 0;
+  const int64_t given = cost(blocks);
+  if (product && !halves && blocks > computeUnits && given > 0) {
+    LoopVar* best = nullptr;
+    int64_t bestTile = 0, bestCost = given;
+    for (int i = 0; i < st.numParallel; ++i) {
+      if (!mayBeSplit(i)) continue;
+      LoopVar& v = st.vars[i];
+      const int64_t tile = v.tile;
+      for (int64_t t = tile + 16; tile % 16 == 0 && 2 * t <= 3 * tile; t += 16) {
+        setTile(v, t);
+        int64_t n = 0, sides = 0;
+        const int64_t c = cost(n);
+        for (int j = 0; j < st.numParallel; ++j) sides += st.vars[j].tile;
+        const bool fits = sides * (points + 4) * 4 * 2 <= kLongSidesLds;
+        if (fits && c > 0 && n <= computeUnits && c < bestCost) {
+          best = &v;
+          bestTile = t;
+          bestCost = c;
+        }
+      }
+      setTile(v, tile);
+    }
+    if (best && 20 * bestCost <= 13 * given) {
+      setTile(*best, bestTile);
+      st.fittedToDevice = true;
+    }
+    return;
+  }
   for (int round = 0; round < 2; ++round) {
     int64_t blocks = 0;
     const int64_t given = cost(blocks);

@@ -150,12 +150,20 @@ def test_errors_on_deviates_stay_within_those_of_float_sums(m, k, n, half):
 
 
 @pytest.mark.parametrize("waves", [4, 8])
-@pytest.mark.parametrize("m,k,n", [(881, 130, 2389), (1479, 221, 1728), (1730, 171, 1478), (764, 258, 3237), (1500, 160, 1700), (2040, 128, 1100), (150, 200, 140)])
-def test_products_with_shortened_sides(m, k, n, waves):
-    """Blocks of 80 to 112 rows or columns (128 given), where those of the given tiles leave compute units idle."""
+@pytest.mark.parametrize("m,k,n", [(881, 130, 2389), (1479, 221, 1728), (1730, 171, 1478), (764, 258, 3237), (1500, 160, 1700), (2040, 128, 1100), (150, 200, 140), (2100, 130, 2100)])
+def test_products_with_fitted_sides(m, k, n, waves):
+    """Blocks of 80 to 144 rows or columns (128 given), where those of the given tiles leave compute units idle."""
     print(f"product {m}x{k}x{n} waves={waves}", flush=True)
     A, Bm = ints((m, k), m + k, np.float32), ints((k, n), k + n, np.float32)
     want = A @ Bm
     options = f"naive;tile=128,128,16;mapToThreads=64,{waves};{TAIL}"
     assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), want)
     assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), want)
+
+
+@pytest.mark.parametrize("m,k,n", [(1100, 264, 1100), (1050, 300, 1080), (1150, 256, 1200)])
+def test_products_with_longer_sides(m, k, n):
+    A, Bm = ints((m, k), m + k, np.float32), ints((k, n), k + n, np.float32)
+    options = f"naive;tile=64,64,32;mapToThreads=64,8;{TAIL}"
+    assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), A @ Bm)
+    assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), A @ Bm)

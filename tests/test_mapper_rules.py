@@ -333,10 +333,14 @@ def test_tiles_made_for_other_sizes(sizes, changes, grid, sums):
     (1500, 800, 1700, "128,128,16", "", (12, 18, 1)),           # 128 x 96, a fifth less
     (1500, 112, 1700, "128,128,16", "", (12, 14, 1)),           # seven reduction tiles: as given
     (2048, 512, 2048, "128,128,16", "", (16, 16, 1)),           # blocks enough
+    (2100, 900, 2100, "128,128,16", "", (15, 17, 1)),           # 144 x 128: one round of blocks for two
+    (1100, 2000, 1100, "64,64,32", "", (12, 18, 1)),            # 96 x 64
+    (1400, 600, 1100, "64,64,32", "", (22, 18, 1)),             # 128 x 64 is no gain
+    (1100, 2000, 1100, "64,64,32", "maxSharedMemory=160000", (18, 18, 1)),
     (881, 655, 2389, "128,128,16", "mapToThreads=64,4", (12, 19, 1)),
     (881, 655, 2389, "128,128,16", "mapToBlocks=7,19", (7, 19, 1)),
 ])
-def test_products_shorten_a_side_to_fill_the_device(m, k, n, tile, changes, grid):
+def test_sides_of_products_fit_the_device(m, k, n, tile, changes, grid):
     text, launches = mapped("def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }", "f", [(m, k), (k, n)],
                             f"naive;tile={tile};{MATRIX};{changes}")
     assert launches[0][0] == grid
