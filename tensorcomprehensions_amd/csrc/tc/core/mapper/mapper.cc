@@ -224,6 +224,9 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
 //   Products whose blocks make a second round for a few: a side up to half as long again under which there is one, where the
 // estimate says two thirds (2100x900x2100: 289 blocks of 128x128 117.7 us, 255 of 144x128 85.2; 1100x2000x1100: 324 of 64x64 72.6,
 // 216 of 96x64 61.7; 1400x600x1100, three quarters: 396 of 64x64 25.8, 198 of 128x64 26.9).
+//   Products whose wavefronts share the reduction of a tile, on half the compute units or fewer: half the longer side, as the
+// staging of a block is what takes the time (116x2960x204: 56 blocks of 16x32 14.6 us, 104 of 16x16 9.5; 108x1643x127 7.8 and 6.1;
+// 128x1000x1024, 256 blocks, 6.1 and 9.9).
 // mapToBlocks sizes that hold exactly the given tiles keep those tiles, as maxSharedMemory keeps those of products.
 void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
   constexpr int64_t kStaging = 2, kLongReduction = 8, kLongSidesLds = 64 << 10;
@@ -255,8 +258,10 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     return false;
   };
   // in units of 1 / waves of an output tile; 0: not a form this speaks of
+  bool onGrid = false, fewTiles = false; // (every tile has a block; fewer output tiles than wavefronts)
   auto cost = [&](int64_t& blocks) -> int64_t {
     blocks = 1;
+    onGrid = fewTiles = false;
     size_t axis = 0;
     for (int i = 0; i < st.numParallel; ++i) {
       if (st.vars[i].numTiles == 1) continue;
@@ -270,6 +275,8 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
       for (const auto& n : st.mfmaN) columns *= w.name == n ? w.tile : 1;
     }
     const int64_t tiles = ceilDiv(rows, 16) * ceilDiv(columns, 16);
+    onGrid = true;
+    fewTiles = tiles < waves;
     if (product && (tiles < waves || !inRectangles(ceilDiv(rows, 16), ceilDiv(columns, 16)))) return 0;
     const int64_t shared = std::max<int64_t>(1, std::min(waves / tiles, points / 4 / StageCodegen::kMinStepsPerSplit));
     const int64_t work = tiles >= waves ? waves * ceilDiv(tiles, waves) : ceilDiv(waves, shared);
@@ -281,6 +288,20 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
   };
   int64_t blocks = 0;
   const int64_t given = cost(blocks);
+  if (product && !halves && fewTiles && 2 * blocks <= computeUnits) {
+    LoopVar* longer = nullptr;
+    for (int i = 0; i < st.numParallel; ++i) {
+      LoopVar& v = st.vars[i];
+      if (mayBeSplit(i) && v.tile % 32 == 0 && (!longer || v.tile >= longer->tile)) longer = &v;
+    }
+    if (!longer) return;
+    const int64_t tile = longer->tile;
+    setTile(*longer, tile / 2);
+    cost(blocks);
+    if (blocks > computeUnits || !onGrid) setTile(*longer, tile);
+    else st.fittedToDevice = true;
+    return;
+  }
   if (product && !halves && blocks > computeUnits && given > 0) {
     LoopVar* best = nullptr;
     int64_t bestTile = 0, bestCost = given;

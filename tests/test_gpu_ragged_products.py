@@ -167,3 +167,12 @@ def test_products_with_longer_sides(m, k, n):
     options = f"naive;tile=64,64,32;mapToThreads=64,8;{TAIL}"
     assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), A @ Bm)
     assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), A @ Bm)
+
+
+@pytest.mark.parametrize("m,k,n", [(116, 2960, 204), (108, 1643, 127), (17, 1100, 33), (16, 1024, 32), (64, 2048, 897)])
+def test_few_blocks_over_long_reductions(m, k, n):
+    """Blocks of 16 x 16 outputs (16 x 32 given), eight wavefronts sharing the reduction."""
+    A, Bm = ints((m, k), m + k, np.float32), ints((k, n), k + n, np.float32)
+    options = f"naive;tile=16,32,128;mapToThreads=64,8;{TAIL}"
+    assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), A @ Bm)
+    assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), A @ Bm)

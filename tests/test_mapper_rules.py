@@ -336,6 +336,10 @@ def test_tiles_made_for_other_sizes(sizes, changes, grid, sums):
     (2100, 900, 2100, "128,128,16", "", (15, 17, 1)),           # 144 x 128: one round of blocks for two
     (1100, 2000, 1100, "64,64,32", "", (12, 18, 1)),            # 96 x 64
     (1400, 600, 1100, "64,64,32", "", (22, 18, 1)),             # 128 x 64 is no gain
+    (116, 2960, 204, "16,32,128", "", (8, 13, 1)),              # 16 x 16: half the staging a block
+    (116, 896, 204, "16,32,128", "", (8, 7, 1)),
+    (128, 2960, 1024, "16,32,128", "", (32, 8, 1)),
+    (116, 2960, 204, "16,32,128", "mapToBlocks=8,7", (8, 7, 1)),
     (1100, 2000, 1100, "64,64,32", "maxSharedMemory=160000", (18, 18, 1)),
     (881, 655, 2389, "128,128,16", "mapToThreads=64,4", (12, 19, 1)),
     (881, 655, 2389, "128,128,16", "mapToBlocks=7,19", (7, 19, 1)),
