@@ -50,6 +50,19 @@ def test_products_are_exact(a_transposed, b_transposed, m, n, k, offsets):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("offsets", [(0, 0), (1, 3)])
+@pytest.mark.parametrize("k", [257, 259, 260, 321])
+def test_last_reduction_tiles_of_a_few_rows(k, offsets):
+    """The reduction outermost in both operands may have any number of points: pieces of the last tile without a row."""
+    A, B = ints((k, 264), 8, offsets[0]), ints((k, 256), 9, offsets[1])
+    print(k, offsets, flush=True)
+    ex = tc.compile(source(True, False), "product", [A, B], OPTIONS)
+    assert "__tc::largeHalfProduct<" in ex.compiled_source.split('extern "C"')[-1]
+    out = tc.prepare_outputs(source(True, False), "product", [A, B])
+    tc.run(ex, [A, B], out)
+    assert torch.equal(out[0], A.float().t() @ B.float())
+
+
 @pytest.mark.parametrize("m,n,k", [(257, 511, 264), (510, 259, 320)])
 def test_outputs_of_any_size(m, n, k):
     """Rows and columns need be no multiples of anything where the reduction is innermost in both operands."""
