@@ -91,7 +91,7 @@ def operand():
 
     once(r"__builtin_amdgcn_make_buffer_rsrc\(", "resource(")
     once(r"__amdgpu_buffer_rsrc_t", "Resource")
-    once(r'asm volatile\("s_mov_b32 m0[^;]*?"v"\(from\), "s"\(rs\),\s*"s"\((.*?)\)\s*: "[^;]*;', r"copied(from, rs, \1, dead);")
+    once(r'asm volatile\("s_mov_b32 m0[^;]*?"v"\(from\),\s*"s"\(rs\),\s*"s"\((.*?)\)\s*: "[^;]*;', r"copied(from, rs, \1, dead);")
     once(r'asm volatile\("" : "\+v"\(from\)\);', "")
     once(r"\*\(const halfx8u\*\)(\(.*?\));", r"loaded\1;")
     once(r"\*\(__attribute__\(\(address_space\(3\)\)\) halfx8\*\)\((.*?)\) = v;", r"stored(\1, v);")
@@ -114,3 +114,13 @@ def test_copies_stay_inside_their_operand(tmp_path):
                     str(source), "-o", binary], check=True)
     run = subprocess.run([binary], capture_output=True, text=True)
     assert run.returncode == 0 and run.stdout == "in bounds\n", run.stdout + run.stderr
+
+
+def test_copies_wait_for_the_register_they_read():
+    """m0, the place in LDS, is written by the instruction in front: one wait state has to lie between them (the compiler puts
+    s_nop there where it makes the copy itself), and the assembly says that it writes m0."""
+    text, _ = tc.map_only("def f(float16(M, K) A, float16(N, K) B) -> (O) { O(m, n) +=! float(A(m, r_k)) * float(B(n, r_k)) }", "f",
+                          [ShapeOnly((4096, 4096), "float16")] * 2,
+                          "naive;tile=256,256,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+    blocks = [b for b in re.findall(r"asm volatile\((.*?)\);\n", text, flags=re.S) if "m0" in b]
+    assert blocks and all(re.search(r"s_mov_b32 m0, %0\\n\\ts_nop \d\\n\\tbuffer_load", b) and b.rstrip().endswith('"m0"') for b in blocks)
