@@ -348,3 +348,17 @@ def test_sides_of_products_fit_the_device(m, k, n, tile, changes, grid):
     text, launches = mapped("def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }", "f", [(m, k), (k, n)],
                             f"naive;tile={tile};{MATRIX};{changes}")
     assert launches[0][0] == grid
+
+
+@pytest.mark.parametrize("divisor,known", [
+    ("(float(uint32(3 - 5)) + 11)", False),     # 4294967305
+    ("(float(uint32(3) - uint32(5)) + 11)", False),
+    ("(float(uint64(N - 5)) + 11)", False),
+    ("(N - 5 + 11)", False),                    # (9: a step of it is negative)
+    ("(float(uint32(N)) + 6)", True),
+    ("(N + 11 - 5)", True),
+])
+def test_divisors_of_unsigned_steps(divisor, known):
+    """A divisor counts as a known whole number only where no step of it is negative."""
+    text, _ = mapped("def f(float(N) A) -> (O) { O(n) = A(n) / %s }" % divisor, "f", [(3,)], "naive;tile=256;mapToThreads=256")
+    assert ("/ __tc::Whole<9>()" in text.split('extern "C"')[-1]) == known
