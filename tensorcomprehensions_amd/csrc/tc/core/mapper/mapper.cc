@@ -428,12 +428,16 @@ void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions&
 
 // A contraction whose threads keep whole sums (no matrix cores, no LDS, one axis of threads) under tile sizes that were made
 // for other extents.  Returns the innermost variable where it takes a block axis behind those of the options.
-//   A variable without a block axis is not walked tile by tile where all its points fit the registers: every walk
-// reads the operands that do not depend on it again (tensordot of 7x404x9x4x9x21 in tiles of two of the 4: 12.6 -> 5.7 us).
+//   A variable without a block axis is not walked tile by tile where all its points fit the registers under the tiles given
+// to the others: every walk reads the operands that do not depend on it again (tensordot of 7x404x9x4x9x21 in tiles of two of
+// the 4: 12.6 -> 5.7 us).  Where they would fit only once the tiles of others are halved the walk stays: 90 such tensordots
+// took 0.5 to 1.5 times as long with the variable whole, as often longer as shorter.
 //   Blocks with fewer than six wavefronts a compute unit get less work each, until there are sixteen: a block's loads wait for
 // each other and there is nobody to fill in.  First the points a thread takes of the innermost variable go to blocks
 // of their own, then the largest tile of the others is halved; more blocks along a variable than the options allow
-// it there are not (tensordot 4x17x8x4x47x25, 12 blocks of 256 threads and 80 sums each, 29.7 us; 180 blocks of 8 sums
+// it there are not, and no variable loses its block axis to one in front of it, unless all its points fit the registers: it
+// would be walked in every block (3x7x15x79x14x13, c1 on the axis of 40 tiles of c3: 33.2 us, 12.4 as given;
+// 2x84x12x3x49x37 in tiles of four of c3 under mapToBlocks=32,64,8: 17.2 and 8.1) (tensordot 4x17x8x4x47x25, 12 blocks of 256 threads and 80 sums each, 29.7 us; 180 blocks of 8 sums
 // 3.9; 10x285x12x2x29x31, 360 blocks 45.7, 1440 32.3; 7x33x12x2x39x56 83.6 and 7.7).  Beyond that there is nothing to gain:
 // 16x286x3x2x25x30, 576 blocks of nine wavefronts a unit, 16.1 us, in 1728 shorter pieces of its rows 20.6.
 const LoopVar* spreadContraction(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits) {
@@ -451,36 +455,36 @@ const LoopVar* spreadContraction(const KernelPlan& k, StagePlan& st, const HipMa
   }
   if (vars.size() < 2) return nullptr;
   LoopVar& inner = *vars.back();
-  const int64_t unroll = o.generic.hasUnroll ? static_cast<int64_t>(o.generic.unrollValue) : 1;
+  const int64_t mostSums = std::min<int64_t>(kMostSums, o.generic.hasUnroll ? static_cast<int64_t>(o.generic.unrollValue) : 1);
   const int64_t threads = std::min<int64_t>(static_cast<int64_t>(o.block[0]), inner.tile);
   auto setTile = [](LoopVar& v, int64_t tile) {
     v.tile = tile;
     v.numTiles = ceilDiv(v.extent, tile);
   };
-  auto isDistributed = [&](const LoopVar& v) {
-    size_t axis = 0;
+  // the block axis a variable takes (as mapKernel gives them out), -1: none
+  const bool hadTiles = inner.numTiles > 1;
+  auto axisOf = [&](const LoopVar& v) -> int {
+    int axis = 0;
     for (const LoopVar* w : vars) {
-      if (w->numTiles == 1) continue;
-      if (w == &v) return axis < o.grid.size();
-      ++axis;
+      const bool takes = w->numTiles > 1 && (axis < static_cast<int>(o.grid.size()) || (w == &inner && !hadTiles && axis < 3));
+      if (w == &v) return takes ? axis : -1;
+      if (takes) ++axis;
     }
-    return false;
+    return -1;
   };
+  auto isDistributed = [&](const LoopVar& v) { return axisOf(v) >= 0; };
   // 0: more tiles than blocks, which are then the ones asked for
   auto blocks = [&]() -> int64_t {
     int64_t n = 1;
-    size_t axis = 0;
     for (size_t i = 0; i < vars.size(); ++i) {
-      if (vars[i]->numTiles == 1 || (vars[i] == &inner && axis >= o.grid.size())) {
-        n *= vars[i]->numTiles;
-        continue;
+      const int axis = axisOf(*vars[i]);
+      if (axis < 0) continue;
+      if (axis < static_cast<int>(o.grid.size())) {
+        uint64_t most = o.grid[axis];
+        if (i < o.grid.size()) most = std::max<uint64_t>(most, o.grid[i]);
+        if (static_cast<uint64_t>(vars[i]->numTiles) > most) return 0;
       }
-      if (axis >= o.grid.size()) continue;
-      uint64_t most = o.grid[axis];
-      if (i < o.grid.size()) most = std::max<uint64_t>(most, o.grid[i]);
-      if (static_cast<uint64_t>(vars[i]->numTiles) > most) return 0;
       n *= vars[i]->numTiles;
-      ++axis;
     }
     return n;
   };
@@ -492,41 +496,55 @@ const LoopVar* spreadContraction(const KernelPlan& k, StagePlan& st, const HipMa
   if (blocks() == 0) return nullptr;
   auto waves = [&]() { return blocks() * ceilDiv(threads, limits.wavefront); };
   const bool isShort = waves() < kFewWaves * limits.computeUnits;
+  std::set<const LoopVar*> whole; // whose tiles stay, as others would lose their axis
   auto largestOuter = [&]() {
     LoopVar* best = nullptr;
     for (LoopVar* v : vars) {
-      if (v != &inner && v->tile > 1 && (v->numTiles == 1 ? v->tile > 2 : isDistributed(*v)) && (!best || v->tile > best->tile)) best = v;
+      if (v != &inner && !whole.count(v) && v->tile > 1 && (v->numTiles == 1 ? v->tile > 2 : isDistributed(*v)) && (!best || v->tile > best->tile)) best = v;
     }
     return best;
   };
-  const bool hadAxis = inner.numTiles > 1;
-  if (isShort && (!hadAxis || isDistributed(inner))) {
-    int distributed = 0;
-    for (const LoopVar* v : vars) distributed += v != &inner && v->numTiles > 1 && isDistributed(*v);
+  if (isShort && (!hadTiles || isDistributed(inner))) {
     const int64_t given = inner.tile, most = ceilDiv(given, threads);
     const int64_t per = std::max<int64_t>(1, most / ceilDiv(kWavesPerUnit * limits.computeUnits, waves()));
-    if (distributed < 3 && per < most) {
+    if (per < most) {
       setTile(inner, per * threads);
-      if (blocks() == 0) setTile(inner, given);
+      if (blocks() == 0 || !isDistributed(inner)) setTile(inner, given);
     }
   }
   for (LoopVar* v : vars) {
     if (v == &inner || v->numTiles == 1 || isDistributed(*v)) continue;
     const int64_t tile = v->tile;
     setTile(*v, v->extent);
-    if (sums() > std::min(kMostSums, unroll)) setTile(*v, tile);
+    if (sums() > mostSums) setTile(*v, tile);
   }
   while (isShort && waves() < kWavesPerUnit * limits.computeUnits) {
     LoopVar* v = largestOuter();
     if (!v) break;
+    std::vector<LoopVar*> distributed;
+    for (LoopVar* w : vars) {
+      if (isDistributed(*w)) distributed.push_back(w);
+    }
+    const int64_t before = blocks();
     const int64_t tile = v->tile, numTiles = v->numTiles;
     setTile(*v, ceilDiv(v->tile, 2));
     if (blocks() == 0 || (numTiles == 1 && !isDistributed(*v))) {
       setTile(*v, tile);
       break;
     }
+    // a variable that loses its axis to this one is taken whole where its sums fit, else this one stays as it was
+    for (LoopVar* w : distributed) {
+      if (isDistributed(*w)) continue;
+      const int64_t given = w->tile;
+      if (w != &inner) setTile(*w, w->extent);
+      if (w != &inner && sums() <= mostSums && blocks() >= before) continue;
+      setTile(*w, given);
+      setTile(*v, tile);
+      whole.insert(v);
+      break;
+    }
   }
-  return inner.numTiles > 1 && !hadAxis ? &inner : nullptr;
+  return inner.numTiles > 1 && !hadTiles ? &inner : nullptr;
 }
 
 void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {

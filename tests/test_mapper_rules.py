@@ -362,3 +362,23 @@ def test_divisors_of_unsigned_steps(divisor, known):
     """A divisor counts as a known whole number only where no step of it is negative."""
     text, _ = mapped("def f(float(N) A) -> (O) { O(n) = A(n) / %s }" % divisor, "f", [(3,)], "naive;tile=256;mapToThreads=256")
     assert ("/ __tc::Whole<9>()" in text.split('extern "C"')[-1]) == known
+
+
+ROWS = "def f(float(N, C1, C2, H) A, float(N, C2, C3, H) B) -> (O) { O(n, c1, c3, h) +=! A(n, c1, r_c2, h) * B(n, r_c2, c3, h) }"
+
+
+@pytest.mark.parametrize("sizes,options,grid", [
+    ((8, 8, 4, 100, 64), "tile=8,1,1,0;mapToThreads=64;mapToBlocks=200,200", (8, 100, 1)),      # a halved n would take c1's axis, c1 that of c3
+    ((2, 8, 2, 4, 56, 56), "tile=1,8,4,0;mapToBlocks=32,64,8", (2, 8, 4)),                       # c3 that of the points in rows
+    ((2, 64, 16, 4, 40, 36), "tile=1,8,4,0;mapToBlocks=32,64,8", (2, 64, 2)),
+    ((3, 7, 15, 79, 14, 13), "", (3, 40, 1)),                                                    # c1 that of c3, of 79 points
+    ((2, 8, 2, 3, 56, 56), "", (2, 4, 4)),                                                       # all three points of c3 fit the registers
+])
+def test_variables_keep_their_blocks_when_others_are_halved(sizes, options, grid):
+    n, c1, c2, c3 = sizes[:4]
+    plane = sizes[4:]
+    source = ROWS if len(plane) == 1 else TENSORDOT
+    base = "naive" if len(plane) == 1 else STREAM
+    text, launches = mapped(source, "f", [(n, c1, c2) + plane, (n, c2, c3) + plane], f"{base};{options}")
+    assert launches[0][0] == grid
+    assert not re.search(r"for \(int t_(?!r_)", text.split('extern "C"')[-1])     # no block walks the tiles of a variable
