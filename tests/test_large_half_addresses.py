@@ -60,8 +60,8 @@ template <bool KInner, int R, int K> void check() {
         o.init((const _Float16*)kBase, (ldschar*)0, first, lane, wave);
         for (int t = 0; t < Operand::kTiles; ++t) {
           for (int i = 0; i < 4; ++i) {
-            o.template copy<true>(i, t, t & 1, lane);
-            o.template copy<false>(i, t, t & 1, lane);
+            o.copy(i, t, t & 1, lane);
+            o.store(i, t, t & 1, lane, o.request(i, t, lane));
           }
         }
       }
@@ -91,8 +91,7 @@ def operand():
 
     once(r"__builtin_amdgcn_make_buffer_rsrc\(", "resource(")
     once(r"__amdgpu_buffer_rsrc_t", "Resource")
-    once(r'asm volatile\("s_mov_b32 m0[^;]*?"v"\(from\),\s*"s"\(rs\),\s*"s"\((.*?)\)\s*: "[^;]*;', r"copied(from, rs, \1, dead);")
-    once(r'asm volatile\("" : "\+v"\(from\)\);', "")
+    once(r'asm volatile\("s_mov_b32 m0[^;]*?"v"\(from\),\s*"s"\(rs\),\s*"s"\((.*?)\)\s*: "[^;]*;', r"copied(from, rs, \1, isDead(i, t, lane));")
     once(r"\*\(const halfx8u\*\)(\(.*?\));", r"loaded\1;")
     once(r"\*\(__attribute__\(\(address_space\(3\)\)\) halfx8\*\)\((.*?)\) = v;", r"stored(\1, v);")
     return body

@@ -1,5 +1,6 @@
 """Registers of __tc::largeHalfProduct as the compiler reports them for gfx950: nothing goes to memory, in any order of the
-operands, whether the number of reduction tiles is even or odd."""
+operands, whether the number of reduction tiles is even or odd; operands that the direct copies cannot take are requested a
+whole tile at a time."""
 import os
 import re
 import subprocess
@@ -30,3 +31,12 @@ def test_no_register_is_spilled(tmp_path, a_transposed, b_transposed, m, n, k):
                     "-o", str(assembly), str(path)], check=True)
     code = assembly.read_text()
     assert re.findall(r"\.vgpr_spill_count: +(\d+)", code) == ["0"] and re.findall(r"\.private_segment_fixed_size: +(\d+)", code) == ["0"]
+    # copies through registers: the eight loads of a tile leave one after the other, nothing waits for memory in between
+    run = longest = 0
+    for line in code.splitlines():
+        if "global_load_dwordx4" in line:
+            run += 1
+            longest = max(longest, run)
+        elif "vmcnt" in line:
+            run = 0
+    assert longest >= 8
