@@ -370,6 +370,12 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
 // 128x256 ones and 0.4 to 0.6 of 128x128 ones, so they may compute a third more outputs, and twice as many where they occupy
 // 7/16 of the compute units (48 products of 800 to 4096 rows and columns, depths 256 to 4096, given / large: as many 1.3 to
 // 1.9, a third more 1.7 and 1.9, twice as many 1.01 to 1.32 from 112 blocks and 0.82 to 0.97 of 80 to 91, four times 0.5 to 0.65).
+// Twice as many pay for a deep reduction only, or one that ends inside a tile of 64 points, which costs the given tiles more:
+// given / large of 112 to 128 blocks at depth 264 to 360 0.95 to 1.15, 392 to 840 1.02 to 1.30; whole tiles, an even number of them: 256
+// 0.88 to 0.99, 384 1.04 to 1.08 where the given blocks leave a seventh of the compute units idle (1808x3688) and 0.92 to 1.02
+// where they do not, 512 to 1024 1.02 to 1.27; an odd number, which the given tiles take faster: 320 0.83 to 0.95, 448 to 1088
+// 0.86 to 1.02 (only 1808x3688, A * B, 1.01 to 1.15), 1344 0.96 to 1.16, 1984 1.0 to 1.2.  (Operands off 16-byte boundaries
+// are not known here: 2 bytes off, twice as many take 0.9 of the given tiles' speed at depths from 768, 0.8 of it at less.)
 constexpr int64_t kLargeHalfBlock = 256, kLargeHalfLds = 2 * 2 * 256 * 64 * 2;
 void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits, bool wide) {
   if (k.stages.size() != 1 || wide || waves != 8 || !o.prefetchSharedValue || !o.useSharedMemoryValue || st.atomic) return;
@@ -415,9 +421,12 @@ void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions&
     ++axis;
   }
   const int64_t blocks = ceilDiv(m.extent, kLargeHalfBlock) * ceilDiv(n.extent, kLargeHalfBlock);
-  const int64_t given = ceilDiv(m.numTiles * n.numTiles, limits.computeUnits) * m.tile * n.tile;
+  const int64_t tiles = m.numTiles * n.numTiles, rounds = ceilDiv(tiles, limits.computeUnits);
+  const int64_t given = rounds * m.tile * n.tile;
   const int64_t large = ceilDiv(blocks, limits.computeUnits) * kLargeHalfBlock * kLargeHalfBlock;
-  if (3 * large > 4 * given && (large > 2 * given || 16 * blocks < 7 * limits.computeUnits)) return;
+  const bool idle = 7 * tiles <= 6 * rounds * limits.computeUnits; // (a seventh of the given blocks' rounds)
+  const bool deep = r.extent % 64 != 0 || (r.extent % 128 == 0 ? r.extent >= (idle ? 384 : 512) : r.extent >= 1344);
+  if (3 * large > 4 * given && (large > 2 * given || 16 * blocks < 7 * limits.computeUnits || !deep)) return;
   std::ostringstream ss;
   ss << (innermost[0] ? "true" : "false") << ", " << (innermost[1] ? "true" : "false") << ", " << m.extent << ", " << n.extent << ", " << r.extent
      << ">(p" << st.tensor << ", p" << tensors[0] << ", p" << tensors[1];

@@ -382,3 +382,19 @@ def test_variables_keep_their_blocks_when_others_are_halved(sizes, options, grid
     text, launches = mapped(source, "f", [(n, c1, c2) + plane, (n, c2, c3) + plane], f"{base};{options}")
     assert launches[0][0] == grid
     assert not re.search(r"for \(int t_(?!r_)", text.split('extern "C"')[-1])     # no block walks the tiles of a variable
+
+
+@pytest.mark.parametrize("m,n,k,large", [
+    (2048, 4096, 256, False), (2048, 4096, 320, False), (1808, 3688, 320, False),
+    (2048, 4096, 384, False),                                   # 512 given blocks fill their two rounds
+    (1808, 3688, 384, True),                                    # 435 of them do not
+    (2048, 4096, 392, True), (2048, 4096, 712, True),           # the last tile is partial
+    (2048, 4096, 512, True), (2048, 4096, 704, False), (2048, 4096, 1280, True),
+    (2816, 2816, 1216, False), (2816, 2816, 1344, True),
+    (2880, 2904, 256, True), (2880, 2904, 320, True),           # three rounds of given blocks: a third more outputs
+    (4096, 4096, 320, True),                                    # as many
+])
+def test_twice_as_many_outputs_need_a_deep_reduction(m, n, k, large):
+    text, _ = tc.map_only(ANY_HALF_PRODUCT % ("M, K", "N, K", "m, r_k", "n, r_k"), "f", [ShapeOnly((m, k), "float16"), ShapeOnly((n, k), "float16")],
+                          f"naive;tile=128,128,64;{MATRIX}")
+    assert ("__tc::largeHalfProduct<" in text.split('extern "C"')[-1]) == large
