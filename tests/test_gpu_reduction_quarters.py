@@ -73,3 +73,23 @@ def test_untiled_products(m, k, n):
         out = tc.prepare_outputs(src, "mm", [A, B])
         tc.run(ex, [A, B], out)
         assert torch.equal(out[0], A @ B)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("c,tile,waves", [(10, 5, 4), (14, 7, 4), (14, 7, 8), (28, 14, 8), (28, 14, 4), (15, 7, 4), (12, 6, 4)])
+def test_quarters_of_tiled_reductions(dtype, c, tile, waves):
+    """Rectangles of output tiles over reduction tiles of any number of channels, with and without whole points a quarter."""
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    ins = [torch.randint(-3, 4, s, generator=gen, device="cuda").to(dtype) for s in ((3, c, 13, 19), (96, c, 3, 3))]
+    name, load = ("float", "%s") if dtype == torch.float32 else ("float16", "float(%s)")
+    src = (f"def conv({name}(N, C, H, W) I, {name}(M, C, KH, KW) W1) -> (O) "
+           f"{{ O(n, m, h, w) +=! {load % 'I(n, r_c, h + r_kh, w + r_kw)'} * {load % 'W1(m, r_c, r_kh, r_kw)'} }}")
+    print(dtype, c, tile, waves, flush=True)
+    want = torch.nn.functional.conv2d(ins[0].double().cpu(), ins[1].double().cpu())
+    for prefetch in (0, 1):
+        ex = tc.compile(src, "conv", ins, f"naive;tile=1,64,5,0,{tile};mapToThreads=64,{waves};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;"
+                                          f"sharedDepth=7;prefetchShared={prefetch}")
+        assert "matrix cores:" in ex.compiled_source
+        out = torch.full((3, 96, 11, 17), float("nan"), device="cuda")
+        tc.run(ex, ins, [out])
+        assert torch.equal(out.double().cpu(), want)

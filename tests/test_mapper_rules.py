@@ -398,3 +398,30 @@ def test_twice_as_many_outputs_need_a_deep_reduction(m, n, k, large):
     text, _ = tc.map_only(ANY_HALF_PRODUCT % ("M, K", "N, K", "m, r_k", "n, r_k"), "f", [ShapeOnly((m, k), "float16"), ShapeOnly((n, k), "float16")],
                           f"naive;tile=128,128,64;{MATRIX}")
     assert ("__tc::largeHalfProduct<" in text.split('extern "C"')[-1]) == large
+
+
+CONVOLUTION = "def f(%s(N, C, H, W) I, %s(M, C, KH, KW) W1) -> (O) { O(n, m, h, w) +=! %s * %s }"
+
+
+@pytest.mark.parametrize("dtype,sizes,tile,waves,steps,half", [
+    ("float16", (16, 84, 128, 22, 18), "1,128,7,0,7", 4, 16, True),     # 18 would leave the half instruction (and 4x4 tiles be dealt one by one)
+    ("float16", (32, 84, 16, 26, 26), "1,64,16,0,7", 4, 16, True),
+    ("float16", (2, 84, 128, 22, 40), "1,32,3,0,7", 8, 18, False),      # eight wavefronts have half the registers each
+    ("float16", (16, 25, 256, 11, 42), "1,32,6,0,5", 8, 12, True),      # 18 for 12 does not pay on eight either
+    ("float16", (32, 84, 256, 27, 12), "1,64,4,0,14", 4, 32, True),
+    ("float16", (16, 72, 256, 29, 17), "1,128,1,0,6", 4, 14, False),    # the same instruction: the fewer steps
+    ("float", (16, 28, 128, 42, 40), "1,128,6,0,7", 8, 16, False),     # 18 would lose the rectangles of 4x4 tiles
+    ("float", (32, 56, 96, 32, 28), "1,32,23,0,7", 8, 18, False),
+    ("float", (16, 42, 64, 17, 27), "1,16,5,0,14", 8, 36, False),       # one tile a wavefront
+    ("float", (32, 60, 32, 35, 35), "1,32,3,0,5", 4, 12, False),        # 18 for 12
+])
+def test_whole_points_in_a_quarter_of_the_reduction(dtype, sizes, tile, waves, steps, half):
+    n, c, m, h, w = sizes
+    load = "%s" if dtype == "float" else "float(%s)"
+    source = CONVOLUTION % (dtype, dtype, load % "I(n, r_c, h + r_kh, w + r_kw)", load % "W1(m, r_c, r_kh, r_kw)")
+    name = "float32" if dtype == "float" else dtype
+    text, _ = tc.map_only(source, "f", [ShapeOnly((n, c, h, w), name), ShapeOnly((m, c, 3, 3), name)],
+                          f"naive;tile={tile};mapToThreads=64,{waves};mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;sharedDepth=7")
+    body = text.split('extern "C"')[-1]
+    assert f", {steps} steps of " in body
+    assert ("__tc::multiplyHalves(" in body) == half
