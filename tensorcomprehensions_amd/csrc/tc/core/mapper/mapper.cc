@@ -210,6 +210,16 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
   }
 }
 
+// Blocks that the options allow a variable on block axis `axis`.  A variable with a single tile uses up no axis, so the ones
+// behind it move up; a variable's size is the one of its place among the options' sizes (`position`, among the
+// parallel variables of the kernel, lanes of a vector left out) as well as that of the axis it moves up to (one image of 11
+// groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).
+int64_t allowedBlocks(const HipMappingOptions& o, int axis, int position) {
+  uint64_t blocks = o.grid[axis];
+  if (position < static_cast<int>(o.grid.size())) blocks = std::max<uint64_t>(blocks, o.grid[position]);
+  return static_cast<int64_t>(std::min<uint64_t>(blocks, std::numeric_limits<int32_t>::max()));
+}
+
 // A matrix-core stage whose blocks leave compute units idle: a block-mapped variable gets the smaller tile
 // that shortens the longest-running compute unit by a quarter or more, if there is one, and then another one (compute units
 // are those of the device, or of its partition).  A compute unit's time is its rounds of blocks times the output tiles
@@ -258,14 +268,17 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     return false;
   };
   // in units of 1 / waves of an output tile; 0: not a form this speaks of
+  bool byAxis = true; // (sizes that hold the given tiles axis by axis are those of the axes)
   bool onGrid = false, fewTiles = false; // (every tile has a block; fewer output tiles than wavefronts)
   auto cost = [&](int64_t& blocks) -> int64_t {
     blocks = 1;
     onGrid = fewTiles = false;
-    size_t axis = 0;
+    int axis = 0, position = -1;
     for (int i = 0; i < st.numParallel; ++i) {
+      if (!st.vars[i].vectorLane) ++position;
       if (st.vars[i].numTiles == 1) continue;
-      if (!mayBeSplit(i) || axis >= o.grid.size() || st.vars[i].numTiles > static_cast<int64_t>(o.grid[axis])) return 0;
+      if (!mayBeSplit(i) || axis >= static_cast<int>(o.grid.size())) return 0;
+      if (st.vars[i].numTiles > (byAxis ? allowedBlocks(o, axis, axis) : allowedBlocks(o, axis, position))) return 0;
       blocks *= st.vars[i].numTiles;
       ++axis;
     }
@@ -287,6 +300,8 @@ void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOption
     v.numTiles = ceilDiv(v.extent, tile);
   };
   int64_t blocks = 0;
+  cost(blocks);
+  byAxis = onGrid;
   const int64_t given = cost(blocks);
   if (product && !halves && fewTiles && 2 * blocks <= computeUnits) {
     LoopVar* longer = nullptr;
@@ -414,10 +429,10 @@ void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions&
   }
   if (r.extent < 256) return;
   const int64_t numTiles[2] = {m.numTiles, n.numTiles};
-  size_t axis = 0;
-  for (int64_t tiles : numTiles) {
-    if (tiles == 1) continue;
-    if (axis >= o.grid.size() || tiles > static_cast<int64_t>(o.grid[axis])) return;
+  int axis = 0;
+  for (int position = 0; position < 2; ++position) {
+    if (numTiles[position] == 1) continue;
+    if (axis >= static_cast<int>(o.grid.size()) || numTiles[position] > allowedBlocks(o, axis, position)) return;
     ++axis;
   }
   const int64_t blocks = ceilDiv(m.extent, kLargeHalfBlock) * ceilDiv(n.extent, kLargeHalfBlock);
@@ -488,11 +503,7 @@ const LoopVar* spreadContraction(const KernelPlan& k, StagePlan& st, const HipMa
     for (size_t i = 0; i < vars.size(); ++i) {
       const int axis = axisOf(*vars[i]);
       if (axis < 0) continue;
-      if (axis < static_cast<int>(o.grid.size())) {
-        uint64_t most = o.grid[axis];
-        if (i < o.grid.size()) most = std::max<uint64_t>(most, o.grid[i]);
-        if (static_cast<uint64_t>(vars[i]->numTiles) > most) return 0;
-      }
+      if (axis < static_cast<int>(o.grid.size()) && vars[i]->numTiles > allowedBlocks(o, axis, static_cast<int>(i))) return 0;
       n *= vars[i]->numTiles;
     }
     return n;
@@ -618,11 +629,7 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
         break;
       }
       v.blockAxis = axis;
-      // The block size of a variable is the one of its place among the options' sizes as well as that of the axis it
-      // moves up to (one image of 11 groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).
-      uint64_t blocks = o.grid[axis];
-      if (position < static_cast<int>(o.grid.size())) blocks = std::max<uint64_t>(blocks, o.grid[position]);
-      v.gridExtent = std::min<int64_t>(static_cast<int64_t>(std::min<uint64_t>(blocks, std::numeric_limits<int32_t>::max())), v.numTiles);
+      v.gridExtent = std::min<int64_t>(allowedBlocks(o, axis, position), v.numTiles);
       gridUse[axis] = std::max(gridUse[axis], v.gridExtent);
       ++axis;
     }

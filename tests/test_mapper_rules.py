@@ -425,3 +425,19 @@ def test_whole_points_in_a_quarter_of_the_reduction(dtype, sizes, tile, waves, s
     body = text.split('extern "C"')[-1]
     assert f", {steps} steps of " in body
     assert ("__tc::multiplyHalves(" in body) == half
+
+
+@pytest.mark.parametrize("blocks", ["256,256,256", "1,256,256", "1,2,256"])
+def test_tiles_that_fill_the_device_see_the_block_sizes_of_their_variables(blocks):
+    """One image: its variable uses up no block axis, and no block size."""
+    source = CONVOLUTION % ("float", "float", "I(n, r_c, h + r_kh, w + r_kw)", "W1(m, r_c, r_kh, r_kw)")
+    _, launches = mapped(source, "f", [(1, 64, 57, 57), (64, 64, 3, 3)],
+                         f"naive;tile=1,32,11,0,8;mapToThreads=64,8;mapToBlocks={blocks};useMfma=1;useSharedMemory=1;prefetchShared=1")
+    assert launches[0][0] == (2, 55, 1)
+
+
+@pytest.mark.parametrize("blocks,large", [("1,8", True), ("1,7", False), ("8,1", True)])
+def test_large_half_products_see_the_block_sizes_of_their_variables(blocks, large):
+    text, _ = tc.map_only(ANY_HALF_PRODUCT % ("M, K", "N, K", "m, r_k", "n, r_k"), "f", [ShapeOnly((256, 1024), "float16"), ShapeOnly((2048, 1024), "float16")],
+                          f"naive;tile=256,256,32;{MATRIX};mapToBlocks={blocks}")
+    assert ("__tc::largeHalfProduct<" in text.split('extern "C"')[-1]) == large
