@@ -38,3 +38,13 @@ def test_against_float64(sizes, changes, op, join, then):
     else:
         # one rounded sum a term; rounding keeps the order
         assert torch.equal(outs[0], (left + right).amax(2).float())
+
+
+@pytest.mark.parametrize("sizes,changes", [
+    ((2, 8, 2, 4, 30, 56), "tile=1,8,4,0;mapToBlocks=32,64,8"),     # axes that a halved tile would have taken from the rows' pieces,
+    ((3, 7, 5, 79, 14, 13), ""),                                     # from c3,
+    ((3, 11, 4, 4, 6, 11), "tile=4,1,1,0;mapToBlocks=200,200"),      # and from c3 by way of c1
+    ((2, 8, 2, 3, 31, 56), ""),                                      # c3 taken whole when c1 takes its axis
+])
+def test_axes_stay_with_their_variables(sizes, changes):
+    test_against_float64(sizes, changes, "+=!", "*", "")
