@@ -232,11 +232,15 @@ int64_t allowedBlocks(const HipMappingOptions& o, int axis, int position) {
 // 35.9; 1500x800x1700: 168 blocks 56.8, 224 of 96x128 46.8; 215x1188x1305: 84 blocks of 64x64 24.2 us, 164 of 64x32 14.8, 287 of 32x32 21.9; 430x1367x1095 27.2 and 18.1; halves
 // 322x2061x993 17.9 and 13.6; where the halves make two rounds there is nothing to gain: 691x1840x792, 143 blocks, 35.7, 36.1).
 //   Products whose blocks make a second round for a few: a side up to half as long again under which there is one, where the
-// estimate says two thirds (2100x900x2100: 289 blocks of 128x128 117.7 us, 255 of 144x128 85.2; 1100x2000x1100: 324 of 64x64 72.6,
+// estimate says 13 / 20 of the time or less (2100x900x2100: 289 blocks of 128x128 117.7 us, 255 of 144x128 85.2; 1100x2000x1100: 324 of 64x64 72.6,
 // 216 of 96x64 61.7; 1400x600x1100, three quarters: 396 of 64x64 25.8, 198 of 128x64 26.9).
 //   Products whose wavefronts share the reduction of a tile, on half the compute units or fewer: half the longer side, as the
 // staging of a block is what takes the time (116x2960x204: 56 blocks of 16x32 14.6 us, 104 of 16x16 9.5; 108x1643x127 7.8 and 6.1;
 // 128x1000x1024, 256 blocks, 6.1 and 9.9).
+//   Of a product's two sides that come out alike the second is taken, a long one unless it makes clearly fewer blocks.  Measured
+// on 70 products that leave the choice: tiles of 64x64 and of halves are as fast either way (3 % at most, the mean the same);
+// in tiles of 128x128 the first side was 2 to 11 % faster in all eight (1789x2010x1391: 252 blocks of 128x80 104.5 us, 253 of
+// 80x128 93.2; 1883x157x1271, 240 blocks either way, 16.9 and 15.3).
 // mapToBlocks sizes that hold exactly the given tiles keep those tiles, as maxSharedMemory keeps those of products.
 void fillComputeUnits(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, int64_t computeUnits) {
   constexpr int64_t kStaging = 2, kLongReduction = 8, kLongSidesLds = 64 << 10;
