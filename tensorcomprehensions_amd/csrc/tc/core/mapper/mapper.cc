@@ -213,10 +213,12 @@ void deepenHalfTile(StagePlan& st, LoopVar& v, const HipMappingOptions& o, int64
 // Blocks that the options allow a variable on block axis `axis`.  A variable with a single tile uses up no axis, so the ones
 // behind it move up; a variable's size is the one of its place among the options' sizes (`position`, among the
 // parallel variables of the kernel, lanes of a vector left out) as well as that of the axis it moves up to (one image of 11
-// groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).
+// groups under mapToBlocks=1,11: on one block 115 us, on eleven 11.5).  The size of a place counts up to 65535: on the second
+// and third axis, which any variable may end up on, a launch takes no more.
 int64_t allowedBlocks(const HipMappingOptions& o, int axis, int position) {
+  constexpr uint64_t kMostAcross = 65535;
   uint64_t blocks = o.grid[axis];
-  if (position < static_cast<int>(o.grid.size())) blocks = std::max<uint64_t>(blocks, o.grid[position]);
+  if (position < static_cast<int>(o.grid.size())) blocks = std::max<uint64_t>(blocks, std::min<uint64_t>(o.grid[position], kMostAcross));
   return static_cast<int64_t>(std::min<uint64_t>(blocks, std::numeric_limits<int32_t>::max()));
 }
 

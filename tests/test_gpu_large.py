@@ -80,3 +80,14 @@ def test_a_single_dimension_of_2_to_the_31_is_refused():
     with pytest.raises(tc.TcError) as e:
         tc.compile("def f(int8(N) A) -> (B) { B(i) = A(i) }", "f", [tc.ShapeOnly((2 ** 31 + 8,), "int8")], "naive")
     assert "dimension of 2^31 or more" in str(e.value)
+
+
+def test_more_tiles_than_a_launch_has_blocks_across():
+    """70000 tiles of a variable that moves up to the second axis, as one in front of it has a single tile."""
+    A = torch.randint(-3, 4, (2, 300), device="cuda").float()
+    W = torch.randint(-3, 4, (70000,), device="cuda").float()
+    src = "def f(float(G, K) A, float(H) W) -> (O) { O(n, g, h) +=! A(g, r_k) * W(h) where n in 0:1 }"
+    ex = tc.compile(src, "f", [A, W], "naive;tile=1,1,1;mapToThreads=1;mapToBlocks=1,2,100000;collapseContiguous=0")
+    out = torch.full((1, 2, 70000), float("nan"), device="cuda")
+    tc.run(ex, [A, W], [out])
+    assert torch.equal(out[0], A.sum(1)[:, None] * W)

@@ -441,3 +441,14 @@ def test_large_half_products_see_the_block_sizes_of_their_variables(blocks, larg
     text, _ = tc.map_only(ANY_HALF_PRODUCT % ("M, K", "N, K", "m, r_k", "n, r_k"), "f", [ShapeOnly((256, 1024), "float16"), ShapeOnly((2048, 1024), "float16")],
                           f"naive;tile=256,256,32;{MATRIX};mapToBlocks={blocks}")
     assert ("__tc::largeHalfProduct<" in text.split('extern "C"')[-1]) == large
+
+
+@pytest.mark.parametrize("sizes,blocks,grid", [
+    ((2, 70000), "1,2,100000", [1, 2, 65535]), ((70000, 2), "1,100000,2", [1, 2, 65535]), ((2, 70000), "1,1,4294967296", [1, 1, 65535]),
+    ((70000, 1), "100000,1", [1, 1, 70000]),                # the axis's own size is as given
+])
+def test_block_sizes_of_places_fit_every_axis(sizes, blocks, grid):
+    """A variable that moves up to another axis brings no more blocks than a launch takes on the second and third."""
+    _, launches = mapped("def f(float(G, H) A) -> (O) { O(n, g, h) = A(g, h) + 1 where n in 0:1 }", "f", [sizes],
+                         f"naive;tile=1,1,1;mapToThreads=1;mapToBlocks={blocks};collapseContiguous=0")
+    assert sorted(launches[0][0]) == grid
