@@ -1275,7 +1275,14 @@ void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
     StageCodegen& g = gens[0];
     em.line("__syncthreads();");
     em.open("if (more_)");
-    for (const auto& p : g.promotions()) g.emitCopyStores(p, "pf_" + p.tensor + "_");
+    std::string start, step;
+    loopHeader(*loops.back(), start, step);
+    g.tileOverride[loops.back()->name] = "(t_" + loops.back()->name + " + " + step + ")";
+    for (const auto& p : g.promotions()) {
+      if (g.copyPlan(p).shifted) g.declareLows(p); // (the shift follows from the place of the tile that was requested)
+      g.emitCopyStores(p, "pf_" + p.tensor + "_");
+    }
+    g.tileOverride.clear();
     em.close();
   }
   emitSync(syncAfter.back());

@@ -93,3 +93,16 @@ def test_lds_limit_of_the_options_keeps_the_given_tile():
                     "naive;tile=128,256,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1;maxSharedMemory=65536")
     assert np.array_equal(got, A.astype(np.float32) @ Bm.astype(np.float32))
     assert "const __tc::halfx8 av_" not in text
+
+
+@pytest.mark.parametrize("m,k,n,tile,blocks", [(126, 81, 44, "16,16,13", "3,256"), (70, 81, 50, "16,16", "2,2"), (191, 105, 34, "4,4,2", "1,256")])
+def test_odd_rows_of_tiles_requested_ahead(m, k, n, tile, blocks):
+    """Blocks that walk several tiles and request the next one's operands ahead, rows of an odd number of halves: vectors across
+    the end of a tensor are shifted by the place of the tile they belong to."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    A, B = (torch.randint(-3, 4, s, generator=g, device="cuda").half() for s in ((m, k), (k, n)))
+    src = "def f(float16(M, K) A, float16(K, N) B) -> (O) { O(m, n) +=! float(A(m, r_k)) * float(B(r_k, n)) }"
+    ex = tc.compile(src, "f", [A, B], f"naive;tile={tile};mapToThreads=64,4;mapToBlocks={blocks};useMfma=1;useSharedMemory=1;prefetchShared=1")
+    out = torch.full((m, n), float("nan"), device="cuda")
+    tc.run(ex, [A, B], [out])
+    assert torch.equal(out, A.float() @ B.float())

@@ -452,3 +452,16 @@ def test_block_sizes_of_places_fit_every_axis(sizes, blocks, grid):
     _, launches = mapped("def f(float(G, H) A) -> (O) { O(n, g, h) = A(g, h) + 1 where n in 0:1 }", "f", [sizes],
                          f"naive;tile=1,1,1;mapToThreads=1;mapToBlocks={blocks};collapseContiguous=0")
     assert sorted(launches[0][0]) == grid
+
+
+@pytest.mark.parametrize("m,k,n,tile,blocks", [(126, 81, 44, "16,16,13", "3,256"), (70, 81, 50, "16,16", "2,2"), (191, 105, 34, "4,4,2", "1,256")])
+def test_shifted_vectors_of_a_tile_requested_ahead(m, k, n, tile, blocks):
+    """Rows of an odd number of halves, walked by blocks that request the next tile's operands while they multiply: the stores
+    shift vectors across the tensor's end by the place of that tile."""
+    source = ANY_HALF_PRODUCT % ("M, K", "K, N", "m, r_k", "r_k, n")
+    shapes = [ShapeOnly((m, k), "float16"), ShapeOnly((k, n), "float16")]
+    options = f"naive;tile={tile};mapToThreads=64,4;mapToBlocks={blocks};useMfma=1;useSharedMemory=1;prefetchShared=1"
+    text, _ = tc.map_only(source, "f", shapes, options)
+    stores = text.split('extern "C"')[-1].rsplit("if (more_)", 1)[1]
+    assert "__tc::shiftDown(" in stores and re.search(r"const int lo0_\w+_\d = .*\(t_\w+ \+ \d+\)", stores)
+    tc.compile(source, "f", shapes, options)
