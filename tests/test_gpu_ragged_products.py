@@ -176,3 +176,28 @@ def test_few_blocks_over_long_reductions(m, k, n):
     options = f"naive;tile=16,32,128;mapToThreads=64,8;{TAIL}"
     assert np.array_equal(run(B.MATMUL, "matmul", [A, Bm], options), A @ Bm)
     assert np.array_equal(run(B.TMM, "tmm", [A, np.ascontiguousarray(Bm.T)], options), A @ Bm)
+
+
+@pytest.mark.parametrize("dtype", ["float", "float16"])
+@pytest.mark.parametrize("m,k,n,options", [
+    (45, 70, 37, "tile=32,32,16;mapToThreads=64,4"),            # rectangles of tiles, the last reduction tile partial
+    (45, 70, 37, "tile=16,32,16;mapToThreads=64,4"),            # tile by tile
+    (130, 93, 75, "tile=64,32,0;mapToThreads=64,4"),            # the whole reduction, 24 steps of a quarter
+    (33, 61, 40, "tile=16,16,0;mapToThreads=64,2"),
+    (50, 131, 33, "tile=32,16,64;mapToThreads=64,2"),           # runs of more steps
+    (50, 300, 33, "tile=32,16,0;mapToThreads=64,4"),
+])
+def test_steps_past_the_reduction_with_operands_from_memory(dtype, m, k, n, options):
+    """Without shared memory: steps that do not exist read an element that does, and count as zeros on both sides (an infinity
+    there makes no NaN)."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    A, B = (torch.randint(1, 4, s, generator=g, device="cuda").to(torch.float16 if dtype == "float16" else torch.float32) for s in ((m, k), (k, n)))
+    A[3, k - 1] = float("inf")
+    load = "%s" if dtype == "float" else "float(%s)"
+    src = f"def f({dtype}(M, K) A, {dtype}(K, N) B) -> (O) {{ O(m, n) +=! {load % 'A(m, r_k)'} * {load % 'B(r_k, n)'} }}"
+    ex = tc.compile(src, "f", [A, B], f"naive;{options};mapToBlocks=64,64;useMfma=1;useSharedMemory=0")
+    assert "matrix cores:" in ex.compiled_source
+    out = torch.full((m, n), float("nan"), device="cuda")
+    tc.run(ex, [A, B], [out])
+    want = (A[:, :, None].double() * B[None].double()).sum(1)
+    assert torch.equal(out.double(), want)

@@ -465,3 +465,19 @@ def test_shifted_vectors_of_a_tile_requested_ahead(m, k, n, tile, blocks):
     stores = text.split('extern "C"')[-1].rsplit("if (more_)", 1)[1]
     assert "__tc::shiftDown(" in stores and re.search(r"const int lo0_\w+_\d = .*\(t_\w+ \+ \d+\)", stores)
     tc.compile(source, "f", shapes, options)
+
+
+@pytest.mark.parametrize("tile,threads,later", [
+    ("32,32,16", "64,4", True),             # rectangles
+    ("16,16,16", "64,8", True),             # tile by tile
+    ("16,16,0", "64,2", True),              # the whole reduction: 22 steps a quarter, no vector of four
+    ("48,16,128", "64,2", False),           # 32 steps of a reduction tile, tile by tile
+])
+def test_loads_from_memory_are_tested_together(tile, threads, later):
+    """A load with its test beside it is waited for before the next one leaves: values from memory get their zeros afterwards."""
+    text, _ = mapped(FLOAT_PRODUCT, "f", [(70, 85 if tile.endswith(",0") else 333), (85 if tile.endswith(",0") else 333, 70)],
+                     f"naive;tile={tile};mapToThreads={threads};mapToBlocks=64,64;useMfma=1;useSharedMemory=0")
+    body = text.split('extern "C"')[-1]
+    assert "kok_" in body
+    assert bool(re.search(r"__tc::keep\(kok_, p[AB]\[", body)) != later
+    assert bool(re.search(r"\[[a-z_]+\] = __tc::keep\(kok_, (ra|rb|aq|bq)_\[", body)) == later
