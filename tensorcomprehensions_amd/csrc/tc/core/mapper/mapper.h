@@ -111,6 +111,10 @@ struct StagePlan {
   // A product of halves with many outputs, computed by __tc::largeHalfProduct (its template arguments;
   // empty: not this stage).
   std::string largeHalfProduct;
+  // A convolution of floats computed by __tc::SplitConvolution (its template arguments and call; empty: not this
+  // stage), and the LDS that takes.
+  std::string splitConvolution;
+  int64_t splitConvolutionLds = 0;
   // The stage adds partial sums into its tensor with atomics: its first parallel variable numbers
   // slices of the reduction and is no subscript of the tensor.
   bool atomic = false;

@@ -1,0 +1,136 @@
+"""Convolutions on the bf16 matrix instruction, each float in three parts (__tc::SplitConvolution): against the same sums in
+64 bits at the edges of pixel tiles, filter tiles, channel chunks and windows, and for values the parts cannot hold."""
+import numpy as np
+import pytest
+import torch
+
+import tensorcomprehensions_amd as tc
+from tensorcomprehensions_amd import ShapeOnly
+
+DENSE = """
+def f(float(N, C, H, W) I, float(M, C, KH, KW) W1, float(M) B) -> (O) {
+    O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw)
+    O(n, m, h, w) = O(n, m, h, w) + B(m)
+}
+"""
+GROUPS = """
+def f(float(N, G, C, H, W) I, float(G, F, C, KH, KW) W1, float(G, F) B) -> (O) {
+    O(n, g, f, h, w) +=! W1(g, f, r_c, r_kh, r_kw) * I(n, g, r_c, h + r_kh, w + r_kw)
+    O(n, g, f, h, w) = B(g, f) + O(n, g, f, h, w)
+}
+"""
+PLAIN = """
+def f(float(N, G, C, H, W) I, float(G, F, C, KH, KW) W1) -> (O) {
+    O(n, g, f, h, w) +=! I(n, g, r_c, h + r_kh, w + r_kw) * W1(g, f, r_c, r_kh, r_kw)
+}
+"""
+SIZES = [
+    # n, g, channels, filters, h, w, kernel
+    (16, 1, 64, 64, 57, 57, (3, 3)),     # four chunks, a last band of 17 pixels
+    (6, 1, 29, 25, 12, 7, (3, 3)),       # five pixels a row, 50 of them
+    (2, 1, 47, 25, 9, 11, (3, 3)),       # a plane of 63 pixels
+    (13, 1, 103, 118, 15, 37, (1, 1)),   # no window
+    (28, 1, 65, 38, 43, 29, (3, 3)),     # one channel more than eight octets
+    (9, 11, 6, 29, 19, 29, (3, 3)),      # a chunk that is not full, 13 filters in the last tile
+    (4, 4, 7, 13, 28, 30, (5, 5)),       # 25 places: one slot of the last step
+    (2, 8, 15, 4, 25, 28, (3, 3)),
+    (3, 5, 17, 20, 22, 26, (5, 3)),      # a window that is no square
+]
+
+
+def options(kernel, sizes):
+    n, g, c, f, h, w, _ = sizes
+    rows, columns = h - kernel[0] + 1, w - kernel[1] + 1
+    if g == 1:
+        band = max(d for d in range(1, 17) if rows % d == 0)
+        return (f"naive;tile=1,32,{band},0,8;mapToThreads=64,8;mapToBlocks=256,256,256;useMfma=1;useSharedMemory=1;"
+                "useReadOnlyCache=1;sharedDepth=7;prefetchShared=1")
+    return f"naive;tile=1,1,{f},{rows},{columns};mapToThreads=64,4;mapToBlocks={n},{g};useMfma=1;useSharedMemory=1;useReadOnlyCache=1"
+
+
+def operands(sizes, make):
+    n, g, c, f, h, w, (kh, kw) = sizes
+    if g == 1:
+        return [make(n, c, h, w), make(f, c, kh, kw), make(f)]
+    return [make(n, g, c, h, w), make(g, f, c, kh, kw), make(g, f)]
+
+
+def run(source, sizes, ins):
+    text, _ = tc.map_only(source, "f", [ShapeOnly(tuple(t.shape)) for t in ins], options(sizes[6], sizes))
+    assert "__tc::SplitConvolution<" in text
+    device = [t.cuda() for t in ins]
+    executor = tc.compile(source, "f", device, options(sizes[6], sizes))
+    outs = tc.prepare_outputs(source, "f", device)
+    outs[0].fill_(float("nan"))
+    tc.run(executor, device, outs)
+    return outs[0].cpu()
+
+
+def reference(sizes, ins):
+    n, g, c, f, h, w, (kh, kw) = sizes
+    x, weights = ins[0].double().reshape(n, g * c, h, w), ins[1].double().reshape(g * f, c, kh, kw)
+    bias = ins[2].double().reshape(-1) if len(ins) > 2 else None
+    sums = torch.nn.functional.conv2d(x, weights, None, groups=g)
+    magnitudes = torch.nn.functional.conv2d(x.abs(), weights.abs(), None, groups=g)
+    if bias is not None:
+        sums, magnitudes = sums + bias.view(1, -1, 1, 1), magnitudes + bias.abs().view(1, -1, 1, 1)
+    return sums, magnitudes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", SIZES, ids=lambda s: "x".join(map(str, s[:6])))
+def test_sums(sizes):
+    print(sizes, flush=True)
+    source = DENSE if sizes[1] == 1 else GROUPS
+    generator = torch.Generator().manual_seed(1)
+    whole = operands(sizes, lambda *s: torch.randint(-8, 9, s, generator=generator).float())
+    got = run(source, sizes, whole)
+    assert torch.equal(got.reshape(-1).double(), reference(sizes, whole)[0].reshape(-1))   # (sums of whole numbers are exact)
+    ins = operands(sizes, lambda *s: torch.randn(s, generator=generator))
+    got = run(source, sizes, ins).double()
+    want, magnitudes = reference(sizes, ins)
+    # one rounding of 2^-24 a term and the bias, in whatever order, and 2^-26 of every product for the parts left out
+    terms = sizes[2] * sizes[6][0] * sizes[6][1]
+    assert ((got.reshape(want.shape) - want).abs() <= (terms + 2) * 2.0 ** -24 * magnitudes).all()
+
+
+@pytest.mark.gpu
+def test_without_a_bias():
+    sizes = next(s for s in SIZES if s[:3] == (9, 11, 6))
+    ins = operands(sizes, lambda *s: torch.randint(-8, 9, s).float())[:2]
+    assert torch.equal(run(PLAIN, sizes, ins).reshape(-1).double(), reference(sizes, ins)[0].reshape(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["infinity", "nan", "rounds to infinity", "small", "denormal", "large sums"])
+def test_values_the_parts_cannot_hold(case):
+    sizes = next(s for s in SIZES if s[:3] == (2, 8, 15))
+    generator = torch.Generator().manual_seed(2)
+    x, weights, bias = operands(sizes, lambda *s: torch.randn(s, generator=generator))
+    flat = x.view(-1)
+    if case == "infinity":
+        flat[[5, 4711, -1]] = torch.tensor([np.inf, -np.inf, np.inf])
+    elif case == "nan":
+        flat[[5, 4711]] = np.nan
+    elif case == "rounds to infinity":
+        flat[::1001] = 3.4e38                   # its nearest bf16 is infinite
+        weights *= 2.0 ** -20
+    elif case == "small":
+        flat[:] *= 2.0 ** -110                  # their low parts would be denormal
+        bias[:] = 0
+    elif case == "denormal":
+        flat[: flat.numel() // 2] *= 2.0 ** -130
+        bias[:] = 0
+    else:
+        flat[:] *= 2.0 ** 100
+        weights *= 2.0 ** 30                    # sums beyond the largest float
+    got = run(GROUPS, sizes, [x, weights, bias]).double()
+    want, magnitudes = reference(sizes, [x, weights, bias])
+    got, want = got.reshape(-1), want.float().double().reshape(-1)   # (the float nearest to the sum: infinite beyond the largest)
+    finite = torch.isfinite(want) & (magnitudes.reshape(-1) < 3.4e38)
+    terms = sizes[2] * 9
+    # (a denormal sum is a whole number of 2^-149)
+    assert ((got - want).abs()[finite] <= (terms + 2) * (2.0 ** -24 * magnitudes.reshape(-1)[finite] + 2.0 ** -149)).all()
+    if case in ("infinity", "nan"):
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
