@@ -13,10 +13,15 @@ namespace hip {
 // products have an accumulator of their own, whose roundings are those of a sum 2^-8 as large.  Error against 64 bits, normal
 // deviates, 2-norm: 96, 992 and 4096 terms 0.6e-7, 1.8e-7, 3.9e-7 (float instruction 1.8e-7, 5.6e-7, 11.5e-7).
 //
-// What the parts cannot hold is computed again with float arithmetic, block by block (see `SplitRange`):
-//  - a value from 2^-100 down, other than zero, whose low part may be below the smallest normal bf16;
-//  - an infinity, or a value that rounds to one: a middle part of infinity minus infinity.  These, and sums that overflow,
-//    are seen by a result that is not finite.
+// What the parts cannot hold is computed again with float arithmetic, block by block:
+//  - infinities, and values that round to one (a middle part of infinity minus infinity), and sums that overflow: seen by a
+//    result that is not finite;
+//  - small values.  A bf16 has the exponents of a float, denormal ones included, so what is left out of a value is below 2^-134.  Where no value
+//    is above 2^32, sums of up to 65536 terms lose less than 2^-86 by that, nothing beside the rounding of a sum from 2^-60 on.  Blocks
+//    with a smaller sum, other than zero, or a larger value go the other way, and so do those with a lane that sees something of an
+//    operand, but nothing from 2^-100 on.  (A sum of zero is taken: it may be one of denormal values below 2^-134 alone, beside other
+//    rows in the block.)
+// The check costs half an instruction a value; one for every value's own exponent cost 1.5, and 1000^3 20.7 us for 17.4.
 constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
 typedef __attribute__((address_space(3))) char ldschar;
@@ -24,14 +29,18 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) bf16x8 ldsbf16x8;
 struct SplitParts { bf16x8 part[3]; };
-// The smallest magnitude but zero that was split: twice the bits of a float order it by magnitude, less one zero comes last.
+// The largest magnitude of one operand that a lane has split.
 struct SplitRange {
-  unsigned least = ~0u;
-  __device__ __forceinline__ void see(float a, float b) {
-    least = __builtin_elementwise_min(least, __builtin_elementwise_min(2 * __builtin_bit_cast(unsigned, a) - 1, 2 * __builtin_bit_cast(unsigned, b) - 1));
-  }
-  __device__ __forceinline__ bool isTooSmall() const { return least < 2u * (27u << 23) - 1; }
+  float most = 0.0f;
+  // (one instruction; fmaxf would quiet NaNs first)
+  __device__ __forceinline__ void see(float a, float b) { asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(a), "v"(b)); }
+  __device__ __forceinline__ bool isUnfit() const { return most > 0x1p32f || (most < 0x1p-100f && most > 0.0f); }
 };
+// (by the bits: fast math takes every float for finite)
+__device__ __forceinline__ bool isUnfitSum(float x) {
+  const unsigned magnitude = 2 * __builtin_bit_cast(unsigned, x); // from 2^-60 on, finite, or zero
+  return magnitude - 2u * (67u << 23) >= 2u * ((255u - 67u) << 23) && magnitude != 0;
+}
 __device__ __forceinline__ SplitParts splitFloats(const float (&v)[8], SplitRange& range) {
   typedef float floatx2 __attribute__((ext_vector_type(2)));
   SplitParts s;
@@ -51,8 +60,6 @@ __device__ __forceinline__ SplitParts splitFloats(const float (&v)[8], SplitRang
   }
   return s;
 }
-// (by the bits: fast math takes every float for finite)
-__device__ __forceinline__ bool isFiniteFloat(float x) { return (__builtin_bit_cast(unsigned, x) & 0x7f800000u) != 0x7f800000u; }
 // The six products of the parts of 16 rows and 16 columns, 32 terms each, in the order of `q`; the last one is high * high.
 constexpr int kSplitProducts = 6;
 __device__ __forceinline__ constexpr int splitPartA(int q) { return q == 0 ? 2 : q == 1 || q == 3 ? 1 : 0; }
@@ -60,7 +67,7 @@ __device__ __forceinline__ constexpr int splitPartB(int q) { return q == 2 ? 2 :
 }
 )HIP";
 
-// A convolution in kernels the mapper gives to it (split_convolution.h), stride 1, no padding:
+// A convolution in kernels the mapper gives to it (mapper.cc, takeSplitConvolution), stride 1, no padding:
 //
 //   O(n, g, f, h, w) = sum over c, kh, kw of I(n, g, c, h + kh, w + kw) * W1(g, f, c, kh, kw)  [+ B(g, f)]
 //
@@ -132,8 +139,8 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 #pragma unroll
         for (int e = 0; e < 8; ++e) rawW[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsW, fromW[i] + e * kPlaces * 4, 0, 0));
     };
-    SplitRange range;
-    auto lay = [&](float (&v)[8], int firstChannel, ldschar* to, int part) __attribute__((always_inline)) {
+    SplitRange rangeI, rangeW;
+    auto lay = [&](float (&v)[8], int firstChannel, ldschar* to, int part, SplitRange& range) __attribute__((always_inline)) {
       if constexpr (C % CC != 0) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = firstChannel + e < C ? v[e] : 0.0f;
@@ -171,9 +178,9 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 #pragma unroll 1
     for (int c = 0; c < kChunks; ++c) {
 #pragma unroll
-      for (int i = 0; i < kTurnsI; ++i) lay(rawI[i], c * CC + 8 * (tmin(i * kThreads + tid, kItemsI - 1) / kPixels), li + toI[i], kPartI);
+      for (int i = 0; i < kTurnsI; ++i) lay(rawI[i], c * CC + 8 * (tmin(i * kThreads + tid, kItemsI - 1) / kPixels), li + toI[i], kPartI, rangeI);
 #pragma unroll
-      for (int i = 0; i < kTurnsW; ++i) lay(rawW[i], c * CC + 8 * (tmin(i * kThreads + tid, kItemsW - 1) % kSlots / kPlaces), lw + toW[i], kPartW);
+      for (int i = 0; i < kTurnsW; ++i) lay(rawW[i], c * CC + 8 * (tmin(i * kThreads + tid, kItemsW - 1) % kSlots / kPlaces), lw + toW[i], kPartW, rangeW);
       __syncthreads();
       load(tmin(c + 1, kChunks - 1) * CC);
 #pragma unroll
@@ -199,14 +206,14 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       }
       __syncthreads();
     }
-    bool again = range.isTooSmall();
+    bool again = rangeI.isUnfit() || rangeW.isUnfit();
 #pragma unroll
     for (int t = 0; t < PW; ++t)
 #pragma unroll
       for (int f = 0; f < FT; ++f) {
         large[t][f] += small[t][f];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) again |= !isFiniteFloat(large[t][f][e]);
+        for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
       }
     if (__syncthreads_or(again)) { // (what the parts cannot hold: rare, and slow)
 #pragma unroll 1
@@ -244,6 +251,221 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
           for (int e = 0; e < 4; ++e) {
             if (p + e < kPlane) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)v[e]), rsO, (at + e) * 4, 0, 16);
           }
+        }
+      }
+    }
+  }
+};
+}
+)HIP";
+
+// A product of matrices in kernels the mapper gives to it (mapper.cc, takeSlicedProduct):
+//
+//   O(m, n) = sum over k of A * B [+ bias(n)], A stored (m, k) or (k, m), B stored (n, k) or (k, n)
+//
+// GA x GB x S wavefronts a block; one computes TA x TB tiles of 16 x 16 outputs over every S-th step of 32 reduction points.
+// There is no LDS and no barrier in its loop: the lanes load what the instruction wants of them straight from memory,
+// a step ahead, and split it in registers.  With the reduction innermost a lane group reads 64 bytes of its rows; with it
+// outermost a lane reads TA (TB) neighbouring positions of a point, which become the same row (column) of as many tiles, so
+// that a tile holds every TA-th position.  As the wavefronts of a block divide the reduction, each element of its rows and
+// columns is loaded and split once a block, and a sum is S short chains.  The partial tiles meet in LDS, are added and
+// stored in 256-byte runs.
+//
+// What bounds it at 1000^3 (64 x 64 outputs a block, 8 slices, one block a compute unit; 17.4 us, 23.4 in the general pipeline, whose matrix
+// cores alone take 13.3): the 11 us of splitting and multiplying, which one wavefront's instructions cannot overlap beyond two
+// vector instructions a multiplication, the first loads (2 us), the sums' way through LDS and the launch.
+// Operands laid in LDS as parts and shared by the wavefronts of a block: 22.4 us there, 92 at 2048^3 (here 89, given tiles
+// 126.7): the same work behind barriers.  Parts through v_dot2_f32_bf16 save a third of the vector instructions, but it occupies the
+// matrix cores.  Steps two ahead in registers, parts of the next step made under the multiplications of this one: 18.2 to 25.
+constexpr const char* kDeviceSlicedProduct = R"HIP(
+namespace __tc {
+typedef __attribute__((address_space(3))) float ldsfloat;
+typedef __attribute__((address_space(3))) floatx4 ldsfloatx4;
+template <bool KInner, int P, int K, int TP> struct SlicedOperand {
+  static constexpr int kOffsets = KInner ? TP : 8;
+  const float* p;
+  int group;             // of 16 lanes
+  int offset[kOffsets];  // bytes from the step's first point: of this lane's rows, or of its points
+  float value[TP][8];
+  // the reduction points of a lane group, the same in both operands
+  static __device__ __forceinline__ constexpr int point(int g, int j) { return 4 * g + (j & 3) + (j >> 2) * 16; }
+  static __device__ __forceinline__ int position(int tile, int r) { return KInner ? 16 * tile + r : TP * r + tile; }
+  __device__ __forceinline__ void init(const float* base, int first, int lane) {
+    p = base;
+    group = lane >> 4;
+    const int r = lane & 15;
+#pragma unroll
+    for (int i = 0; i < kOffsets; ++i) {
+      offset[i] = (KInner ? tmin(first + 16 * i + r, P - 1) * K + point(group, 0) : point(group, i) * P + tmin(first + TP * r, P - 1)) * 4;
+    }
+  }
+  // (the descriptor begins at the step and ends with the operand: what lies behind, and steps past the last, read zeros)
+  __device__ __forceinline__ void load(int k0) {
+    typedef float floatx2 __attribute__((ext_vector_type(2)));
+    const int skip = KInner ? k0 : k0 * P;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(p + (k0 < K ? skip : 0)), 0, k0 < K ? (P * K - skip) * 4 : 0, 0x00020000);
+    if constexpr (KInner) {
+#pragma unroll
+      for (int y = 0; y < TP; ++y)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const floatx4 v = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, offset[y] + 64 * h, 0, 0));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) value[y][4 * h + e] = v[e];
+        }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (TP == 4) {
+          const floatx4 v = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, offset[j], 0, 0));
+#pragma unroll
+          for (int y = 0; y < 4; ++y) value[y][j] = v[y];
+        } else if constexpr (TP == 2) {
+          const floatx2 v = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(rs, offset[j], 0, 0));
+#pragma unroll
+          for (int y = 0; y < 2; ++y) value[y][j] = v[y];
+        } else {
+          value[0][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, offset[j], 0, 0));
+        }
+      }
+    }
+  }
+  // zeros behind the end of a row, where the next one begins
+  __device__ __forceinline__ void cut(int k0) {
+    if constexpr (KInner && K % 32 != 0) {
+      if (k0 + 32 > K) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const bool is = k0 + point(group, j) < K;
+#pragma unroll
+          for (int y = 0; y < TP; ++y) value[y][j] = is ? value[y][j] : 0.0f;
+        }
+      }
+    }
+  }
+};
+
+template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, int TB, int GA, int GB, int S> struct SlicedProduct {
+  static_assert((AKInner || TA == 1 || TA == 2 || TA == 4) && (TB == 1 || TB == 2 || TB == 4), "positions a lane loads at once");
+  static constexpr int kRowsOfBlock = 16 * TA * GA, kColumnsOfBlock = 16 * TB * GB;
+  static constexpr int kRows = (M + kRowsOfBlock - 1) / kRowsOfBlock, kColumns = (N + kColumnsOfBlock - 1) / kColumnsOfBlock, kBlocks = kRows * kColumns;
+  static constexpr int kPitch = 16 * TB + 4, kTile = 16 * TA * kPitch, kLds = 4 * GA * GB * S * kTile; // (floats of a row and a tile of partial sums, bytes of all)
+  static __device__ __forceinline__ void run(float* pO, const float* pA, const float* pB, const float* pBias, ldschar* lds) {
+    const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int r = lane & 15, g = lane >> 4, slice = wave % S, ga = wave / S % GA, gb = wave / S / GA;
+    // Blocks go round-robin to the 8 XCDs: each takes a run of them in stripes of four block columns, which share rows in its L2.
+    const int id = blockIdx.x + gridDim.x * blockIdx.y, xcd = id & 7, run = xcd * (kBlocks / 8) + tmin(xcd, kBlocks % 8) + (id >> 3);
+    const int stripe = run / (4 * kRows), width = tmin(4, kColumns - 4 * stripe), in = run - stripe * 4 * kRows;
+    const int m0 = in / width * kRowsOfBlock + 16 * TA * ga, n0 = (4 * stripe + in % width) * kColumnsOfBlock + 16 * TB * gb;
+    SlicedOperand<AKInner, M, K, TA> a;
+    SlicedOperand<BKInner, N, K, TB> b;
+    a.init(pA, m0, lane);
+    b.init(pB, n0, lane);
+    // (small products have sums of their own where the registers hold them)
+    constexpr int kSums = TA * TB < 16 ? 2 : 1;
+    floatx4 sums[kSums][TB][TA];
+#pragma unroll
+    for (int d = 0; d < kSums; ++d)
+#pragma unroll
+      for (int x = 0; x < TB; ++x)
+#pragma unroll
+        for (int y = 0; y < TA; ++y) sums[d][x][y] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    SplitRange rangeA, rangeB;
+    a.load(32 * slice);
+    b.load(32 * slice);
+    constexpr int kTurns = ((K + 31) / 32 + S - 1) / S;
+#pragma unroll 1
+    for (int t = 0; t < kTurns; ++t) {
+      const int k0 = 32 * (slice + t * S);
+      SplitParts pa[TA], pb[TB];
+      a.cut(k0);
+#pragma unroll
+      for (int y = 0; y < TA; ++y) pa[y] = splitFloats(a.value[y], rangeA);
+      // (or the scheduler puts the loads in front of the last uses of what they overwrite, and waits for them at the end of the turn)
+      __builtin_amdgcn_sched_barrier(0);
+      a.load(k0 + 32 * S);
+      b.cut(k0);
+#pragma unroll
+      for (int x = 0; x < TB; ++x) pb[x] = splitFloats(b.value[x], rangeB);
+      b.load(k0 + 32 * S);
+#pragma unroll
+      for (int x = 0; x < TB; ++x)
+#pragma unroll
+        for (int q = 0; q < kSplitProducts; ++q)
+#pragma unroll
+          for (int y = 0; y < TA; ++y) {
+            floatx4& sum = sums[q == kSplitProducts - 1 ? 0 : kSums - 1][x][y];
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[x].part[splitPartB(q)], pa[y].part[splitPartA(q)], sum, 0, 0, 0);
+          }
+    }
+    // A lane holds columns 4 g ... 4 g + 3 of its tiles, in whatever order the tiles hold the positions: four neighbouring ones in LDS.
+    ldsfloat* mine = (ldsfloat*)lds + wave * kTile;
+#pragma unroll
+    for (int y = 0; y < TA; ++y) {
+#pragma unroll
+      for (int x = 0; x < TB; ++x) {
+        if constexpr (kSums == 2) sums[0][x][y] += sums[1][x][y];
+      }
+      ldsfloat* row = mine + a.position(y, r) * kPitch;
+#pragma unroll
+      for (int x = 0; x < TB; ++x) {
+        if constexpr (BKInner) {
+          *(ldsfloatx4*)(row + 16 * x + 4 * g) = sums[0][x][y];
+        } else {
+          floatx4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = sums[0][(4 * x + e) % TB][y][(4 * x + e) / TB];
+          *(ldsfloatx4*)(row + 4 * TB * g + 4 * x) = v;
+        }
+      }
+    }
+    __syncthreads();
+    constexpr int kVectors = 4 * TB, kUnits = 16 * TA * kVectors / 64, kShare = (kUnits + S - 1) / S; // 16-byte vectors of a row, 64 of them, of a slice
+    const ldsfloat* from = (const ldsfloat*)lds + (wave - slice) * kTile;
+    floatx4 sum[kShare];
+    bool again = rangeA.isUnfit() || rangeB.isUnfit();
+#pragma unroll
+    for (int i = 0; i < kShare; ++i) {
+      const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
+      const ldsfloat* at = from + unit / kVectors * kPitch + unit % kVectors * 4;
+      sum[i] = *(const ldsfloatx4*)at;
+#pragma unroll
+      for (int s = 1; s < S; ++s) sum[i] += *(const ldsfloatx4*)(at + s * kTile);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) again |= isUnfitSum(sum[i][e]);
+    }
+    if (__syncthreads_or(again)) { // (what the parts cannot hold: rare, and slow)
+      constexpr int kOutputs = 16 * TA * 16 * TB / S;
+#pragma unroll 1
+      for (int i = slice * kOutputs + lane; i < (slice + 1) * kOutputs; i += 64) {
+        const int m = m0 + i / (16 * TB), n = n0 + i % (16 * TB);
+        if (m >= M || n >= N) continue;
+        float v = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) v = __builtin_fmaf(pA[AKInner ? m * K + k : k * M + m], pB[BKInner ? n * K + k : k * N + n], v);
+        if constexpr (Bias) v += pBias[n];
+        pO[m * N + n] = v;
+      }
+      return;
+    }
+    typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)pO, 0, M * N * 4, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kShare; ++i) {
+      if (kUnits % kShare != 0 && slice * kShare + i >= kUnits) continue;
+      if (kShare * S > kUnits && slice * kShare + i >= kUnits) continue;
+      const int unit = (slice * kShare + i) * 64 + lane, m = m0 + unit / kVectors, n = n0 + unit % kVectors * 4;
+      if (M % kRowsOfBlock != 0 && m >= M) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (Bias) sum[i][e] += pBias[tmin(n + e, N - 1)];
+      }
+      if (N % kColumnsOfBlock == 0 || n + 4 <= N) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, sum[i]), rs, (m * N + n) * 4, 0, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (n + e < N) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)sum[i][e]), rs, (m * N + n + e) * 4, 0, 16);
         }
       }
     }

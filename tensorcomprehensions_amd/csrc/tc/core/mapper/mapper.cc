@@ -624,6 +624,125 @@ void takeSplitConvolution(KernelPlan& k, StagePlan& st, const HipMappingOptions&
   k.block = {{64, shape.filterWaves * shape.pixelWaves, 1}};
 }
 
+// Products of float matrices O(m, n) +=! A * B, whichever side of the operands the reduction is on, with or without a bias
+// of the columns added behind them, go to __tc::SlicedProduct (hip_split_products.h) where that is the faster form.
+// Both forms are judged by an estimate in microseconds, fitted by least squares of the relative error to the times of 75 products
+// (8 to 4096 rows, columns and points, 6e7 to 9e9 multiplications; twelve shapes of the sliced form each): 9 % off on average for the sliced
+// form, 11 % for the given tiles.  The shape the estimate takes is 4 % slower than the best one timed on average.  The sliced form is
+// taken where it comes out 10 % faster (a quarter with the reduction innermost in both operands, which the general pipeline copies best): 1000^3
+// 23.8 -> 16.5 us, 691x1840x792 36 -> 25, 45x2699x2516 27.5 -> 13.3, 986x1987x71 14.6 -> 10.2, 2048^3 127 -> 94; of the 75 it took
+// 53, 1.23 times as fast by geometric mean, the worst 15 % slower (blocks of four wavefronts in more than one round of two a compute unit, which
+// are left out since).
+// Tiles that were fitted to the device stay as they are, and are taken where the sliced form has their shape.  The general
+// pipeline keeps products of fewer than 1.06e8 multiplications or 128 reduction points and those whose tiles leave two compute units of three
+// idle.
+struct SlicedProductShape {
+  int64_t rowTiles = 0, columnTiles = 0, rowWaves = 0, columnWaves = 0, slices = 0, lds = 0;
+  double microseconds = 0;
+};
+void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits, bool wide) {
+  if (k.stages.size() != 1 || wide || waves != 8 || !o.prefetchSharedValue || !o.useSharedMemoryValue || st.atomic) return;
+  if (st.stmts.size() > 2 || !st.stmts[0].init || st.vars.size() != 3 || st.numParallel != 2 || st.lhsSubs.size() != 2) return;
+  LoopVar &m = st.vars[0], &n = st.vars[1];
+  const LoopVar& r = st.vars[2];
+  for (const auto& v : st.vars) {
+    if (v.min != 0) return;
+  }
+  auto isVar = [](const ExprRef& e, const LoopVar& v) { return e->kind == Expr::Var && e->name == v.name; };
+  auto hasExtents = [&](const std::string& tensor, const std::vector<int64_t>& extents) {
+    const auto& view = st.views.at(tensor);
+    int64_t bytes = 4;
+    for (auto e : extents) bytes *= e;
+    return view.type == ScalarType{ScalarType::Float, 32} && view.extents == extents && bytes < (int64_t(1) << 31);
+  };
+  if (!isVar(st.lhsSubs[0], m) || !isVar(st.lhsSubs[1], n) || !hasExtents(st.tensor, {m.extent, n.extent})) return;
+  std::string tensors[2], bias;  // of the m and of the n side
+  bool innermost[2];             // the reduction is the last subscript
+  for (const auto& load : st.stmts[0].rhs->args) {
+    if (load->kind != Expr::Load || load->args.size() != 2) return;
+    bool found = false;
+    for (int side = 0; side < 2; ++side) {
+      const LoopVar& v = side == 0 ? m : n;
+      for (int last = 0; last < 2; ++last) {
+        const LoopVar &outer = last ? v : r, &inner = last ? r : v;
+        if (!isVar(load->args[0], outer) || !isVar(load->args[1], inner)) continue;
+        if (!hasExtents(load->name, {outer.extent, inner.extent}) || !tensors[side].empty()) return;
+        tensors[side] = load->name;
+        innermost[side] = last == 1;
+        found = true;
+      }
+    }
+    if (!found) return;
+  }
+  if (st.stmts.size() == 2) { // O(m, n) = O(m, n) + B(n)
+    const StageStmt& add = st.stmts[1];
+    if (add.op != ReduceOp::None || !add.redVars.empty() || add.rhs->kind != Expr::Binary || add.rhs->name != "+") return;
+    for (const auto& load : add.rhs->args) {
+      if (load->kind != Expr::Load) return;
+      if (load->name == st.tensor && load->args.size() == 2 && isVar(load->args[0], m) && isVar(load->args[1], n)) continue;
+      if (!bias.empty() || load->name == st.tensor || load->args.size() != 1 || !isVar(load->args[0], n) || !hasExtents(load->name, {n.extent})) return;
+      bias = load->name;
+    }
+    if (bias.empty()) return;
+  }
+  const double multiplications = 1.0 * m.extent * n.extent * r.extent;
+  if (multiplications < 1.06e8 || r.extent < 128 || r.extent > 65536) return;  // (longer sums are not what isUnfitSum counts on)
+  // a block for every tile of these sizes?
+  auto isOneBlockATile = [&](int64_t rows, int64_t columns) {
+    int axis = 0;
+    for (int position = 0; position < 2; ++position) {
+      const int64_t tiles = position == 0 ? ceilDiv(m.extent, rows) : ceilDiv(n.extent, columns);
+      if (tiles == 1) continue;
+      if (axis >= static_cast<int>(o.grid.size()) || tiles > allowedBlocks(o, axis, position)) return false;
+      ++axis;
+    }
+    return true;
+  };
+  if (!isOneBlockATile(m.tile, n.tile) || 3 * m.numTiles * n.numTiles < limits.computeUnits) return;
+  int64_t lds = limits.ldsBytesPerBlock;
+  if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
+  static const int64_t kShapes[][5] = { // tiles of a wavefront, wavefronts along rows and columns, slices
+      {1, 1, 1, 1, 8}, {1, 2, 1, 1, 8}, {2, 2, 1, 1, 8}, {2, 4, 1, 1, 8}, {4, 2, 1, 1, 8}, {4, 4, 1, 1, 8}, {2, 2, 1, 1, 4}, {2, 4, 1, 1, 4},
+      {4, 4, 1, 1, 4}, {2, 2, 1, 2, 4}, {2, 4, 2, 1, 4}, {4, 2, 1, 2, 4}, {4, 4, 2, 1, 4}, {4, 4, 1, 2, 4}, {2, 2, 2, 2, 2}, {4, 4, 2, 2, 2}};
+  SlicedProductShape best;
+  for (const auto& s : kShapes) {
+    SlicedProductShape c;
+    c.rowTiles = s[0], c.columnTiles = s[1], c.rowWaves = s[2], c.columnWaves = s[3], c.slices = s[4];
+    const int64_t rows = 16 * c.rowTiles * c.rowWaves, columns = 16 * c.columnTiles * c.columnWaves;
+    if (st.fittedToDevice ? rows != m.tile || columns != n.tile : !isOneBlockATile(rows, columns)) continue;
+    const int64_t used = c.rowWaves * c.columnWaves * c.slices, area = c.rowTiles * c.columnTiles;
+    c.lds = 64 * used * c.rowTiles * (16 * c.columnTiles + 4);
+    const int64_t blocks = ceilDiv(m.extent, rows) * ceilDiv(n.extent, columns), rounds = ceilDiv(blocks, limits.computeUnits);
+    if (c.lds > lds || (used == 4 && area == 16 && rounds > 2)) continue;
+    const int64_t resident = std::max<int64_t>(1, std::min(limits.ldsBytesPerBlock / c.lds, (area <= 4 ? 16 : 8) / used));
+    const int64_t steps = ceilDiv(ceilDiv(r.extent, 32), c.slices), inTurn = ceilDiv(rounds, resident);
+    c.microseconds = 2.71 + 0.01 * rounds * used * (steps * (0.52 * area + 2.31 * (c.rowTiles + c.columnTiles) +
+                                                             0.81 * (innermost[0] * c.rowTiles + innermost[1] * c.columnTiles)) + 0.66 * area) +
+        inTurn * (0.1 + 0.267 * steps) + 0.66e-6 * m.extent * n.extent;
+    if (best.slices == 0 || c.microseconds < best.microseconds) best = c;
+  }
+  if (best.slices == 0) return;
+  // the general pipeline under the tiles the stage has now
+  const int64_t tiles = ceilDiv(m.tile, 16) * ceilDiv(n.tile, 16), rounds = ceilDiv(m.numTiles * n.numTiles, limits.computeUnits);
+  const double points = 1e-3 * (r.numTiles > 1 ? r.numTiles * r.tile : 16 * ceilDiv(r.extent, 16));
+  const double given = 1.37 + rounds * (points * (0.89 * tiles + 0.211 * std::sqrt(1.0 * tiles)) + 0.608) + 0.13 * r.numTiles +
+      (tiles < 8 ? 1.93 * points : 0) + 1.21e-6 * m.extent * n.extent;
+  if ((innermost[0] && innermost[1] ? 1.25 : 1.1) * best.microseconds >= given) return;
+  m.tile = 16 * best.rowTiles * best.rowWaves;
+  n.tile = 16 * best.columnTiles * best.columnWaves;
+  for (LoopVar* v : {&m, &n}) {
+    v->tile = std::min(v->tile, v->extent);
+    v->numTiles = ceilDiv(v->extent, v->tile);
+  }
+  std::ostringstream ss;
+  ss << (bias.empty() ? "false" : "true") << ", " << (innermost[0] ? "true" : "false") << ", " << (innermost[1] ? "true" : "false");
+  for (int64_t x : {m.extent, n.extent, r.extent, best.rowTiles, best.columnTiles, best.rowWaves, best.columnWaves, best.slices}) ss << ", " << x;
+  ss << ">::run(p" << st.tensor << ", p" << tensors[0] << ", p" << tensors[1] << ", " << (bias.empty() ? "nullptr" : "p" + bias);
+  st.slicedProduct = ss.str();
+  st.slicedProductLds = best.lds;
+  st.waves = best.rowWaves * best.columnWaves * best.slices;
+}
+
 // A contraction whose threads keep whole sums (no matrix cores, no LDS, one axis of threads) under tile sizes that were made
 // for other extents.  Returns the innermost variable where it takes a block axis behind those of the options.
 //   A variable without a block axis is not walked tile by tile where all its points fit the registers under the tiles given
@@ -787,6 +906,7 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) takeLargeHalfProduct(k, st, o, waves, limits, kc.wide);
     if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
+    if (st.mfma) takeSlicedProduct(k, st, o, waves, limits, kc.wide);
     if (st.mfma) takeSplitConvolution(k, st, o, waves, limits, kc.wide);
     if (!st.splitConvolution.empty()) return;
     const LoopVar* spread = spreadContraction(k, st, o, limits);
@@ -808,6 +928,10 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
       v.gridExtent = std::min<int64_t>(allowedBlocks(o, axis, position), v.numTiles);
       gridUse[axis] = std::max(gridUse[axis], v.gridExtent);
       ++axis;
+    }
+    if (!st.slicedProduct.empty()) {
+      blockUse = {{64, st.waves, 1}};
+      continue;
     }
     if (st.mfma) {
       // one wavefront per 16x16 output tile; the block holds as many wavefronts as the block
@@ -998,6 +1122,16 @@ void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
     em.line("__tc::largeHalfProduct<" + k.stages[0].largeHalfProduct + ", (__tc::ldschar*)tiles_);");
     em.close();
     k.ldsBytes = kLargeHalfLds;
+    return;
+  }
+  if (!k.stages[0].slicedProduct.empty()) {
+    em.open(kernelSignature(kc.f, k.name, kc.NT()));
+    for (const auto& p : kc.f.params) em.line("(void)" + p.first + ";");
+    em.line("// matrix cores: the bf16 parts of floats, each wavefront a slice of the reduction");
+    em.line("__shared__ __attribute__((aligned(16))) char sums_[" + std::to_string(k.stages[0].slicedProductLds) + "];");
+    em.line("__tc::SlicedProduct<" + k.stages[0].slicedProduct + ", (__tc::ldschar*)sums_);");
+    em.close();
+    k.ldsBytes = k.stages[0].slicedProductLds;
     return;
   }
   if (!k.stages[0].splitConvolution.empty()) {
@@ -1859,14 +1993,17 @@ MappedProgram mapToHip(
     emitKernel(kc, limits, *bodies.back());
   }
   src << "// generated by the TC HIP mapper for gfx950; function " << f.name << "\n";
-  bool halfProducts = false, largeHalfProducts = false, splitConvolutions = false;
+  bool halfProducts = false, largeHalfProducts = false, splitConvolutions = false, slicedProducts = false;
   for (const auto& b : bodies) {
     halfProducts |= b->out.str().find("__tc::multiplyHalves(") != std::string::npos;
     largeHalfProducts |= b->out.str().find("__tc::largeHalfProduct<") != std::string::npos;
     splitConvolutions |= b->out.str().find("__tc::SplitConvolution<") != std::string::npos;
+    slicedProducts |= b->out.str().find("__tc::SlicedProduct<") != std::string::npos;
   }
   src << hip::deviceLibrary(anyThreadReduction, halfProducts, largeHalfProducts);
-  if (splitConvolutions) src << hip::kDeviceSplitParts << hip::kDeviceSplitConvolution;
+  if (splitConvolutions || slicedProducts) src << hip::kDeviceSplitParts;
+  if (splitConvolutions) src << hip::kDeviceSplitConvolution;
+  if (slicedProducts) src << hip::kDeviceSlicedProduct;
   for (const auto& b : bodies) src << "\n" << b->out.str();
   prog.source = src.str();
   return prog;

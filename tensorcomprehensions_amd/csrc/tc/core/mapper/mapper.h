@@ -115,6 +115,9 @@ struct StagePlan {
   // stage), and the LDS that takes.
   std::string splitConvolution;
   int64_t splitConvolutionLds = 0;
+  // A product of floats computed by __tc::SlicedProduct (likewise).
+  std::string slicedProduct;
+  int64_t slicedProductLds = 0;
   // The stage adds partial sums into its tensor with atomics: its first parallel variable numbers
   // slices of the reduction and is no subscript of the tensor.
   bool atomic = false;

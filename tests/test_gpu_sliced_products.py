@@ -1,0 +1,103 @@
+"""Products of float matrices whose wavefronts divide the reduction, each float in three bf16 parts (__tc::SlicedProduct): every order
+of the two operands against the same sums in 64 bits, at sizes around the tiles and steps, and for values the parts cannot hold."""
+import numpy as np
+import pytest
+import torch
+
+import tensorcomprehensions_amd as tc
+
+pytestmark = pytest.mark.gpu
+
+
+def source(a_inner, b_inner, bias=False):
+    a = ("M, K", "m, r_k") if a_inner else ("K, M", "r_k, m")
+    b = ("N, K", "n, r_k") if b_inner else ("K, N", "r_k, n")
+    return (f"def f(float({a[0]}) A, float({b[0]}) B{', float(N) C' if bias else ''}) -> (O) {{ O(m, n) +=! A({a[1]}) * B({b[1]})"
+            + (" O(m, n) = O(m, n) + C(n) }" if bias else " }"))
+
+
+def run(m, n, k, a_inner, b_inner, a, b, bias=None):
+    outputs = m * n
+    tile = "16,32,128" if outputs <= 1 << 18 else "64,64,32" if outputs <= 1 << 21 else "128,128,16"
+    text = source(a_inner, b_inner, bias is not None)
+    ins = [(a if a_inner else a.t()).contiguous().cuda(), (b if b_inner else b.t()).contiguous().cuda()] + ([] if bias is None else [bias.cuda()])
+    executor = tc.compile(text, "f", ins, f"naive;tile={tile};mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1")
+    assert "__tc::SlicedProduct<" in executor.compiled_source.split('extern "C"')[-1]
+    out = torch.full((m, n), float("nan"), device="cuda")
+    tc.run(executor, ins, [out])
+    return out.cpu()
+
+
+SIZES = [
+    (1000, 1000, 1000),     # 64 x 64 outputs a block, the last step of eight points
+    (691, 792, 1840),
+    (254, 292, 1500),       # 16 x 32
+    (655, 1031, 513),       # one point in the last step, an odd number of columns
+    (45, 2516, 2699),       # fewer rows than a tile of 48 has
+    (986, 71, 1987),
+    (497, 681, 1530),       # 64 x 32
+    (2048, 2048, 160),      # fewer steps than slices have turns
+    (2062, 1895, 768),      # 128 x 128, four rectangles of wavefronts
+]
+
+
+@pytest.mark.parametrize("a_inner,b_inner,bias", [(True, False, False), (True, True, True), (False, False, False), (False, True, True)])
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_sums(m, n, k, a_inner, b_inner, bias):
+    print(m, n, k, a_inner, b_inner, flush=True)
+    generator = torch.Generator().manual_seed(m)
+    ints = lambda *s: torch.randint(-8, 9, s, generator=generator).float()  # noqa: E731
+    a, b, c = ints(m, k), ints(n, k), ints(n)
+    try:
+        got = run(m, n, k, a_inner, b_inner, a, b, c if bias else None)
+    except AssertionError:
+        if a_inner and not b_inner:
+            raise
+        pytest.skip("the general pipeline is as fast for this order of the operands")
+    want = a.double() @ b.double().t()
+    assert torch.equal(got.double(), want + c if bias else want)     # (sums of whole numbers are exact)
+    a, b, c = (torch.randn(s, generator=generator) for s in ((m, k), (n, k), (n,)))
+    got = run(m, n, k, a_inner, b_inner, a, b, c if bias else None).double()
+    want, magnitudes = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    if bias:
+        want, magnitudes = want + c, magnitudes + c.abs()
+    # one rounding of 2^-24 a term and the bias, in whatever order, and 2^-26 of every product for the parts left out
+    assert ((got - want).abs() <= (k + 2) * 2.0 ** -24 * magnitudes).all()
+
+
+@pytest.mark.parametrize("case", ["infinity", "nan", "rounds to infinity", "small", "small rows", "denormal", "large", "large sums", "zero rows"])
+def test_values_the_parts_cannot_hold(case):
+    m, n, k = 254, 292, 1500
+    generator = torch.Generator().manual_seed(2)
+    a, b = torch.randn(m, k, generator=generator), torch.randn(n, k, generator=generator)
+    if case == "infinity":
+        a.view(-1)[[5, 47110, -1]] = torch.tensor([np.inf, -np.inf, np.inf])
+    elif case == "nan":
+        a.view(-1)[[5, 47110]] = np.nan
+    elif case == "rounds to infinity":
+        a.view(-1)[::10001] = 3.4e38              # its nearest bf16 is infinite
+        b *= 2.0 ** -20
+    elif case == "small":
+        a *= 2.0 ** -110                          # what is below 2^-134 of them is lost
+    elif case == "small rows":
+        a[::7] *= 2.0 ** -120
+    elif case == "denormal":
+        a *= 2.0 ** -140
+    elif case == "large":
+        a[3] *= 2.0 ** -110                       # beside values that lift its low parts out of the denormal numbers
+        b *= 2.0 ** 90
+    elif case == "large sums":
+        a *= 2.0 ** 100
+        b *= 2.0 ** 30                            # beyond the largest float
+    else:
+        a[::3] = 0
+    got = run(m, n, k, True, False, a, b).double()
+    want, magnitudes = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    finite = torch.isfinite(want) & (magnitudes < 3.4e38)
+    # (a denormal sum is a whole number of 2^-149)
+    assert ((got - want).abs()[finite] <= (k + 2) * (2.0 ** -24 * magnitudes[finite] + 2.0 ** -149)).all()
+    if case in ("infinity", "nan"):
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]) and torch.equal(torch.isinf(got), torch.isinf(want))
+    if case == "zero rows":
+        assert (got[::3] == 0).all()
