@@ -11,6 +11,7 @@
 #include <sstream>
 
 #include "tc/core/check.h"
+#include "tc/core/hip/hip_column_sums.h"
 #include "tc/core/hip/hip_libraries.h"
 #include "tc/core/hip/hip_split_products.h"
 
@@ -743,6 +744,31 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
   st.waves = best.rowWaves * best.columnWaves * best.slices;
 }
 
+// Sums of the columns of a float matrix, O(n) +=! A(r, n), whose threads keep whole sums, under tiles that leave three quarters of the
+// device's wavefronts out, go to __tc::columnSums (hip_column_sums.h): rows on other threads as well, whatever the options say about
+// unrolling.  (One axis of threads, one block a tile, no matchLibraryCalls, which has the rows on threads as it is.)
+constexpr int64_t kColumnSumWaves = 16;
+void takeColumnSums(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits, bool wide) {
+  if (k.stages.size() != 1 || wide || st.atomic || o.generic.matchLibraryCallsValue || o.block.size() != 1 || !o.generic.hasTiling) return;
+  if (st.stmts.size() != 1 || !st.stmts[0].init || st.stmts[0].op != ReduceOp::Plus || st.vars.size() != 2 || st.numParallel != 1) return;
+  const LoopVar &n = st.vars[0], &r = st.vars[1];
+  if (n.min != 0 || r.min != 0 || !r.reduction || st.lhsSubs.size() != 1) return;
+  auto isVar = [](const ExprRef& e, const LoopVar& v) { return e->kind == Expr::Var && e->name == v.name; };
+  const ExprRef& load = st.stmts[0].rhs;
+  const ScalarType f32{ScalarType::Float, 32};
+  if (load->kind != Expr::Load || load->args.size() != 2 || !isVar(load->args[0], r) || !isVar(load->args[1], n) || !isVar(st.lhsSubs[0], n)) return;
+  const auto &a = st.views.at(load->name), &out = st.views.at(st.tensor);
+  if (a.type != f32 || out.type != f32 || a.extents != std::vector<int64_t>{r.extent, n.extent} || out.extents != std::vector<int64_t>{n.extent}) return;
+  const int64_t waves = n.numTiles * ceilDiv(std::min<int64_t>(static_cast<int64_t>(o.block[0]), n.tile), limits.wavefront);
+  if (n.numTiles > allowedBlocks(o, 0, 0) || waves >= limits.computeUnits || r.extent < 4 * kColumnSumWaves || r.extent * n.extent >= (int64_t(1) << 29)) return;
+  if (limits.maxThreadsPerBlock < 64 * kColumnSumWaves) return;
+  std::ostringstream ss;
+  ss << r.extent << ", " << n.extent << ", " << kColumnSumWaves << ">(p" << st.tensor << ", p" << load->name;
+  st.columnSums = ss.str();
+  k.grid = {{ceilDiv(n.extent, 16), 1, 1}};
+  k.block = {{64, kColumnSumWaves, 1}};
+}
+
 // A contraction whose threads keep whole sums (no matrix cores, no LDS, one axis of threads) under tile sizes that were made
 // for other extents.  Returns the innermost variable where it takes a block axis behind those of the options.
 //   A variable without a block axis is not walked tile by tile where all its points fit the registers under the tiles given
@@ -909,6 +935,8 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) takeSlicedProduct(k, st, o, waves, limits, kc.wide);
     if (st.mfma) takeSplitConvolution(k, st, o, waves, limits, kc.wide);
     if (!st.splitConvolution.empty()) return;
+    takeColumnSums(k, st, o, limits, kc.wide);
+    if (!st.columnSums.empty()) return;
     const LoopVar* spread = spreadContraction(k, st, o, limits);
     // blocks: outermost shared parallel variables, x first
     int axis = 0, position = -1;
@@ -1122,6 +1150,15 @@ void emitKernel(KernelCtx& kc, const DeviceLimits& limits, Emitter& em) {
     em.line("__tc::largeHalfProduct<" + k.stages[0].largeHalfProduct + ", (__tc::ldschar*)tiles_);");
     em.close();
     k.ldsBytes = kLargeHalfLds;
+    return;
+  }
+  if (!k.stages[0].columnSums.empty()) {
+    em.open(kernelSignature(kc.f, k.name, kc.NT()));
+    for (const auto& p : kc.f.params) em.line("(void)" + p.first + ";");
+    em.line("__shared__ float sums_[" + std::to_string(64 * kColumnSumWaves) + "];");
+    em.line("__tc::columnSums<" + k.stages[0].columnSums + ", sums_);");
+    em.close();
+    k.ldsBytes = 4 * 64 * kColumnSumWaves;
     return;
   }
   if (!k.stages[0].slicedProduct.empty()) {
@@ -1993,17 +2030,19 @@ MappedProgram mapToHip(
     emitKernel(kc, limits, *bodies.back());
   }
   src << "// generated by the TC HIP mapper for gfx950; function " << f.name << "\n";
-  bool halfProducts = false, largeHalfProducts = false, splitConvolutions = false, slicedProducts = false;
+  bool halfProducts = false, largeHalfProducts = false, splitConvolutions = false, slicedProducts = false, columnSums = false;
   for (const auto& b : bodies) {
     halfProducts |= b->out.str().find("__tc::multiplyHalves(") != std::string::npos;
     largeHalfProducts |= b->out.str().find("__tc::largeHalfProduct<") != std::string::npos;
     splitConvolutions |= b->out.str().find("__tc::SplitConvolution<") != std::string::npos;
     slicedProducts |= b->out.str().find("__tc::SlicedProduct<") != std::string::npos;
+    columnSums |= b->out.str().find("__tc::columnSums<") != std::string::npos;
   }
   src << hip::deviceLibrary(anyThreadReduction, halfProducts, largeHalfProducts);
   if (splitConvolutions || slicedProducts) src << hip::kDeviceSplitParts;
   if (splitConvolutions) src << hip::kDeviceSplitConvolution;
   if (slicedProducts) src << hip::kDeviceSlicedProduct;
+  if (columnSums) src << hip::kDeviceColumnSums;
   for (const auto& b : bodies) src << "\n" << b->out.str();
   prog.source = src.str();
   return prog;

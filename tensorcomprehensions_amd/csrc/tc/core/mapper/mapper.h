@@ -118,6 +118,8 @@ struct StagePlan {
   // A product of floats computed by __tc::SlicedProduct (likewise).
   std::string slicedProduct;
   int64_t slicedProductLds = 0;
+  // Sums of the columns of a matrix, computed by __tc::columnSums (likewise).
+  std::string columnSums;
   // The stage adds partial sums into its tensor with atomics: its first parallel variable numbers
   // slices of the reduction and is no subscript of the tensor.
   bool atomic = false;
