@@ -629,11 +629,11 @@ void takeSplitConvolution(KernelPlan& k, StagePlan& st, const HipMappingOptions&
 // of the columns added behind them, go to __tc::SlicedProduct (hip_split_products.h) where that is the faster form.
 // Both forms are judged by an estimate in microseconds, fitted by least squares of the relative error to the times of 75 products
 // (8 to 4096 rows, columns and points, 6e7 to 9e9 multiplications; twelve shapes of the sliced form each): 9 % off on average for the sliced
-// form, 11 % for the given tiles.  The shape the estimate takes is 4 % slower than the best one timed on average.  The sliced form is
-// taken where it comes out 10 % faster (a quarter with the reduction innermost in both operands, which the general pipeline copies best): 1000^3
-// 23.8 -> 16.5 us, 691x1840x792 36 -> 25, 45x2699x2516 27.5 -> 13.3, 986x1987x71 14.6 -> 10.2, 2048^3 127 -> 94; of the 75 it took
-// 53, 1.23 times as fast by geometric mean, the worst 15 % slower (blocks of four wavefronts in more than one round of two a compute unit, which
-// are left out since).
+// form, 11 % for the given tiles; full tiles in four slices took a quarter longer than that fit says in 66 others, and are judged so.
+// The sliced form is taken where it comes out 10 % faster (25 % below 320 points, 35 % with the reduction innermost in both operands, which the
+// general pipeline copies best: with smaller margins products of 250 to 500 thousand results and some 200 points took up to 1.4 times as long
+// as before, 1250 x 208 x 1015 14.6 us for 10.8): 1000^3 22 -> 17 us, 45 x 2516 x 2699 27.1 -> 13.5, 1250 x 1015 x 208 14.5 -> 10.3,
+// 2048^3 126 -> 93 (rows, points, columns); 251 products drawn over these ranges and taken: 1.27 times as fast, the worst 6 % slower.
 // Tiles that were fitted to the device stay as they are, and are taken where the sliced form has their shape.  The general
 // pipeline keeps products of fewer than 1.06e8 multiplications or 128 reduction points and those whose tiles leave two compute units of three
 // idle.
@@ -714,12 +714,13 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
     const int64_t used = c.rowWaves * c.columnWaves * c.slices, area = c.rowTiles * c.columnTiles;
     c.lds = 64 * used * c.rowTiles * (16 * c.columnTiles + 4);
     const int64_t blocks = ceilDiv(m.extent, rows) * ceilDiv(n.extent, columns), rounds = ceilDiv(blocks, limits.computeUnits);
-    if (c.lds > lds || (used == 4 && area == 16 && rounds > 2)) continue;
+    if (c.lds > lds) continue;
     const int64_t resident = std::max<int64_t>(1, std::min(limits.ldsBytesPerBlock / c.lds, (area <= 4 ? 16 : 8) / used));
     const int64_t steps = ceilDiv(ceilDiv(r.extent, 32), c.slices), inTurn = ceilDiv(rounds, resident);
     c.microseconds = 2.71 + 0.01 * rounds * used * (steps * (0.52 * area + 2.31 * (c.rowTiles + c.columnTiles) +
                                                              0.81 * (innermost[0] * c.rowTiles + innermost[1] * c.columnTiles)) + 0.66 * area) +
         inTurn * (0.1 + 0.267 * steps) + 0.66e-6 * m.extent * n.extent;
+    if (area == 16 && c.slices == 4) c.microseconds *= 1.25;
     if (best.slices == 0 || c.microseconds < best.microseconds) best = c;
   }
   if (best.slices == 0) return;
@@ -728,7 +729,8 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
   const double points = 1e-3 * (r.numTiles > 1 ? r.numTiles * r.tile : 16 * ceilDiv(r.extent, 16));
   const double given = 1.37 + rounds * (points * (0.89 * tiles + 0.211 * std::sqrt(1.0 * tiles)) + 0.608) + 0.13 * r.numTiles +
       (tiles < 8 ? 1.93 * points : 0) + 1.21e-6 * m.extent * n.extent;
-  if ((innermost[0] && innermost[1] ? 1.25 : 1.1) * best.microseconds >= given) return;
+  const double margin = innermost[0] && innermost[1] ? 1.35 : r.extent < 320 ? 1.25 : 1.1;
+  if (margin * best.microseconds >= given) return;
   m.tile = 16 * best.rowTiles * best.rowWaves;
   n.tile = 16 * best.columnTiles * best.columnWaves;
   for (LoopVar* v : {&m, &n}) {
