@@ -746,6 +746,37 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
   st.waves = best.rowWaves * best.columnWaves * best.slices;
 }
 
+// A batch of float products, a block for every product and tile of it, whose rows or columns take two tiles: one product a block where
+// there are two products a compute unit.  Every block copies the operands it needs to LDS behind one barrier, so the second tile of rows
+// copies the whole other operand again, often for a few rows: 1024 products 65x128x65 (rows, points, columns) 52 -> 27 us, 768 of 80x80x80 28.9 -> 16.0,
+// 512 of 100x100x100 32.5 -> 23.2, 654 of 68x108x45 19.8 -> 12.5.
+// The tiles stay where the second is nearly full or one product takes more than half of the LDS, with one block of four wavefronts a compute unit
+// then (600 of 128x128x128 34.8 us in tiles, 51 whole; 1314 of 98x128x98 80 and 100; 600 of 128x32x128 12.7 and 15.4), where the
+// rows alone have two tiles and are more than 96 (700 of 128x64x64 13.5 and 14.4; 643 of 101x127x40 21.5 and 23.6) or the blocks are too few without them
+// (716 of 79x12x8 2.9 and 3.8; 586 of 81x18x37 5.5 and 6.1), and of fewer products (140 of 111x67x83 9.4 and 11.0).
+void takeProductsWhole(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits) {
+  constexpr int64_t kMostTiles = 49, kMostRows = 120, kMostRowsAlone = 96;
+  if (k.stages.size() != 1 || st.mfmaBatch.size() != 1 || st.stmts.size() != 1 || !o.useSharedMemoryValue || o.prefetchSharedValue || st.atomic) return;
+  if (st.vars.size() != 4 || st.numParallel != 3 || k.sharedDepth < 3) return;
+  for (const auto& load : st.stmts[0].rhs->args) {
+    if (load->kind != Expr::Load || st.views.at(load->name).type != ScalarType{ScalarType::Float, 32}) return;
+  }
+  const LoopVar &b = st.vars[0], &r = st.vars[3];
+  LoopVar &m = st.vars[1], &n = st.vars[2];
+  if (b.name != st.mfmaBatch[0] || b.tile != 1 || r.numTiles != 1 || b.extent < 2 * limits.computeUnits) return;
+  if (b.numTiles > allowedBlocks(o, 0, 0)) return;
+  if (m.numTiles > 2 || n.numTiles > 2 || m.numTiles * n.numTiles == 1) return;
+  if (ceilDiv(m.extent, 16) * ceilDiv(n.extent, 16) > kMostTiles || m.extent > kMostRows) return;
+  if (n.numTiles == 1 && (m.extent > kMostRowsAlone || b.extent < 3 * limits.computeUnits)) return;
+  int64_t lds = limits.ldsBytesPerBlock / 2;
+  if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
+  if (4 * r.extent * (m.extent + n.extent + 8) > lds) return;
+  for (LoopVar* v : {&m, &n}) {
+    v->tile = v->extent;
+    v->numTiles = 1;
+  }
+}
+
 // Sums of the columns of a float matrix, O(n) +=! A(r, n), whose threads keep whole sums, under tiles that leave three quarters of the
 // device's wavefronts out, go to __tc::columnSums (hip_column_sums.h): rows on other threads as well, whatever the options say about
 // unrolling.  (One axis of threads, one block a tile, no matchLibraryCalls, which has the rows on threads as it is.)
@@ -934,6 +965,7 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) takeLargeHalfProduct(k, st, o, waves, limits, kc.wide);
     if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
+    if (st.mfma) takeProductsWhole(k, st, o, limits);
     if (st.mfma) takeSlicedProduct(k, st, o, waves, limits, kc.wide);
     if (st.mfma) takeSplitConvolution(k, st, o, waves, limits, kc.wide);
     if (!st.splitConvolution.empty()) return;
