@@ -464,9 +464,11 @@ void takeLargeHalfProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions&
 // (1 to 64 images, 3 to 128 channels, 4 to 128 filters, planes of 7 x 7 to 64 x 64, windows of 1, 3 and 5; 7 to 16 shapes of the split form
 // each): 11 % off on average for the split form, 16 % for the given tiles.
 // The shape the estimate takes is 2 % slower than the best one timed on average, a quarter at most.  The split form is taken where it comes
-// out 15 % faster, and half as fast again where an output has fewer than 48 terms (the results' stores bound such a kernel, and the general pipeline
-// has less in front of them).  On 180 other convolutions: group convolutions 1.11 and 1.34 times as fast by geometric
-// mean (of all, taken or not), dense ones 1.03 and 1.04, none of at least 48 terms slower by more than 3 %.  What gains are the
+// out 15 % faster, 40 % without groups, and half as fast again where an output has fewer than 48 terms (the results' stores bound such a kernel, and the general
+// pipeline has less in front of them).  Without groups and with a window of one point the estimate of the given tiles is too high below 96 channels:
+// 12 x 60 x 43 x 22, 60 filters, 4.0 us as given and 5.1 split, 9 x 29 x 31 x 23, 119 filters, 3.9 and 4.9, and they keep them.  With 15 % for all, 12 of 80 drawn
+// convolutions without groups were slower (27 x 8 x 46 x 59, 28 filters 3 x 3, 6.0 and 7.9).  Of 125 drawn group convolutions that were taken none is
+// slower by more than 1 %, 1.7 to 1.8 times as fast by geometric mean; of 70 without groups the worst 7 % slower, 1.33.  What gains are the
 // large ones (16 x 64 x 57 x 57, 64 filters 3 x 3, 42.5 -> 29.6 us; 28 x 65 x 43 x 29, 38 filters, 41 -> 24) and those whose given tiles
 // make few blocks (2 images x 8 groups of 15 channels, 25 x 28, 4 filters 3 x 3, 11.4 -> 4.1; 1 x 5 x 18 x 20 x 27, 18 filters
 // 5 x 5, 36 -> 6.7).
@@ -612,7 +614,8 @@ void takeSplitConvolution(KernelPlan& k, StagePlan& st, const HipMappingOptions&
   int64_t lds = limits.ldsBytesPerBlock;
   if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
   const SplitConvolutionShape shape = bestSplitConvolution(s, waves, lds, limits);
-  const double margin = s.channels * s.kernelHeight * s.kernelWidth < 48 ? 1.5 : 1.15;
+  if (s.groups == 1 && s.kernelHeight * s.kernelWidth == 1 && s.channels < 96) return;
+  const double margin = s.channels * s.kernelHeight * s.kernelWidth < 48 ? 1.5 : s.groups == 1 ? 1.4 : 1.15;
   if (shape.blocks == 0 || margin * shape.microseconds >= givenConvolutionMicroseconds(st, rank, s, waves, limits)) return;
   std::ostringstream ss;
   ss << (bias.empty() ? "false" : "true");
