@@ -798,6 +798,7 @@ void takeColumnSums(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, co
   const int64_t waves = n.numTiles * ceilDiv(std::min<int64_t>(static_cast<int64_t>(o.block[0]), n.tile), limits.wavefront);
   if (n.numTiles > allowedBlocks(o, 0, 0) || waves >= limits.computeUnits || r.extent < 4 * kColumnSumWaves || r.extent * n.extent >= (int64_t(1) << 29)) return;
   if (limits.maxThreadsPerBlock < 64 * kColumnSumWaves) return;
+  if (o.hasMaxSharedMemory && static_cast<int64_t>(o.maxSharedMemoryValue) < 4 * 64 * kColumnSumWaves) return;
   std::ostringstream ss;
   ss << r.extent << ", " << n.extent << ", " << kColumnSumWaves << ">(p" << st.tensor << ", p" << load->name;
   st.columnSums = ss.str();

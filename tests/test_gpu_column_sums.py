@@ -39,6 +39,8 @@ def test_column_sums(rows, columns):
     (SOURCE.replace("A(r_r, n) }", "A(r_r, n) * A(r_r, n) }"), 1024, 1024, OPTIONS, False),
     (SOURCE.replace("+=!", "+="), 1024, 1024, OPTIONS, False),
     (SOURCE.replace("+=!", "max=!"), 1024, 1024, OPTIONS, False),
+    (SOURCE, 1024, 1024, OPTIONS + ";maxSharedMemory=4095", False),                 # the partial sums take 4 KiB of LDS
+    (SOURCE, 1024, 1024, OPTIONS + ";maxSharedMemory=4096", True),
     (SOURCE, 1024, 1024, OPTIONS, True),
 ])
 def test_which_sums_are_taken(source, rows, columns, options, taken):
