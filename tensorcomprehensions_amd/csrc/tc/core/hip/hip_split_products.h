@@ -25,6 +25,7 @@ namespace hip {
 constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
 typedef __attribute__((address_space(3))) char ldschar;
+typedef __attribute__((address_space(3))) int ldsint;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) bf16x8 ldsbf16x8;
@@ -40,6 +41,12 @@ struct SplitRange {
 __device__ __forceinline__ bool isUnfitSum(float x) {
   const unsigned magnitude = 2 * __builtin_bit_cast(unsigned, x); // from 2^-60 on, finite, or zero
   return magnitude - 2u * (67u << 23) >= 2u * ((255u - 67u) << 23) && magnitude != 0;
+}
+// Whether any thread of the block says so.  The flag is zero at the barrier before.  (__syncthreads_or has 256 bytes of LDS of its own.)
+__device__ __forceinline__ bool isAnyOfBlock(bool is, ldsint* flag) {
+  if (is) *flag = 1;
+  __syncthreads();
+  return *flag != 0;
 }
 __device__ __forceinline__ SplitParts splitFloats(const float (&v)[8], SplitRange& range) {
   typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -97,6 +104,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
   static constexpr int kItemsI = kPixels * kOctets, kTurnsI = (kItemsI + kThreads - 1) / kThreads;
   static constexpr int kItemsW = kFiltersOfBlock * kSlots, kTurnsW = (kItemsW + kThreads - 1) / kThreads;
   static constexpr int kChunks = (C + CC - 1) / CC;
+  static constexpr int kFlag = 3 * (kPartI + kPartW); // 16 bytes behind the parts
   static constexpr int FT = FB / WF, PW = PT / WP; // tiles of a wavefront
 
   static __device__ __forceinline__ void run(float* pO, const float* pI, const float* pW, const float* pB, ldschar* lds) {
@@ -150,6 +158,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       for (int q = 0; q < 3; ++q) *(ldsbf16x8*)(to + q * part) = s.part[q];
     };
     load(0);
+    if (tid == 0) *(ldsint*)(lds + kFlag) = 0;
     if constexpr (kSlots % 4 != 0) { // the weights of slots that do not exist; the input is read at some other place there
       constexpr int kMissing = 4 * kSteps - kSlots;
       for (int i = tid; i < 3 * kFiltersOfBlock * kMissing; i += kThreads) {
@@ -215,7 +224,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
       }
-    if (__syncthreads_or(again)) { // (what the parts cannot hold: rare, and slow)
+    if (isAnyOfBlock(again, (ldsint*)(lds + kFlag))) { // (what the parts cannot hold: rare, and slow)
 #pragma unroll 1
       for (int i = tid; i < kFiltersOfBlock * kPixelsOfBlock; i += kThreads) {
         const int filter = f0 + i / kPixelsOfBlock, p = p0 + i % kPixelsOfBlock;
@@ -398,6 +407,8 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
             sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[x].part[splitPartB(q)], pa[y].part[splitPartA(q)], sum, 0, 0, 0);
           }
     }
+    ldsint* const flag = (ldsint*)lds + 16 * TB; // (behind the first row of the first tile, where no sum is)
+    if (lane + wave == 0) *flag = 0;
     // A lane holds columns 4 g ... 4 g + 3 of its tiles, in whatever order the tiles hold the positions: four neighbouring ones in LDS.
     ldsfloat* mine = (ldsfloat*)lds + wave * kTile;
 #pragma unroll
@@ -434,7 +445,7 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
 #pragma unroll
       for (int e = 0; e < 4; ++e) again |= isUnfitSum(sum[i][e]);
     }
-    if (__syncthreads_or(again)) { // (what the parts cannot hold: rare, and slow)
+    if (isAnyOfBlock(again, flag)) { // (what the parts cannot hold: rare, and slow)
       constexpr int kOutputs = 16 * TA * 16 * TB / S;
 #pragma unroll 1
       for (int i = slice * kOutputs + lane; i < (slice + 1) * kOutputs; i += 64) {

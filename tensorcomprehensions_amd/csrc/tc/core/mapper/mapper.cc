@@ -497,7 +497,7 @@ SplitConvolutionShape bestSplitConvolution(const ConvolutionSizes& s, int64_t wa
             SplitConvolutionShape c;
             c.pixelTiles = pt * pixelWaves;
             const int64_t pixels = (std::min(rows, (16 * c.pixelTiles + columns - 2) / columns + 1) + s.kernelHeight - 1) * s.width;
-            c.lds = 3 * 16 * (pixels * (octets | 1) + 16 * filterTiles * ((4 * steps) | 1));
+            c.lds = 3 * 16 * (pixels * (octets | 1) + 16 * filterTiles * ((4 * steps) | 1)) + 16; // (a flag)
             if (c.lds > ldsBudget) continue;
             const int64_t items = ceilDiv(pixels * octets, 64 * used) + ceilDiv(16 * filterTiles * slots, 64 * used);
             const int64_t registers = 10 * items + 8 * ft * pt + 16 * (ft + pt) + steps + pt + 30;

@@ -1,5 +1,9 @@
 """Convolutions on the bf16 matrix instruction, each float in three parts (__tc::SplitConvolution): against the same sums in
 64 bits at the edges of pixel tiles, filter tiles, channel chunks and windows, and for values the parts cannot hold."""
+import os
+import re
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -7,6 +11,7 @@ import torch
 import tensorcomprehensions_amd as tc
 from tensorcomprehensions_amd import ShapeOnly
 
+HIPCC = "/opt/rocm/bin/hipcc"
 DENSE = """
 def f(float(N, C, H, W) I, float(M, C, KH, KW) W1, float(M) B) -> (O) {
     O(n, m, h, w) +=! I(n, r_c, h + r_kh, w + r_kw) * W1(m, r_c, r_kh, r_kw)
@@ -143,3 +148,29 @@ def test_which_convolutions_are_taken(sizes, taken):
     ins = operands(sizes, lambda *s: ShapeOnly(s))
     text, _ = tc.map_only(DENSE if sizes[1] == 1 else GROUPS, "f", ins, options(sizes[6], sizes))
     assert ("__tc::SplitConvolution<" in text.split('extern "C"')[-1]) == taken
+
+
+@pytest.mark.parametrize("sizes", [(16, 1, 79, 117, 23, 41, (3, 3)), (23, 1, 126, 64, 83, 19, (3, 3)), (9, 16, 54, 50, 64, 10, (3, 3)), (8, 1, 120, 73, 61, 35, (3, 3))],
+                         ids=lambda s: "x".join(map(str, s[:6])))
+def test_all_of_the_shared_memory(sizes):
+    """Blocks whose parts take all but 16 to 256 bytes of a compute unit's LDS: what else the kernel declares has to fit there too."""
+    source, ins = DENSE if sizes[1] == 1 else GROUPS, operands(sizes, lambda *s: ShapeOnly(s))
+    assert tc.compile(source, "f", ins, options(sizes[6], sizes)).lds_bytes() <= 160 * 1024
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
+@pytest.mark.parametrize("kernel", ["convolution", "product"])
+def test_no_other_shared_memory_than_the_options_see(tmp_path, kernel):
+    if kernel == "convolution":
+        sizes = SIZES[0]
+        source, ins, opts = DENSE, operands(sizes, lambda *s: ShapeOnly(s)), options(sizes[6], sizes)
+    else:
+        source, ins = "def f(float(M, K) A, float(K, N) B) -> (O) { O(m, n) +=! A(m, r_k) * B(r_k, n) }", [ShapeOnly((1000, 1000))] * 2
+        opts = "naive;tile=64,64,32;mapToThreads=64,8;mapToBlocks=256,256;useMfma=1;useSharedMemory=1;prefetchShared=1"
+    text, _ = tc.map_only(source, "f", ins, opts)
+    declared = int(re.search(r"char (?:window|sums)_\[(\d+)\]", text).group(1))
+    path, assembly = tmp_path / "f.hip", tmp_path / "f.s"
+    path.write_text(text)
+    subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "--offload-device-only", "-O3", "-std=c++17", "-Xclang", "-target-feature",
+                    "-Xclang", "-packed-fp32-ops", "-include", "hip/hip_runtime.h", "-w", "-S", "-o", str(assembly), str(path)], check=True)
+    assert int(re.search(r"amdhsa_group_segment_fixed_size (\d+)", assembly.read_text()).group(1)) == declared
