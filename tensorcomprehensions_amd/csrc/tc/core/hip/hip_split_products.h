@@ -16,11 +16,11 @@ namespace hip {
 // What the parts cannot hold is computed again with float arithmetic, block by block:
 //  - infinities, and values that round to one (a middle part of infinity minus infinity), and sums that overflow: seen by a
 //    result that is not finite;
-//  - small values.  A bf16 has the exponents of a float, denormal ones included, so what is left out of a value is below 2^-134.  Where no value
-//    is above 2^32, sums of up to 65536 terms lose less than 2^-86 by that, nothing beside the rounding of a sum from 2^-60 on.  Blocks
-//    with a smaller sum, other than zero, or a larger value go the other way, and so do those with a lane that sees something of an
-//    operand, but nothing from 2^-100 on.  (A sum of zero is taken: it may be one of denormal values below 2^-134 alone, beside other
-//    rows in the block.)
+//  - small values.  A bf16 has the exponents of a float, denormal ones included, so the parts are exact from 2^-110 on, and below it
+//    less than 2^-134 is left out of a value.  Where no value is above 2^32, sums of up to 65536 terms lose less than 2^-85 by that, nothing
+//    beside the rounding of a sum from 2^-60 on.  A block with a larger value or a smaller sum, zero among them (it may be one of small values
+//    alone, whatever stands beside them), looks its operands over: with a value other than zero below 2^-110 it goes the other way,
+//    and with sums other than zero below 2^-100, which the products of parts that are below 2^-149 could be missed in.
 // The check costs half an instruction a value; one for every value's own exponent cost 1.5, and 1000^3 20.7 us for 17.4.
 constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
@@ -35,13 +35,21 @@ struct SplitRange {
   float most = 0.0f;
   // (one instruction; fmaxf would quiet NaNs first)
   __device__ __forceinline__ void see(float a, float b) { asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(a), "v"(b)); }
-  __device__ __forceinline__ bool isUnfit() const { return most > 0x1p32f || (most < 0x1p-100f && most > 0.0f); }
+  __device__ __forceinline__ bool isDoubtful() const { return most > 0x1p32f; }
 };
 // (by the bits: fast math takes every float for finite)
-__device__ __forceinline__ bool isUnfitSum(float x) {
-  const unsigned magnitude = 2 * __builtin_bit_cast(unsigned, x); // from 2^-60 on, finite, or zero
-  return magnitude - 2u * (67u << 23) >= 2u * ((255u - 67u) << 23) && magnitude != 0;
+__device__ __forceinline__ unsigned magnitudeBits(float x) { return 2 * __builtin_bit_cast(unsigned, x); }
+__device__ __forceinline__ constexpr unsigned magnitudeBitsOfPower(int exponent) { return 2u * ((unsigned)(127 + exponent) << 23); }
+// a sum that is zero, below 2^-60 or not finite
+__device__ __forceinline__ bool isDoubtfulSum(float x) {
+  return magnitudeBits(x) - magnitudeBitsOfPower(-60) >= magnitudeBitsOfPower(128) - magnitudeBitsOfPower(-60);
 }
+// one that is not finite, or below 2^-100 but not zero
+__device__ __forceinline__ bool isUnfitSum(float x) {
+  return magnitudeBits(x) - magnitudeBitsOfPower(-100) >= magnitudeBitsOfPower(128) - magnitudeBitsOfPower(-100) && magnitudeBits(x) != 0;
+}
+// a value below 2^-110 but not zero
+__device__ __forceinline__ bool isUnfitValue(float x) { return magnitudeBits(x) - 1 < magnitudeBitsOfPower(-110) - 1; }
 // Whether any thread of the block says so.  The flag is zero at the barrier before.  (__syncthreads_or has 256 bytes of LDS of its own.)
 __device__ __forceinline__ bool isAnyOfBlock(bool is, ldsint* flag) {
   if (is) *flag = 1;
@@ -158,7 +166,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       for (int q = 0; q < 3; ++q) *(ldsbf16x8*)(to + q * part) = s.part[q];
     };
     load(0);
-    if (tid == 0) *(ldsint*)(lds + kFlag) = 0;
+    if (tid < 2) ((ldsint*)(lds + kFlag))[tid] = 0;
     if constexpr (kSlots % 4 != 0) { // the weights of slots that do not exist; the input is read at some other place there
       constexpr int kMissing = 4 * kSteps - kSlots;
       for (int i = tid; i < 3 * kFiltersOfBlock * kMissing; i += kThreads) {
@@ -215,16 +223,38 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       }
       __syncthreads();
     }
-    bool again = rangeI.isUnfit() || rangeW.isUnfit();
+    bool doubtful = rangeI.isDoubtful() || rangeW.isDoubtful();
 #pragma unroll
     for (int t = 0; t < PW; ++t)
 #pragma unroll
       for (int f = 0; f < FT; ++f) {
         large[t][f] += small[t][f];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
+        for (int e = 0; e < 4; ++e) doubtful |= isDoubtfulSum(large[t][f][e]);
       }
-    if (isAnyOfBlock(again, (ldsint*)(lds + kFlag))) { // (what the parts cannot hold: rare, and slow)
+    ldsint* const flags = (ldsint*)(lds + kFlag);
+    bool again = false;
+    if (isAnyOfBlock(doubtful, flags)) {
+#pragma unroll
+      for (int t = 0; t < PW; ++t)
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
+#pragma unroll 1
+      for (int c = 0; c < kChunks; ++c) { // (channels behind the last one are another filter's: at worst a block too many computes again)
+        load(c * CC);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+          for (int i = 0; i < kTurnsI; ++i) again |= isUnfitValue(rawI[i][e]);
+#pragma unroll
+          for (int i = 0; i < kTurnsW; ++i) again |= isUnfitValue(rawW[i][e]);
+        }
+      }
+      again = isAnyOfBlock(again, flags + 1);
+    }
+    if (again) { // (what the parts cannot hold: rare, and slow)
 #pragma unroll 1
       for (int i = tid; i < kFiltersOfBlock * kPixelsOfBlock; i += kThreads) {
         const int filter = f0 + i / kPixelsOfBlock, p = p0 + i % kPixelsOfBlock;
@@ -352,6 +382,14 @@ template <bool KInner, int P, int K, int TP> struct SlicedOperand {
       }
     }
   }
+  __device__ __forceinline__ bool isUnfit() const {
+    bool is = false;
+#pragma unroll
+    for (int y = 0; y < TP; ++y)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) is |= isUnfitValue(value[y][j]);
+    return is;
+  }
 };
 
 template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, int TB, int GA, int GB, int S> struct SlicedProduct {
@@ -407,8 +445,8 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
             sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[x].part[splitPartB(q)], pa[y].part[splitPartA(q)], sum, 0, 0, 0);
           }
     }
-    ldsint* const flag = (ldsint*)lds + 16 * TB; // (behind the first row of the first tile, where no sum is)
-    if (lane + wave == 0) *flag = 0;
+    ldsint* const flags = (ldsint*)lds + 16 * TB; // (behind the first row of the first tile, where no sum is)
+    if (wave == 0 && lane < 2) flags[lane] = 0;
     // A lane holds columns 4 g ... 4 g + 3 of its tiles, in whatever order the tiles hold the positions: four neighbouring ones in LDS.
     ldsfloat* mine = (ldsfloat*)lds + wave * kTile;
 #pragma unroll
@@ -434,7 +472,7 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
     constexpr int kVectors = 4 * TB, kUnits = 16 * TA * kVectors / 64, kShare = (kUnits + S - 1) / S; // 16-byte vectors of a row, 64 of them, of a slice
     const ldsfloat* from = (const ldsfloat*)lds + (wave - slice) * kTile;
     floatx4 sum[kShare];
-    bool again = rangeA.isUnfit() || rangeB.isUnfit();
+    bool doubtful = rangeA.isDoubtful() || rangeB.isDoubtful(), again = false;
 #pragma unroll
     for (int i = 0; i < kShare; ++i) {
       const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
@@ -443,9 +481,23 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
 #pragma unroll
       for (int s = 1; s < S; ++s) sum[i] += *(const ldsfloatx4*)(at + s * kTile);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) again |= isUnfitSum(sum[i][e]);
+      for (int e = 0; e < 4; ++e) doubtful |= isDoubtfulSum(sum[i][e]);
     }
-    if (isAnyOfBlock(again, flag)) { // (what the parts cannot hold: rare, and slow)
+    if (isAnyOfBlock(doubtful, flags)) {
+#pragma unroll
+      for (int i = 0; i < kShare; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) again |= isUnfitSum(sum[i][e]);
+#pragma unroll 1
+      for (int t = 0; t < kTurns; ++t) {
+        const int k0 = 32 * (slice + t * S);
+        a.load(k0);
+        b.load(k0);
+        again |= a.isUnfit() || b.isUnfit(); // (what lies behind the end of a row is of the next one: at worst a block too many computes again)
+      }
+      again = isAnyOfBlock(again, flags + 1);
+    }
+    if (again) { // (what the parts cannot hold: rare, and slow)
       constexpr int kOutputs = 16 * TA * 16 * TB / S;
 #pragma unroll 1
       for (int i = slice * kOutputs + lane; i < (slice + 1) * kOutputs; i += 64) {

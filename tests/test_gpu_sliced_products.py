@@ -119,3 +119,36 @@ def test_which_products_are_taken(m, n, k, a_inner, b_inner, taken):
     shapes = [(m, k) if a_inner else (k, m), (n, k) if b_inner else (k, n)]
     text, _ = tc.map_only(source(a_inner, b_inner), "f", [ShapeOnly(s) for s in shapes], options(m, n))
     assert ("__tc::SlicedProduct<" in text.split('extern "C"')[-1]) == taken
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tiles", [(1000, 1000, 1000, "4, 4, 1, 1, 8"), (254, 292, 1500, "1, 2, 1, 1, 8")])
+@pytest.mark.parametrize("case", ["denormal rows", "denormal columns", "denormal terms", "denormal rows, small sums", "zero rows", "large, zero rows"])
+def test_small_values_beside_others(m, n, k, tiles, case):
+    """Values below what the parts hold, beside ordinary ones and times large ones, where a lane sees several rows."""
+    generator = torch.Generator().manual_seed(3)
+    a, b = torch.randn(m, k, generator=generator), torch.randn(n, k, generator=generator)
+    if case == "denormal rows":
+        a[::7] *= 2.0 ** -140
+        b *= 2.0 ** 28
+    elif case == "denormal columns":
+        b[::5] *= 2.0 ** -139
+        a *= 2.0 ** 29
+    elif case == "denormal terms":                # ordinary values meet zeros: the sum is one of the others
+        a[3, 1::2] *= 2.0 ** -140
+        b[17, ::2] = 0
+        b[17] *= 2.0 ** 30
+    elif case == "denormal rows, small sums":
+        a[::7] *= 2.0 ** -137
+        b *= 2.0 ** -5
+    elif case == "zero rows":
+        a[::3] = 0
+    else:
+        a[::3] = 0
+        a[1] *= 2.0 ** 60
+    text, _ = tc.map_only(source(True, False), "f", [ShapeOnly((m, k)), ShapeOnly((k, n))], options(m, n))
+    assert f"{m}, {n}, {k}, {tiles}>" in text
+    got = run(m, n, k, True, False, a, b).double()
+    want, magnitudes = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    # (a denormal sum is a whole number of 2^-149)
+    assert ((got - want).abs() <= (k + 2) * (2.0 ** -24 * magnitudes + 2.0 ** -149)).all()

@@ -141,6 +141,37 @@ def test_values_the_parts_cannot_hold(case):
         assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["denormal image", "denormal rows", "denormal filters", "denormal terms", "zero image"])
+def test_small_values_beside_others(case):
+    """Values below what the parts hold, beside ordinary ones and times large ones."""
+    sizes = next(s for s in SIZES if s[:3] == (2, 8, 15))
+    generator = torch.Generator().manual_seed(3)
+    x, weights, bias = operands(sizes, lambda *s: torch.randn(s, generator=generator))
+    bias[:] = 0
+    if case == "denormal image":
+        x[0] *= 2.0 ** -140
+        weights *= 2.0 ** 29
+    elif case == "denormal rows":
+        x[:, :, :, 3:9] *= 2.0 ** -140
+        weights *= 2.0 ** 29
+    elif case == "denormal filters":
+        weights[:, 1] *= 2.0 ** -139
+        x *= 2.0 ** 28
+    elif case == "denormal terms":                # ordinary weights meet zeros: the sum is one of the others
+        weights[:, :, :5] *= 2.0 ** -140
+        x[:, :, 5:] = 0
+        x *= 2.0 ** 28
+    else:
+        x[1] = 0
+    got = run(GROUPS, sizes, [x, weights, bias]).double()
+    want, magnitudes = reference(sizes, [x, weights, bias])
+    got = got.reshape(want.shape)
+    terms = sizes[2] * 9
+    # (a denormal sum is a whole number of 2^-149)
+    assert ((got - want).abs() <= (terms + 2) * (2.0 ** -24 * magnitudes + 2.0 ** -149)).all()
+
+
 # (in 80 drawn dense convolutions taken with less of a margin these took up to 1.3 times as long as in the general pipeline)
 @pytest.mark.parametrize("sizes,taken", [((27, 1, 8, 28, 46, 59, (3, 3)), False), ((30, 1, 10, 73, 39, 47, (3, 3)), False), ((12, 1, 60, 60, 43, 22, (1, 1)), False),
                                          ((16, 1, 96, 110, 35, 9, (3, 3)), False), ((16, 1, 64, 64, 57, 57, (3, 3)), True), ((2, 8, 15, 4, 25, 28, (3, 3)), True)])
