@@ -241,16 +241,21 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
         for (int f = 0; f < FT; ++f)
 #pragma unroll
           for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
+      // (in loops of their own: with the staging's offsets kept for them the kernel took up to 60 registers more)
+      constexpr int kFlight = 16, kValuesI = C * kPixels;
+      const int valuesW = tmin(kFiltersOfBlock, F - f0) * (C * kPlaces);
 #pragma unroll 1
-      for (int c = 0; c < kChunks; ++c) { // (channels behind the last one are another filter's: at worst a block too many computes again)
-        load(c * CC);
+      for (int i0 = tid; i0 < kValuesI; i0 += kFlight * kThreads) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-#pragma unroll
-          for (int i = 0; i < kTurnsI; ++i) again |= isUnfitValue(rawI[i][e]);
-#pragma unroll
-          for (int i = 0; i < kTurnsW; ++i) again |= isUnfitValue(rawW[i][e]);
+        for (int j = 0; j < kFlight; ++j) {
+          const int i = tmin(i0 + j * kThreads, kValuesI - 1);
+          again |= isUnfitValue(image[i / kPixels * (H * W) + row0 * W + i % kPixels]);
         }
+      }
+#pragma unroll 1
+      for (int i0 = tid; i0 < valuesW; i0 += kFlight * kThreads) {
+#pragma unroll
+        for (int j = 0; j < kFlight; ++j) again |= isUnfitValue(weights[f0 * (C * kPlaces) + tmin(i0 + j * kThreads, valuesW - 1)]);
       }
       again = isAnyOfBlock(again, flags + 1);
     }
