@@ -13,7 +13,8 @@ namespace hip {
 // products have an accumulator of their own, whose roundings are those of a sum 2^-8 as large.  Error against 64 bits, normal
 // deviates, 2-norm: 96, 992 and 4096 terms 0.6e-7, 1.8e-7, 3.9e-7 (float instruction 1.8e-7, 5.6e-7, 11.5e-7).
 //
-// What the parts cannot hold is computed again with float arithmetic, block by block:
+// What the parts cannot hold is computed again on the float instruction, block by block, from the same tiles (one infinity: 1000^3 16.5 -> 39.2 us,
+// the convolution below 30.3 -> 61.9):
 //  - infinities, and values that round to one (a middle part of infinity minus infinity), and sums that overflow: seen by a
 //    result that is not finite;
 //  - small values.  A bf16 has the exponents of a float, denormal ones included, so the parts are exact from 2^-110 on, and below it
@@ -26,6 +27,8 @@ constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
 typedef __attribute__((address_space(3))) char ldschar;
 typedef __attribute__((address_space(3))) int ldsint;
+typedef __attribute__((address_space(3))) float ldsfloat;
+typedef __attribute__((address_space(3))) floatx4 ldsfloatx4;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) bf16x8 ldsbf16x8;
@@ -115,17 +118,27 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
   static constexpr int kFlag = 3 * (kPartI + kPartW); // 16 bytes behind the parts
   static constexpr int FT = FB / WF, PW = PT / WP; // tiles of a wavefront
 
-  static __device__ __forceinline__ void run(float* pO, const float* pI, const float* pW, const float* pB, ldschar* lds) {
-    const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y), tid = lane + 64 * wave;
-    int block = blockIdx.x;
-    const int band = block % kBands;
-    block /= kBands;
-    const int f0 = block % kFilterBlocks * kFiltersOfBlock;
-    block /= kFilterBlocks;
-    const int group = block % G, n = block / G;
-    const int p0 = band * kPixelsOfBlock, row0 = tmin(p0 / OW, H - kRows);
-    const float* const image = pI + (n * G + group) * (C * H * W);
-    const float* const weights = pW + group * (F * C * kPlaces);
+  // Where a block and a thread are.
+  struct Place {
+    int tid, lane, wave, f0, group, n, p0, row0;
+    const float *image, *weights;
+    __device__ __forceinline__ Place(const float* pI, const float* pW, int t) : tid(t), lane(t & 63), wave(__builtin_amdgcn_readfirstlane(t >> 6)) {
+      int block = blockIdx.x;
+      const int band = block % kBands;
+      block /= kBands;
+      f0 = block % kFilterBlocks * kFiltersOfBlock;
+      block /= kFilterBlocks;
+      group = block % G, n = block / G;
+      p0 = band * kPixelsOfBlock, row0 = tmin(p0 / OW, H - kRows);
+      image = pI + (n * G + group) * (C * H * W);
+      weights = pW + group * (F * C * kPlaces);
+    }
+  };
+
+  // The sums of a lane, of the parts of the floats or of the floats themselves (two planes of four channels instead of three).
+  template <bool InParts> static __device__ __forceinline__ void multiply(const Place& at, ldschar* lds, floatx4 (&large)[PW][FT], SplitRange& rangeI, SplitRange& rangeW) {
+    const int tid = at.tid, lane = at.lane, wave = at.wave, f0 = at.f0, p0 = at.p0, row0 = at.row0;
+    const float *const image = at.image, *const weights = at.weights;
     ldschar *li = lds, *lw = lds + 3 * kPartI;
     // What a thread stages: eight channels of a pixel, or of a place of a filter (threads without an item repeat the last one).
     int fromI[kTurnsI], toI[kTurnsI], fromW[kTurnsW], toW[kTurnsW];
@@ -155,19 +168,23 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 #pragma unroll
         for (int e = 0; e < 8; ++e) rawW[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsW, fromW[i] + e * kPlaces * 4, 0, 0));
     };
-    SplitRange rangeI, rangeW;
     auto lay = [&](float (&v)[8], int firstChannel, ldschar* to, int part, SplitRange& range) __attribute__((always_inline)) {
       if constexpr (C % CC != 0) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = firstChannel + e < C ? v[e] : 0.0f;
       }
-      const SplitParts s = splitFloats(v, range);
+      if constexpr (InParts) {
+        const SplitParts s = splitFloats(v, range);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) *(ldsbf16x8*)(to + q * part) = s.part[q];
+        for (int q = 0; q < 3; ++q) *(ldsbf16x8*)(to + q * part) = s.part[q];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) *(ldsfloatx4*)(to + q * part) = floatx4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+      }
     };
     load(0);
-    if (tid < 2) ((ldsint*)(lds + kFlag))[tid] = 0;
-    if constexpr (kSlots % 4 != 0) { // the weights of slots that do not exist; the input is read at some other place there
+    if (InParts && tid < 2) ((ldsint*)(lds + kFlag))[tid] = 0;
+    if constexpr (InParts && kSlots % 4 != 0) { // the weights of slots that do not exist; the input is read at some other place there
       constexpr int kMissing = 4 * kSteps - kSlots;
       for (int i = tid; i < 3 * kFiltersOfBlock * kMissing; i += kThreads) {
         *(ldsbf16x8*)(lw + i / kMissing * kPitchW + 16 * (kSlots + i % kMissing)) = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
@@ -187,7 +204,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       slotI[j] = (place / KW * W + place % KW) * kPitchI + 16 * (slot % kOctets);
     }
     const int atW = (16 * wf * FT + r) * kPitchW + 16 * g;
-    floatx4 large[PW][FT], small[PW][FT];
+    floatx4 small[PW][FT];
 #pragma unroll
     for (int t = 0; t < PW; ++t)
 #pragma unroll
@@ -202,36 +219,70 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       load(tmin(c + 1, kChunks - 1) * CC);
 #pragma unroll
       for (int j = 0; j < kSteps; ++j) {
-        bf16x8 vw[FT][3], vi[PW][3];
+        if constexpr (InParts) {
+          bf16x8 vw[FT][3], vi[PW][3];
 #pragma unroll
-        for (int f = 0; f < FT; ++f)
+          for (int f = 0; f < FT; ++f)
 #pragma unroll
-          for (int q = 0; q < 3; ++q) vw[f][q] = *(const ldsbf16x8*)(lw + atW + f * 16 * kPitchW + 64 * j + q * kPartW);
-#pragma unroll
-        for (int t = 0; t < PW; ++t)
-#pragma unroll
-          for (int q = 0; q < 3; ++q) vi[t][q] = *(const ldsbf16x8*)(li + atI[t] + slotI[j] + q * kPartI);
-#pragma unroll
-        for (int q = 0; q < kSplitProducts; ++q)
+            for (int q = 0; q < 3; ++q) vw[f][q] = *(const ldsbf16x8*)(lw + atW + f * 16 * kPitchW + 64 * j + q * kPartW);
 #pragma unroll
           for (int t = 0; t < PW; ++t)
 #pragma unroll
-            for (int f = 0; f < FT; ++f) {
-              floatx4& sum = q == kSplitProducts - 1 ? large[t][f] : small[t][f];
-              sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vi[t][splitPartA(q)], vw[f][splitPartB(q)], sum, 0, 0, 0);
+            for (int q = 0; q < 3; ++q) vi[t][q] = *(const ldsbf16x8*)(li + atI[t] + slotI[j] + q * kPartI);
+#pragma unroll
+          for (int q = 0; q < kSplitProducts; ++q)
+#pragma unroll
+            for (int t = 0; t < PW; ++t)
+#pragma unroll
+              for (int f = 0; f < FT; ++f) {
+                floatx4& sum = q == kSplitProducts - 1 ? large[t][f] : small[t][f];
+                sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vi[t][splitPartA(q)], vw[f][splitPartB(q)], sum, 0, 0, 0);
+              }
+        } else {
+          floatx4 vw[FT][2], vi[PW][2];
+          const bool isSlot = 4 * j + g < kSlots; // (the weights are zero where there is none, the input need not be finite)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int f = 0; f < FT; ++f) vw[f][q] = *(const ldsfloatx4*)(lw + atW + f * 16 * kPitchW + 64 * j + q * kPartW);
+#pragma unroll
+            for (int t = 0; t < PW; ++t) {
+              vi[t][q] = *(const ldsfloatx4*)(li + atI[t] + slotI[j] + q * kPartI);
+              if (4 * j + 3 >= kSlots) vi[t][q] = isSlot ? vi[t][q] : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
             }
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int t = 0; t < PW; ++t)
+#pragma unroll
+              for (int f = 0; f < FT; ++f) large[t][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(vi[t][e / 4][e % 4], vw[f][e / 4][e % 4], large[t][f], 0, 0, 0);
+        }
       }
       __syncthreads();
     }
+    if constexpr (InParts) {
+#pragma unroll
+      for (int t = 0; t < PW; ++t)
+#pragma unroll
+        for (int f = 0; f < FT; ++f) large[t][f] += small[t][f];
+    }
+  }
+
+  static __device__ __forceinline__ void run(float* pO, const float* pI, const float* pW, const float* pB, ldschar* lds) {
+    int t = threadIdx.x + 64 * threadIdx.y;
+    const Place at(pI, pW, t);
+    floatx4 large[PW][FT];
+    SplitRange rangeI, rangeW;
+    multiply<true>(at, lds, large, rangeI, rangeW);
+    const int tid = at.tid, f0 = at.f0, group = at.group, n = at.n, p0 = at.p0, r = at.lane & 15, g = at.lane >> 4, wf = at.wave % WF, wp = at.wave / WF;
     bool doubtful = rangeI.isDoubtful() || rangeW.isDoubtful();
 #pragma unroll
     for (int t = 0; t < PW; ++t)
 #pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        large[t][f] += small[t][f];
+      for (int f = 0; f < FT; ++f)
 #pragma unroll
         for (int e = 0; e < 4; ++e) doubtful |= isDoubtfulSum(large[t][f][e]);
-      }
     ldsint* const flags = (ldsint*)(lds + kFlag);
     bool again = false;
     if (isAnyOfBlock(doubtful, flags)) {
@@ -249,31 +300,19 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 #pragma unroll
         for (int j = 0; j < kFlight; ++j) {
           const int i = tmin(i0 + j * kThreads, kValuesI - 1);
-          again |= isUnfitValue(image[i / kPixels * (H * W) + row0 * W + i % kPixels]);
+          again |= isUnfitValue(at.image[i / kPixels * (H * W) + at.row0 * W + i % kPixels]);
         }
       }
 #pragma unroll 1
       for (int i0 = tid; i0 < valuesW; i0 += kFlight * kThreads) {
 #pragma unroll
-        for (int j = 0; j < kFlight; ++j) again |= isUnfitValue(weights[f0 * (C * kPlaces) + tmin(i0 + j * kThreads, valuesW - 1)]);
+        for (int j = 0; j < kFlight; ++j) again |= isUnfitValue(at.weights[f0 * (C * kPlaces) + tmin(i0 + j * kThreads, valuesW - 1)]);
       }
       again = isAnyOfBlock(again, flags + 1);
     }
-    if (again) { // (what the parts cannot hold: rare, and slow)
-#pragma unroll 1
-      for (int i = tid; i < kFiltersOfBlock * kPixelsOfBlock; i += kThreads) {
-        const int filter = f0 + i / kPixelsOfBlock, p = p0 + i % kPixelsOfBlock;
-        if (filter >= F || p >= kPlane) continue;
-        float sum = 0.0f;
-#pragma unroll 1
-        for (int k = 0; k < C * kPlaces; ++k) {
-          const int place = k % kPlaces;
-          sum = __builtin_fmaf(image[k / kPlaces * (H * W) + (p / OW + place / KW) * W + p % OW + place % KW], weights[filter * (C * kPlaces) + k], sum);
-        }
-        if constexpr (Bias) sum += pB[group * F + filter];
-        pO[((n * G + group) * F + filter) * kPlane + p] = sum;
-      }
-      return;
+    if (again) {
+      asm("" : "+v"(t)); // (or the offsets of this pass are those of the first one, kept)
+      multiply<false>(Place(pI, pW, t), lds, large, rangeI, rangeW);
     }
     typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
     const __amdgpu_buffer_rsrc_t rsO = __builtin_amdgcn_make_buffer_rsrc((void*)pO, 0, N * G * F * kPlane * 4, 0x00020000);
@@ -323,8 +362,6 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 // matrix cores.  Steps two ahead in registers, parts of the next step made under the multiplications of this one: 18.2 to 25.
 constexpr const char* kDeviceSlicedProduct = R"HIP(
 namespace __tc {
-typedef __attribute__((address_space(3))) float ldsfloat;
-typedef __attribute__((address_space(3))) floatx4 ldsfloatx4;
 template <bool KInner, int P, int K, int TP> struct SlicedOperand {
   static constexpr int kOffsets = KInner ? TP : 8;
   const float* p;
@@ -402,6 +439,98 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
   static constexpr int kRowsOfBlock = 16 * TA * GA, kColumnsOfBlock = 16 * TB * GB;
   static constexpr int kRows = (M + kRowsOfBlock - 1) / kRowsOfBlock, kColumns = (N + kColumnsOfBlock - 1) / kColumnsOfBlock, kBlocks = kRows * kColumns;
   static constexpr int kPitch = 16 * TB + 4, kTile = 16 * TA * kPitch, kLds = 4 * GA * GB * S * kTile; // (floats of a row and a tile of partial sums, bytes of all)
+  static constexpr int kTurns = ((K + 31) / 32 + S - 1) / S;
+  static constexpr int kVectors = 4 * TB, kUnits = 16 * TA * kVectors / 64, kShare = (kUnits + S - 1) / S; // 16-byte vectors of a row, 64 of them, of a slice
+  // The sums of a wavefront's steps: of the parts of the floats, or of the floats themselves.
+  template <bool InParts> static __device__ __forceinline__ void multiply(SlicedOperand<AKInner, M, K, TA>& a, SlicedOperand<BKInner, N, K, TB>& b, int slice,
+                                                                          floatx4 (&sum)[TB][TA], SplitRange& rangeA, SplitRange& rangeB) {
+    // (small products have sums of their own where the registers hold them)
+    constexpr int kSums = InParts && TA * TB < 16 ? 2 : 1;
+    floatx4 sums[kSums][TB][TA];
+#pragma unroll
+    for (int d = 0; d < kSums; ++d)
+#pragma unroll
+      for (int x = 0; x < TB; ++x)
+#pragma unroll
+        for (int y = 0; y < TA; ++y) sums[d][x][y] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    a.load(32 * slice);
+    b.load(32 * slice);
+#pragma unroll 1
+    for (int t = 0; t < kTurns; ++t) {
+      const int k0 = 32 * (slice + t * S);
+      if constexpr (InParts) {
+        SplitParts pa[TA], pb[TB];
+        a.cut(k0);
+#pragma unroll
+        for (int y = 0; y < TA; ++y) pa[y] = splitFloats(a.value[y], rangeA);
+        // (or the scheduler puts the loads in front of the last uses of what they overwrite, and waits for them at the end of the turn)
+        __builtin_amdgcn_sched_barrier(0);
+        a.load(k0 + 32 * S);
+        b.cut(k0);
+#pragma unroll
+        for (int x = 0; x < TB; ++x) pb[x] = splitFloats(b.value[x], rangeB);
+        b.load(k0 + 32 * S);
+#pragma unroll
+        for (int x = 0; x < TB; ++x)
+#pragma unroll
+          for (int q = 0; q < kSplitProducts; ++q)
+#pragma unroll
+            for (int y = 0; y < TA; ++y) {
+              floatx4& sum = sums[q == kSplitProducts - 1 ? 0 : kSums - 1][x][y];
+              sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[x].part[splitPartB(q)], pa[y].part[splitPartA(q)], sum, 0, 0, 0);
+            }
+      } else {
+        a.cut(k0);
+        b.cut(k0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int x = 0; x < TB; ++x)
+#pragma unroll
+            for (int y = 0; y < TA; ++y) sums[0][x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.value[x][j], a.value[y][j], sums[0][x][y], 0, 0, 0);
+        a.load(k0 + 32 * S);
+        b.load(k0 + 32 * S);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < TB; ++x)
+#pragma unroll
+      for (int y = 0; y < TA; ++y) {
+        sum[x][y] = sums[0][x][y];
+        if constexpr (kSums == 2) sum[x][y] += sums[1][x][y];
+      }
+  }
+  // Adds the slices of a rectangle of tiles; a lane gets its share of them, vectors of four neighbouring columns.
+  static __device__ __forceinline__ void meet(const floatx4 (&mine)[TB][TA], const SlicedOperand<AKInner, M, K, TA>& a, int wave, int slice, int lane, ldschar* lds, floatx4 (&sum)[kShare]) {
+    const int r = lane & 15, g = lane >> 4;
+    // A lane holds columns 4 g ... 4 g + 3 of its tiles, in whatever order the tiles hold the positions: four neighbouring ones in LDS.
+    ldsfloat* const tile = (ldsfloat*)lds + wave * kTile;
+#pragma unroll
+    for (int y = 0; y < TA; ++y) {
+      ldsfloat* row = tile + a.position(y, r) * kPitch;
+#pragma unroll
+      for (int x = 0; x < TB; ++x) {
+        if constexpr (BKInner) {
+          *(ldsfloatx4*)(row + 16 * x + 4 * g) = mine[x][y];
+        } else {
+          floatx4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = mine[(4 * x + e) % TB][y][(4 * x + e) / TB];
+          *(ldsfloatx4*)(row + 4 * TB * g + 4 * x) = v;
+        }
+      }
+    }
+    __syncthreads();
+    const ldsfloat* from = (const ldsfloat*)lds + (wave - slice) * kTile;
+#pragma unroll
+    for (int i = 0; i < kShare; ++i) {
+      const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
+      const ldsfloat* at = from + unit / kVectors * kPitch + unit % kVectors * 4;
+      sum[i] = *(const ldsfloatx4*)at;
+#pragma unroll
+      for (int s = 1; s < S; ++s) sum[i] += *(const ldsfloatx4*)(at + s * kTile);
+    }
+  }
   static __device__ __forceinline__ void run(float* pO, const float* pA, const float* pB, const float* pBias, ldschar* lds) {
     const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int r = lane & 15, g = lane >> 4, slice = wave % S, ga = wave / S % GA, gb = wave / S / GA;
@@ -413,81 +542,17 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
     SlicedOperand<BKInner, N, K, TB> b;
     a.init(pA, m0, lane);
     b.init(pB, n0, lane);
-    // (small products have sums of their own where the registers hold them)
-    constexpr int kSums = TA * TB < 16 ? 2 : 1;
-    floatx4 sums[kSums][TB][TA];
-#pragma unroll
-    for (int d = 0; d < kSums; ++d)
-#pragma unroll
-      for (int x = 0; x < TB; ++x)
-#pragma unroll
-        for (int y = 0; y < TA; ++y) sums[d][x][y] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    floatx4 mine[TB][TA], sum[kShare];
     SplitRange rangeA, rangeB;
-    a.load(32 * slice);
-    b.load(32 * slice);
-    constexpr int kTurns = ((K + 31) / 32 + S - 1) / S;
-#pragma unroll 1
-    for (int t = 0; t < kTurns; ++t) {
-      const int k0 = 32 * (slice + t * S);
-      SplitParts pa[TA], pb[TB];
-      a.cut(k0);
-#pragma unroll
-      for (int y = 0; y < TA; ++y) pa[y] = splitFloats(a.value[y], rangeA);
-      // (or the scheduler puts the loads in front of the last uses of what they overwrite, and waits for them at the end of the turn)
-      __builtin_amdgcn_sched_barrier(0);
-      a.load(k0 + 32 * S);
-      b.cut(k0);
-#pragma unroll
-      for (int x = 0; x < TB; ++x) pb[x] = splitFloats(b.value[x], rangeB);
-      b.load(k0 + 32 * S);
-#pragma unroll
-      for (int x = 0; x < TB; ++x)
-#pragma unroll
-        for (int q = 0; q < kSplitProducts; ++q)
-#pragma unroll
-          for (int y = 0; y < TA; ++y) {
-            floatx4& sum = sums[q == kSplitProducts - 1 ? 0 : kSums - 1][x][y];
-            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[x].part[splitPartB(q)], pa[y].part[splitPartA(q)], sum, 0, 0, 0);
-          }
-    }
+    multiply<true>(a, b, slice, mine, rangeA, rangeB);
     ldsint* const flags = (ldsint*)lds + 16 * TB; // (behind the first row of the first tile, where no sum is)
     if (wave == 0 && lane < 2) flags[lane] = 0;
-    // A lane holds columns 4 g ... 4 g + 3 of its tiles, in whatever order the tiles hold the positions: four neighbouring ones in LDS.
-    ldsfloat* mine = (ldsfloat*)lds + wave * kTile;
-#pragma unroll
-    for (int y = 0; y < TA; ++y) {
-#pragma unroll
-      for (int x = 0; x < TB; ++x) {
-        if constexpr (kSums == 2) sums[0][x][y] += sums[1][x][y];
-      }
-      ldsfloat* row = mine + a.position(y, r) * kPitch;
-#pragma unroll
-      for (int x = 0; x < TB; ++x) {
-        if constexpr (BKInner) {
-          *(ldsfloatx4*)(row + 16 * x + 4 * g) = sums[0][x][y];
-        } else {
-          floatx4 v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = sums[0][(4 * x + e) % TB][y][(4 * x + e) / TB];
-          *(ldsfloatx4*)(row + 4 * TB * g + 4 * x) = v;
-        }
-      }
-    }
-    __syncthreads();
-    constexpr int kVectors = 4 * TB, kUnits = 16 * TA * kVectors / 64, kShare = (kUnits + S - 1) / S; // 16-byte vectors of a row, 64 of them, of a slice
-    const ldsfloat* from = (const ldsfloat*)lds + (wave - slice) * kTile;
-    floatx4 sum[kShare];
+    meet(mine, a, wave, slice, lane, lds, sum);
     bool doubtful = rangeA.isDoubtful() || rangeB.isDoubtful(), again = false;
 #pragma unroll
-    for (int i = 0; i < kShare; ++i) {
-      const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
-      const ldsfloat* at = from + unit / kVectors * kPitch + unit % kVectors * 4;
-      sum[i] = *(const ldsfloatx4*)at;
-#pragma unroll
-      for (int s = 1; s < S; ++s) sum[i] += *(const ldsfloatx4*)(at + s * kTile);
+    for (int i = 0; i < kShare; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) doubtful |= isDoubtfulSum(sum[i][e]);
-    }
     if (isAnyOfBlock(doubtful, flags)) {
 #pragma unroll
       for (int i = 0; i < kShare; ++i)
@@ -502,19 +567,9 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
       }
       again = isAnyOfBlock(again, flags + 1);
     }
-    if (again) { // (what the parts cannot hold: rare, and slow)
-      constexpr int kOutputs = 16 * TA * 16 * TB / S;
-#pragma unroll 1
-      for (int i = slice * kOutputs + lane; i < (slice + 1) * kOutputs; i += 64) {
-        const int m = m0 + i / (16 * TB), n = n0 + i % (16 * TB);
-        if (m >= M || n >= N) continue;
-        float v = 0.0f;
-#pragma unroll 1
-        for (int k = 0; k < K; ++k) v = __builtin_fmaf(pA[AKInner ? m * K + k : k * M + m], pB[BKInner ? n * K + k : k * N + n], v);
-        if constexpr (Bias) v += pBias[n];
-        pO[m * N + n] = v;
-      }
-      return;
+    if (again) {
+      multiply<false>(a, b, slice, mine, rangeA, rangeB);
+      meet(mine, a, wave, slice, lane, lds, sum);
     }
     typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)pO, 0, M * N * 4, 0x00020000);

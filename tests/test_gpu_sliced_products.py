@@ -152,3 +152,45 @@ def test_small_values_beside_others(m, n, k, tiles, case):
     want, magnitudes = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     # (a denormal sum is a whole number of 2^-149)
     assert ((got - want).abs() <= (k + 2) * (2.0 ** -24 * magnitudes + 2.0 ** -149)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("a_inner,b_inner,bias", [(True, False, False), (True, True, True), (False, False, False), (False, True, True)])
+@pytest.mark.parametrize("m,n,k", [(1000, 1000, 1000), (254, 292, 1500), (655, 1031, 545), (2062, 1895, 768)])
+def test_sums_of_floats_themselves(m, n, k, a_inner, b_inner, bias):
+    """Blocks that compute again, with every order of the operands: an infinity and a NaN reach their row and column alone, also where the last step
+    has fewer points, and denormal operands keep their sums."""
+    generator = torch.Generator().manual_seed(4)
+    a, b, c = (torch.randn(s, generator=generator) for s in ((m, k), (n, k), (n,)))
+    text, _ = tc.map_only(source(a_inner, b_inner, bias), "f", [ShapeOnly((m, k) if a_inner else (k, m)), ShapeOnly((n, k) if b_inner else (k, n))] +
+                          ([ShapeOnly((n,))] if bias else []), options(m, n))
+    if "__tc::SlicedProduct<" not in text.split('extern "C"')[-1]:
+        pytest.skip("the general pipeline is as fast for this order of the operands")
+    for scale in (1.0, 2.0 ** -125):
+        x, y = a * scale, b.clone()
+        if scale == 1.0:
+            x[0, k - 1], x[m - 1, 0], y[n - 1, k - 1] = np.inf, -np.inf, np.nan
+        got = run(m, n, k, a_inner, b_inner, x, y, c if bias and scale == 1.0 else 0 * c if bias else None).double()
+        x, y = x.double(), y.double()
+        want, magnitudes = x @ y.t(), x.abs() @ y.abs().t()
+        if bias and scale == 1.0:
+            want, magnitudes = want + c, magnitudes + c.abs()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+        finite = torch.isfinite(want)
+        # (a denormal sum is a whole number of 2^-149)
+        assert ((got - want).abs()[finite] <= (k + 2) * (2.0 ** -24 * magnitudes[finite] + 2.0 ** -149)).all()
+
+
+@pytest.mark.gpu
+def test_time_of_sums_of_floats_themselves():
+    """A block that computes again uses the matrix cores too: one infinity makes a product take some 2.4 times as long (without them 50 times)."""
+    m = n = k = 1000
+    a, b = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    executor = tc.compile(source(True, False), "f", [a, b], options(m, n))
+    out = torch.empty(m, n, device="cuda")
+    times = []
+    for value in (1.0, float("inf")):
+        a[5, 7] = value
+        tc.run(executor, [a, b], [out])
+        times.append(min(tc.profile_repeated(executor, [a, b], [out], 20) for _ in range(5)))
+    assert times[1] < 8 * times[0]

@@ -172,6 +172,43 @@ def test_small_values_beside_others(case):
     assert ((got - want).abs() <= (terms + 2) * (2.0 ** -24 * magnitudes + 2.0 ** -149)).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", SIZES, ids=lambda s: "x".join(map(str, s[:6])))
+def test_sums_of_floats_themselves(sizes):
+    """Blocks that compute again: infinities and NaNs at the corners of an image reach the windows they are in and no other, whatever the weights of
+    steps and channels that do not exist, and denormal images keep their sums."""
+    source = DENSE if sizes[1] == 1 else GROUPS
+    generator = torch.Generator().manual_seed(4)
+    x, weights, bias = operands(sizes, lambda *s: torch.randn(s, generator=generator))
+    terms = sizes[2] * sizes[6][0] * sizes[6][1]
+    corners = x.clone()
+    flat = corners.view(sizes[0] * sizes[1], sizes[2], sizes[4], sizes[5])
+    flat[0, 0, 0, 0], flat[0, -1, -1, -1], flat[-1, -1, 0, -1], flat[-1, 0, -1, 0] = np.inf, -np.inf, np.nan, np.inf
+    for ins in ([corners, weights, bias], [x * 2.0 ** -125, weights, 0 * bias]):
+        got = run(source, sizes, ins).double()
+        want, magnitudes = reference(sizes, ins)
+        got = got.reshape(want.shape)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+        finite = torch.isfinite(want)
+        # (a denormal sum is a whole number of 2^-149)
+        assert ((got - want).abs()[finite] <= (terms + 2) * (2.0 ** -24 * magnitudes[finite] + 2.0 ** -149)).all()
+
+
+@pytest.mark.gpu
+def test_time_of_sums_of_floats_themselves():
+    """A block that computes again uses the matrix cores too: one infinity makes a convolution take some 2.1 times as long (without them 62 times)."""
+    sizes = SIZES[0]
+    ins = [t.cuda() for t in operands(sizes, lambda *s: torch.randn(s))]
+    executor = tc.compile(DENSE, "f", ins, options(sizes[6], sizes))
+    outs = tc.prepare_outputs(DENSE, "f", ins)
+    times = []
+    for value in (1.0, float("inf")):
+        ins[0][3, 5, 7, 9] = value
+        tc.run(executor, ins, outs)
+        times.append(min(tc.profile_repeated(executor, ins, outs, 20) for _ in range(5)))
+    assert times[1] < 8 * times[0]
+
+
 # (in 80 drawn dense convolutions taken with less of a margin these took up to 1.3 times as long as in the general pipeline)
 @pytest.mark.parametrize("sizes,taken", [((27, 1, 8, 28, 46, 59, (3, 3)), False), ((30, 1, 10, 73, 39, 47, (3, 3)), False), ((12, 1, 60, 60, 43, 22, (1, 1)), False),
                                          ((16, 1, 96, 110, 35, 9, (3, 3)), False), ((16, 1, 64, 64, 57, 57, (3, 3)), True), ((2, 8, 15, 4, 25, 28, (3, 3)), True)])
