@@ -18,10 +18,13 @@ namespace hip {
 //  - infinities, and values that round to one (a middle part of infinity minus infinity), and sums that overflow: seen by a
 //    result that is not finite;
 //  - small values.  A bf16 has the exponents of a float, denormal ones included, so the parts are exact from 2^-110 on, and below it
-//    less than 2^-134 is left out of a value.  Where no value is above 2^32, sums of up to 65536 terms lose less than 2^-85 by that, nothing
-//    beside the rounding of a sum from 2^-60 on.  A block with a larger value or a smaller sum, zero among them (it may be one of small values
-//    alone, whatever stands beside them), looks its operands over: with a value other than zero below 2^-110 it goes the other way,
-//    and with sums other than zero below 2^-100, which the products of parts that are below 2^-149 could be missed in.
+//    less than 2^-134 is left out of a value: of a sum of up to 65536 terms less than 2^-117 of the largest value that is in it, nothing
+//    beside the rounding of a sum from 2^-92 of that value on, nor of a sum whose values on one side are zeros.  And products of parts
+//    below 2^-149 are nothing beside the rounding of a sum from 2^-100 on.
+//    A lane keeps the largest value it has split.  A block in which all sums are 2^-60 or more and all values 2^32 or less is done.  Another one
+//    looks at its sums beside the largest values of their row and column (of the window and the filters).  A sum that is still too small may be one
+//    of larger terms that cancelled, as the slices of a product and a few of the terms can tell, or of small values alone, whatever stands
+//    beside them: where that is left open the block looks its operands over for values other than zero below 2^-110.
 // The check costs half an instruction a value; one for every value's own exponent cost 1.5, and 1000^3 20.7 us for 17.4.
 constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
@@ -51,8 +54,16 @@ __device__ __forceinline__ bool isDoubtfulSum(float x) {
 __device__ __forceinline__ bool isUnfitSum(float x) {
   return magnitudeBits(x) - magnitudeBitsOfPower(-100) >= magnitudeBitsOfPower(128) - magnitudeBitsOfPower(-100) && magnitudeBits(x) != 0;
 }
+// what small values could have been lost in, beside the largest values on its two sides: a sum, or the largest one of its parts
+__device__ __forceinline__ bool isUnsureSum(float x, float mostA, float mostB) {
+  const float most = __builtin_fmaxf(mostA, mostB);
+  return __builtin_bit_cast(int, mostA) != 0 && __builtin_bit_cast(int, mostB) != 0 && __builtin_fabsf(x) < 0x1p-92f * most;
+}
 // a value below 2^-110 but not zero
 __device__ __forceinline__ bool isUnfitValue(float x) { return magnitudeBits(x) - 1 < magnitudeBitsOfPower(-110) - 1; }
+__device__ __forceinline__ void raiseTo(ldsfloat* most, float x) { // (floats from zero on are in the order of their bits)
+  __hip_atomic_fetch_max((ldsint*)most, __builtin_bit_cast(int, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 // Whether any thread of the block says so.  The flag is zero at the barrier before.  (__syncthreads_or has 256 bytes of LDS of its own.)
 __device__ __forceinline__ bool isAnyOfBlock(bool is, ldsint* flag) {
   if (is) *flag = 1;
@@ -183,7 +194,7 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
       }
     };
     load(0);
-    if (InParts && tid < 2) ((ldsint*)(lds + kFlag))[tid] = 0;
+    if (InParts && tid < 4) ((ldsint*)(lds + kFlag))[tid] = 0;
     if constexpr (InParts && kSlots % 4 != 0) { // the weights of slots that do not exist; the input is read at some other place there
       constexpr int kMissing = 4 * kSteps - kSlots;
       for (int i = tid; i < 3 * kFiltersOfBlock * kMissing; i += kThreads) {
@@ -286,29 +297,60 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
     ldsint* const flags = (ldsint*)(lds + kFlag);
     bool again = false;
     if (isAnyOfBlock(doubtful, flags)) {
+      ldsfloat* const most = (ldsfloat*)lds; // of the window, of the filters
+      if (tid < 2) most[tid] = 0.0f;
+      __syncthreads();
+      float mostI = rangeI.most, mostW = rangeW.most;
+#pragma unroll
+      for (int d = 32; d > 0; d /= 2) { // (64 lanes at one word are 64 turns)
+        mostI = __builtin_fmaxf(mostI, __shfl_xor(mostI, d));
+        mostW = __builtin_fmaxf(mostW, __shfl_xor(mostW, d));
+      }
+      if (at.lane == 0) {
+        raiseTo(most, mostI);
+        raiseTo(most + 1, mostW);
+      }
+      __syncthreads();
+      bool unsure = false;
 #pragma unroll
       for (int t = 0; t < PW; ++t)
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) again |= isUnfitSum(large[t][f][e]);
+          for (int e = 0; e < 4; ++e) {
+            again |= isUnfitSum(large[t][f][e]);
+            unsure |= isUnsureSum(large[t][f][e], most[0], most[1]);
+          }
+      if (unsure) flags[1] = 1;
+      again = isAnyOfBlock(again, flags + 2);
+      doubtful = !again && flags[1] != 0;
+    } else {
+      doubtful = false;
+    }
+    if (doubtful) {
       // (in loops of their own: with the staging's offsets kept for them the kernel took up to 60 registers more)
-      constexpr int kFlight = 16, kValuesI = C * kPixels;
-      const int valuesW = tmin(kFiltersOfBlock, F - f0) * (C * kPlaces);
+      constexpr int kFlight = 16, kTurnsOfWindow = (C * kPixels + kFlight * kThreads - 1) / (kFlight * kThreads);
+      const __amdgpu_buffer_rsrc_t rsI = __builtin_amdgcn_make_buffer_rsrc((void*)(at.image + at.row0 * W), 0, (C * H * W - at.row0 * W) * 4, 0x00020000);
+      int pixel = tid % kPixels;
+      unsigned from = tid / kPixels * (H * W) + pixel;
 #pragma unroll 1
-      for (int i0 = tid; i0 < kValuesI; i0 += kFlight * kThreads) {
+      for (int i = 0; i < kTurnsOfWindow; ++i) {
 #pragma unroll
-        for (int j = 0; j < kFlight; ++j) {
-          const int i = tmin(i0 + j * kThreads, kValuesI - 1);
-          again |= isUnfitValue(at.image[i / kPixels * (H * W) + at.row0 * W + i % kPixels]);
+        for (int j = 0; j < kFlight; ++j) { // (behind the last channel it reads zeros)
+          again |= isUnfitValue(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsI, from * 4, 0, 0)));
+          pixel += kThreads % kPixels;
+          from += kThreads / kPixels * (H * W) + kThreads % kPixels;
+          if (pixel >= kPixels) pixel -= kPixels, from += H * W - kPixels;
         }
       }
+      const int valuesW = tmin(kFiltersOfBlock, F - f0) * (C * kPlaces);
+      const __amdgpu_buffer_rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc((void*)(at.weights + f0 * (C * kPlaces)), 0, valuesW * 4, 0x00020000);
 #pragma unroll 1
-      for (int i0 = tid; i0 < valuesW; i0 += kFlight * kThreads) {
+      for (int i = tid; i < valuesW; i += kFlight * kThreads) {
 #pragma unroll
-        for (int j = 0; j < kFlight; ++j) again |= isUnfitValue(at.weights[f0 * (C * kPlaces) + tmin(i0 + j * kThreads, valuesW - 1)]);
+        for (int j = 0; j < kFlight; ++j) again |= isUnfitValue(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsW, (i + j * kThreads) * 4, 0, 0)));
       }
-      again = isAnyOfBlock(again, flags + 1);
+      again = isAnyOfBlock(again, flags + 3);
     }
     if (again) {
       asm("" : "+v"(t)); // (or the offsets of this pass are those of the first one, kept)
@@ -434,16 +476,23 @@ template <bool KInner, int P, int K, int TP> struct SlicedOperand {
   }
 };
 
+// Outputs whose sums are in doubt: how many, and the first ones.
+constexpr int kMostNoted = 256, kSampledTerms = 16;
+__device__ __forceinline__ void note(ldsint* noted, int output) {
+  const int at = __hip_atomic_fetch_add(noted, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (at < kMostNoted) noted[1 + at] = output;
+}
 template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, int TB, int GA, int GB, int S> struct SlicedProduct {
   static_assert((AKInner || TA == 1 || TA == 2 || TA == 4) && (TB == 1 || TB == 2 || TB == 4), "positions a lane loads at once");
   static constexpr int kRowsOfBlock = 16 * TA * GA, kColumnsOfBlock = 16 * TB * GB;
   static constexpr int kRows = (M + kRowsOfBlock - 1) / kRowsOfBlock, kColumns = (N + kColumnsOfBlock - 1) / kColumnsOfBlock, kBlocks = kRows * kColumns;
   static constexpr int kPitch = 16 * TB + 4, kTile = 16 * TA * kPitch, kLds = 4 * GA * GB * S * kTile; // (floats of a row and a tile of partial sums, bytes of all)
+  static_assert(kLds >= 4 * (128 + kRowsOfBlock + kColumnsOfBlock + 1 + kMostNoted), "what doubts are looked into with");
   static constexpr int kTurns = ((K + 31) / 32 + S - 1) / S;
   static constexpr int kVectors = 4 * TB, kUnits = 16 * TA * kVectors / 64, kShare = (kUnits + S - 1) / S; // 16-byte vectors of a row, 64 of them, of a slice
   // The sums of a wavefront's steps: of the parts of the floats, or of the floats themselves.
   template <bool InParts> static __device__ __forceinline__ void multiply(SlicedOperand<AKInner, M, K, TA>& a, SlicedOperand<BKInner, N, K, TB>& b, int slice,
-                                                                          floatx4 (&sum)[TB][TA], SplitRange& rangeA, SplitRange& rangeB) {
+                                                                          floatx4 (&sum)[TB][TA], SplitRange (&rangeA)[TA], SplitRange (&rangeB)[TB]) {
     // (small products have sums of their own where the registers hold them)
     constexpr int kSums = InParts && TA * TB < 16 ? 2 : 1;
     floatx4 sums[kSums][TB][TA];
@@ -462,13 +511,13 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
         SplitParts pa[TA], pb[TB];
         a.cut(k0);
 #pragma unroll
-        for (int y = 0; y < TA; ++y) pa[y] = splitFloats(a.value[y], rangeA);
+        for (int y = 0; y < TA; ++y) pa[y] = splitFloats(a.value[y], rangeA[y]);
         // (or the scheduler puts the loads in front of the last uses of what they overwrite, and waits for them at the end of the turn)
         __builtin_amdgcn_sched_barrier(0);
         a.load(k0 + 32 * S);
         b.cut(k0);
 #pragma unroll
-        for (int x = 0; x < TB; ++x) pb[x] = splitFloats(b.value[x], rangeB);
+        for (int x = 0; x < TB; ++x) pb[x] = splitFloats(b.value[x], rangeB[x]);
         b.load(k0 + 32 * S);
 #pragma unroll
         for (int x = 0; x < TB; ++x)
@@ -500,6 +549,11 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
         if constexpr (kSums == 2) sum[x][y] += sums[1][x][y];
       }
   }
+  // Where the i-th vector of a lane's share is in a tile.
+  static __device__ __forceinline__ int place(int slice, int i, int lane) {
+    const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
+    return unit / kVectors * kPitch + unit % kVectors * 4;
+  }
   // Adds the slices of a rectangle of tiles; a lane gets its share of them, vectors of four neighbouring columns.
   static __device__ __forceinline__ void meet(const floatx4 (&mine)[TB][TA], const SlicedOperand<AKInner, M, K, TA>& a, int wave, int slice, int lane, ldschar* lds, floatx4 (&sum)[kShare]) {
     const int r = lane & 15, g = lane >> 4;
@@ -524,8 +578,7 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
     const ldsfloat* from = (const ldsfloat*)lds + (wave - slice) * kTile;
 #pragma unroll
     for (int i = 0; i < kShare; ++i) {
-      const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
-      const ldsfloat* at = from + unit / kVectors * kPitch + unit % kVectors * 4;
+      const ldsfloat* at = from + place(slice, i, lane);
       sum[i] = *(const ldsfloatx4*)at;
 #pragma unroll
       for (int s = 1; s < S; ++s) sum[i] += *(const ldsfloatx4*)(at + s * kTile);
@@ -543,21 +596,73 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
     a.init(pA, m0, lane);
     b.init(pB, n0, lane);
     floatx4 mine[TB][TA], sum[kShare];
-    SplitRange rangeA, rangeB;
+    SplitRange rangeA[TA], rangeB[TB];
     multiply<true>(a, b, slice, mine, rangeA, rangeB);
     ldsint* const flags = (ldsint*)lds + 16 * TB; // (behind the first row of the first tile, where no sum is)
-    if (wave == 0 && lane < 2) flags[lane] = 0;
+    if (wave == 0 && lane < 4) flags[lane] = 0;
     meet(mine, a, wave, slice, lane, lds, sum);
-    bool doubtful = rangeA.isDoubtful() || rangeB.isDoubtful(), again = false;
+    bool doubtful = false, again = false;
+#pragma unroll
+    for (int y = 0; y < TA; ++y) doubtful |= rangeA[y].isDoubtful();
+#pragma unroll
+    for (int x = 0; x < TB; ++x) doubtful |= rangeB[x].isDoubtful();
 #pragma unroll
     for (int i = 0; i < kShare; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) doubtful |= isDoubtfulSum(sum[i][e]);
     if (isAnyOfBlock(doubtful, flags)) {
+      // A sum that cancels has larger ones of its slices in it.
+      floatx4 largest[kShare];
 #pragma unroll
-      for (int i = 0; i < kShare; ++i)
+      for (int i = 0; i < kShare; ++i) {
+        const ldsfloat* at = (const ldsfloat*)lds + (wave - slice) * kTile + place(slice, i, lane);
+        largest[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int s = 0; s < S; ++s)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) again |= isUnfitSum(sum[i][e]);
+          for (int e = 0; e < 4; ++e) largest[i][e] = __builtin_fmaxf(largest[i][e], __builtin_fabsf(at[s * kTile + e]));
+      }
+      __syncthreads();
+      ldsfloat* const most = (ldsfloat*)lds + 128; // of the block's rows, of its columns (where partial sums were)
+      for (int i = lane + 64 * wave; i <= kRowsOfBlock + kColumnsOfBlock; i += 64 * GA * GB * S) most[i] = 0.0f; // (and the count behind them)
+      __syncthreads();
+#pragma unroll
+      for (int y = 0; y < TA; ++y) raiseTo(most + 16 * TA * ga + a.position(y, r), rangeA[y].most);
+#pragma unroll
+      for (int x = 0; x < TB; ++x) raiseTo(most + kRowsOfBlock + 16 * TB * gb + b.position(x, r), rangeB[x].most);
+      __syncthreads();
+      ldsint* const noted = (ldsint*)(most + kRowsOfBlock + kColumnsOfBlock);
+#pragma unroll
+      for (int i = 0; i < kShare; ++i) {
+        const int unit = tmin(slice * kShare + i, kUnits - 1) * 64 + lane;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          again |= isUnfitSum(sum[i][e]);
+          const int row = 16 * TA * ga + unit / kVectors, column = 16 * TB * gb + unit % kVectors * 4 + e;
+          if (isUnsureSum(largest[i][e], most[row], most[kRowsOfBlock + column])) note(noted, row * kColumnsOfBlock + column);
+        }
+      }
+      again = isAnyOfBlock(again, flags + 1);
+      doubtful = !again && *noted != 0;
+      if (doubtful && *noted <= kMostNoted) { // or larger terms
+        bool isSure = true;
+        for (int i = lane + 64 * wave; i < *noted; i += 64 * GA * GB * S) {
+          const int output = noted[1 + i], row = output / kColumnsOfBlock, column = output % kColumnsOfBlock;
+          const int m = tmin(m0 - 16 * TA * ga + row, M - 1), n = tmin(n0 - 16 * TB * gb + column, N - 1);
+          bool is = false;
+#pragma unroll
+          for (int j = 0; j < kSampledTerms; ++j) {
+            const int k = (i + j * (K / kSampledTerms | 1)) % K;
+            is |= !isUnsureSum(pA[AKInner ? m * K + k : k * M + m] * pB[BKInner ? n * K + k : k * N + n], most[row], most[kRowsOfBlock + column]);
+          }
+          isSure &= is;
+        }
+        doubtful = isAnyOfBlock(!isSure, flags + 2);
+      }
+    } else {
+      doubtful = false;
+    }
+    if (doubtful) {
 #pragma unroll 1
       for (int t = 0; t < kTurns; ++t) {
         const int k0 = 32 * (slice + t * S);
@@ -565,7 +670,7 @@ template <bool Bias, bool AKInner, bool BKInner, int M, int N, int K, int TA, in
         b.load(k0);
         again |= a.isUnfit() || b.isUnfit(); // (what lies behind the end of a row is of the next one: at worst a block too many computes again)
       }
-      again = isAnyOfBlock(again, flags + 1);
+      again = isAnyOfBlock(again, flags + 3);
     }
     if (again) {
       multiply<false>(a, b, slice, mine, rangeA, rangeB);
