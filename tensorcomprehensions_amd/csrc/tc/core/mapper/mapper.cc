@@ -486,6 +486,9 @@ SplitConvolutionShape bestSplitConvolution(const ConvolutionSizes& s, int64_t wa
     const int64_t channels = 8 * ceilDiv(ceilDiv(s.channels, chunks), 8);
     if (channels == last) continue;
     last = channels;
+    // (byte offsets are 32 bits, also those of channels behind the last one.  16 chunks of what LDS holds are 27 000 terms at most, and
+    // isUnsureSum counts on 65536.)
+    if (std::max(channels * s.height * s.width, (s.filters * s.channels + channels) * s.kernelHeight * s.kernelWidth) >= (int64_t(1) << 29)) continue;
     const int64_t octets = channels / 8, slots = s.kernelHeight * s.kernelWidth * octets, steps = ceilDiv(slots, 4), turns = ceilDiv(s.channels, channels);
     for (int64_t used = 4; used <= std::min<int64_t>(waves, 8); used *= 2) {
       for (int64_t filterTiles = 1; filterTiles <= std::min<int64_t>(8, ceilDiv(s.filters, 16)); ++filterTiles) {

@@ -242,3 +242,12 @@ def test_no_other_shared_memory_than_the_options_see(tmp_path, kernel):
     subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "--offload-device-only", "-O3", "-std=c++17", "-Xclang", "-target-feature",
                     "-Xclang", "-packed-fp32-ops", "-include", "hip/hip_runtime.h", "-w", "-S", "-o", str(assembly), str(path)], check=True)
     assert int(re.search(r"amdhsa_group_segment_fixed_size (\d+)", assembly.read_text()).group(1)) == declared
+
+
+@pytest.mark.parametrize("height,taken", [(1 << 18, True), (1 << 18 | 1 << 11, False)])
+def test_offsets_of_channels_that_do_not_exist(height, taken):
+    """Eight channels to a chunk: with five of them the offsets of the others stay below 2^31 bytes too."""
+    sizes = (1, 1, 5, 7, height, 255, (5, 5))
+    ins = operands(sizes, lambda *s: ShapeOnly(s))
+    text, _ = tc.map_only(DENSE, "f", ins, "naive;tile=1,16,1,16;mapToThreads=64,8;mapToBlocks=1000000,1000000,1000000;useMfma=1;useSharedMemory=1;useReadOnlyCache=1")
+    assert ("__tc::SplitConvolution<" in text.split('extern "C"')[-1]) == taken
