@@ -786,6 +786,10 @@ void takeProductsWhole(const KernelPlan& k, StagePlan& st, const HipMappingOptio
 // Sums of the columns of a float matrix, O(n) +=! A(r, n), whose threads keep whole sums, under tiles that leave three quarters of the
 // device's wavefronts out, go to __tc::columnSums (hip_column_sums.h): rows on other threads as well, whatever the options say about
 // unrolling.  (One axis of threads, one block a tile, no matchLibraryCalls, which has the rows on threads as it is.)
+// Beyond half as many tiles as compute units (8192 columns) one thread a column has the device half full, and two blocks of 16 columns, on different
+// XCDs, read every line of 128 bytes twice.  Of 200 sizes timed there these were slower and stay: few rows (64 x 12288 2.2 -> 2.4 us, 100 x 15360 2.6 -> 2.7),
+// whole tiles of a matrix that is more than half of the L2 caches but fits them (320 x 14336 5.0 -> 6.7, 512 x 12288 7.3 -> 8.6; 200 x 14336 4.0 -> 2.9 and
+// 1024 x 9216 20 -> 13.5 go), and other tiles on nearly all compute units (200 x 16001 5.8 -> 6.5; 200 x 15001 6.5 -> 4.9).
 constexpr int64_t kColumnSumWaves = 16;
 void takeColumnSums(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits, bool wide) {
   if (k.stages.size() != 1 || wide || st.atomic || o.generic.matchLibraryCallsValue || o.block.size() != 1 || !o.generic.hasTiling) return;
@@ -800,6 +804,11 @@ void takeColumnSums(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, co
   if (a.type != f32 || out.type != f32 || a.extents != std::vector<int64_t>{r.extent, n.extent} || out.extents != std::vector<int64_t>{n.extent}) return;
   const int64_t waves = n.numTiles * ceilDiv(std::min<int64_t>(static_cast<int64_t>(o.block[0]), n.tile), limits.wavefront);
   if (n.numTiles > allowedBlocks(o, 0, 0) || waves >= limits.computeUnits || r.extent < 4 * kColumnSumWaves || r.extent * n.extent >= (int64_t(1) << 29)) return;
+  if (2 * waves > limits.computeUnits) {
+    const bool whole = n.extent % n.tile == 0;
+    const int64_t mebibytes = r.extent * n.extent >> 18;
+    if (r.extent < (whole ? 128 : 80) || (whole ? mebibytes >= 16 && mebibytes < 36 : 16 * waves > 15 * limits.computeUnits)) return;
+  }
   if (limits.maxThreadsPerBlock < 64 * kColumnSumWaves) return;
   if (o.hasMaxSharedMemory && static_cast<int64_t>(o.maxSharedMemoryValue) < 4 * 64 * kColumnSumWaves) return;
   std::ostringstream ss;

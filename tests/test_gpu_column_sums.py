@@ -42,6 +42,15 @@ def test_column_sums(rows, columns):
     (SOURCE, 1024, 1024, OPTIONS + ";maxSharedMemory=4095", False),                 # the partial sums take 4 KiB of LDS
     (SOURCE, 1024, 1024, OPTIONS + ";maxSharedMemory=4096", True),
     (SOURCE, 1024, 1024, OPTIONS, True),
+    (SOURCE, 64, 8192, OPTIONS, True),
+    (SOURCE, 64, 8256, OPTIONS, False),                                             # few rows beside columns on more than half of the compute units
+    (SOURCE, 80, 8257, OPTIONS, True),
+    (SOURCE, 200, 14336, OPTIONS, True),
+    (SOURCE, 320, 14336, OPTIONS, False),                                           # lines read twice, from beyond the L2 caches
+    (SOURCE, 512, 12288, OPTIONS, False),
+    (SOURCE, 1024, 9216, OPTIONS, True),
+    (SOURCE, 200, 15001, OPTIONS, True),
+    (SOURCE, 200, 16001, OPTIONS, False),
 ])
 def test_which_sums_are_taken(source, rows, columns, options, taken):
     text, _ = tc.map_only(source, "f", [ShapeOnly((rows, columns))], options)
