@@ -760,7 +760,11 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
 // then (600 of 128x128x128 34.8 us in tiles, 51 whole; 1314 of 98x128x98 80 and 100; 600 of 128x32x128 12.7 and 15.4), where the
 // rows alone have two tiles and are more than 96 (700 of 128x64x64 13.5 and 14.4; 643 of 101x127x40 21.5 and 23.6) or the blocks are too few without them
 // (716 of 79x12x8 2.9 and 3.8; 586 of 81x18x37 5.5 and 6.1), and of fewer products (140 of 111x67x83 9.4 and 11.0).
-void takeProductsWhole(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, const DeviceLimits& limits) {
+// They stay too where the blocks have fewer than eight wavefronts a compute unit between them (blocks of two: 998 of 60x9x114 9.4 and 11.2, 694 of 79x2x82
+// 7.2 and 8.5; 1507 of 119x7x67 goes, 17.6 -> 16.7), with reductions of less than four points (1982 of 108x1x102 19.8 and 23.7), which leave little to
+// copy twice, and with 5 to 8 columns on four wavefronts (2233 of 85x7x5 4.4 and 6.8, nine of nine such; eight wavefronts 14.2 -> 8.3 for 1830 of 88x47x5).  Of
+// 231 others drawn with up to 48 points one is 14 % slower (861 of 95x7x104, 10.4 and 12.0) and none of the rest more than 3 %, 1.24 times as fast by geometric mean.
+void takeProductsWhole(const KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits) {
   constexpr int64_t kMostTiles = 49, kMostRows = 120, kMostRowsAlone = 96;
   if (k.stages.size() != 1 || st.mfmaBatch.size() != 1 || st.stmts.size() != 1 || !o.useSharedMemoryValue || o.prefetchSharedValue || st.atomic) return;
   if (st.vars.size() != 4 || st.numParallel != 3 || k.sharedDepth < 3) return;
@@ -773,7 +777,9 @@ void takeProductsWhole(const KernelPlan& k, StagePlan& st, const HipMappingOptio
   if (b.numTiles > allowedBlocks(o, 0, 0)) return;
   if (m.numTiles > 2 || n.numTiles > 2 || m.numTiles * n.numTiles == 1) return;
   if (ceilDiv(m.extent, 16) * ceilDiv(n.extent, 16) > kMostTiles || m.extent > kMostRows) return;
+  if (r.extent < 4 || b.extent * waves < 8 * limits.computeUnits) return;
   if (n.numTiles == 1 && (m.extent > kMostRowsAlone || b.extent < 3 * limits.computeUnits)) return;
+  if (n.numTiles == 1 && waves == 4 && n.extent > 4 && n.extent <= 8) return;
   int64_t lds = limits.ldsBytesPerBlock / 2;
   if (o.hasMaxSharedMemory) lds = std::min<int64_t>(lds, o.maxSharedMemoryValue);
   if (4 * r.extent * (m.extent + n.extent + 8) > lds) return;
@@ -981,7 +987,7 @@ void mapKernel(KernelCtx& kc, const DeviceLimits& limits) {
     if (st.mfma) takeLargeHalfProduct(k, st, o, waves, limits, kc.wide);
     if (!st.largeHalfProduct.empty()) return;
     if (st.mfma) fillComputeUnits(k, st, o, waves, limits.computeUnits);
-    if (st.mfma) takeProductsWhole(k, st, o, limits);
+    if (st.mfma) takeProductsWhole(k, st, o, waves, limits);
     if (st.mfma) takeSlicedProduct(k, st, o, waves, limits, kc.wide);
     if (st.mfma) takeSplitConvolution(k, st, o, waves, limits, kc.wide);
     if (!st.splitConvolution.empty()) return;
