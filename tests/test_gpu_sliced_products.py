@@ -30,33 +30,49 @@ def run(m, n, k, a_inner, b_inner, a, b, bias=None):
     return out.cpu()
 
 
-SIZES = [
-    (1000, 1000, 1000),     # 64 x 64 outputs a block, the last step of eight points
-    (691, 792, 1840),
-    (254, 292, 1500),       # 16 x 32
-    (655, 1031, 545),       # one point in the last step, an odd number of columns
-    (45, 2516, 2699),       # fewer rows than a tile of 48 has
-    (986, 71, 1987),
-    (497, 681, 1530),       # 64 x 32
-    (2048, 2048, 160),      # an odd number of steps for two slices; taken with both reductions outermost
-    (2062, 1895, 768),      # 128 x 128, four rectangles of wavefronts
+# whether the reduction is innermost in the first operand, in the second one, and whether a bias is added
+ORDERS = {"mk,kn": (True, False, False), "mk,nk": (True, True, True), "km,kn": (False, False, False), "km,nk": (False, True, True)}
+SIZES = [  # sizes, orders of the operands in which they are taken, tiles of a wavefront, wavefronts and slices
+    (1000, 1000, 1000, "mk,kn mk,nk km,kn km,nk", "4, 4, 1, 1, 8"),  # 64 x 64 outputs a block, the last step of eight points
+    (691, 792, 1840, "mk,kn mk,nk km,kn km,nk", "4, 4, 1, 1, 8"),
+    (254, 292, 1500, "mk,kn km,kn", "1, 2, 1, 1, 8"),                # 16 x 32
+    (655, 1031, 545, "mk,kn km,kn km,nk", "4, 4, 1, 1, 8"),          # one point in the last step, an odd number of columns
+    (45, 2516, 2699, "mk,kn km,kn km,nk", "1, 2, 1, 1, 8"),          # fewer rows than a tile of 48 has
+    (986, 71, 1987, "mk,kn km,kn", "1, 2, 1, 1, 8"),
+    (497, 681, 1530, "mk,kn km,kn km,nk", "4, 2, 1, 1, 8"),          # 64 x 32
+    (617, 467, 6106, "mk,nk", "4, 2, 1, 1, 8"),
+    (2048, 2048, 160, "km,kn", "4, 4, 2, 2, 2"),                     # an odd number of steps for two slices
+    (2062, 1895, 768, "mk,kn mk,nk km,kn km,nk", "4, 4, 2, 2, 2"),   # 128 x 128, four rectangles of wavefronts
+    (451, 349, 996, "km,nk", "2, 2, 1, 1, 8"),
+    (1171, 37, 2759, "km,nk", "1, 1, 1, 1, 8"),                      # fewer outputs to a slice than a wavefront has lanes
+    (907, 2194, 798, "km,nk", "2, 4, 1, 1, 4"),
+    (1401, 1122, 366, "km,nk", "4, 2, 1, 2, 4"),                     # two rectangles side by side
 ]
+TAKEN = [(*size[:3], order) for size in SIZES for order in size[3].split()]
+
+
+def mapped(m, n, k, order):
+    a_inner, b_inner, bias = ORDERS[order]
+    shapes = [(m, k) if a_inner else (k, m), (n, k) if b_inner else (k, n)] + ([(n,)] if bias else [])
+    text, _ = tc.map_only(source(a_inner, b_inner, bias), "f", [ShapeOnly(s) for s in shapes], options(m, n))
+    return text.split('extern "C"')[-1]
+
+
+@pytest.mark.parametrize("m,n,k,orders,tiles", SIZES)
+def test_shapes_of_the_sizes_below(m, n, k, orders, tiles):
+    for order in orders.split():
+        assert f"{m}, {n}, {k}, {tiles}>" in mapped(m, n, k, order)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("a_inner,b_inner,bias", [(True, False, False), (True, True, True), (False, False, False), (False, True, True)])
-@pytest.mark.parametrize("m,n,k", SIZES)
-def test_sums(m, n, k, a_inner, b_inner, bias):
-    print(m, n, k, a_inner, b_inner, flush=True)
+@pytest.mark.parametrize("m,n,k,order", TAKEN)
+def test_sums(m, n, k, order):
+    print(m, n, k, order, flush=True)
+    a_inner, b_inner, bias = ORDERS[order]
     generator = torch.Generator().manual_seed(m)
     ints = lambda *s: torch.randint(-8, 9, s, generator=generator).float()  # noqa: E731
     a, b, c = ints(m, k), ints(n, k), ints(n)
-    try:
-        got = run(m, n, k, a_inner, b_inner, a, b, c if bias else None)
-    except AssertionError:
-        if (a_inner and not b_inner and k > 160) or not (a_inner or b_inner):
-            raise
-        pytest.skip("the general pipeline is as fast for this order of the operands")
+    got = run(m, n, k, a_inner, b_inner, a, b, c if bias else None)
     want = a.double() @ b.double().t()
     assert torch.equal(got.double(), want + c if bias else want)     # (sums of whole numbers are exact)
     a, b, c = (torch.randn(s, generator=generator) for s in ((m, k), (n, k), (n,)))
@@ -64,8 +80,30 @@ def test_sums(m, n, k, a_inner, b_inner, bias):
     want, magnitudes = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     if bias:
         want, magnitudes = want + c, magnitudes + c.abs()
-    # one rounding of 2^-24 a term and the bias, in whatever order, and 2^-26 of every product for the parts left out
+    # one rounding of 2^-24 a term and the bias, in whatever order, and up to 2^-24 of every product for the parts left out
     assert ((got - want).abs() <= (k + 2) * 2.0 ** -24 * magnitudes).all()
+    # Roundings do not add up like that: 0.7e-7 to 2.9e-7 here.  Without any one of the six products of parts it is 2.4e-6 or more.
+    assert (got - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,order", TAKEN)
+def test_every_product_of_parts(m, n, k, order):
+    """Sums of 24 bits, which are exact only with all six products of parts: values 1 + y 2^-9 + z 2^-18 (y, z of -1, 0, 1) in 24 points a row."""
+    a_inner, b_inner, bias = ORDERS[order]
+    generator = torch.Generator().manual_seed(k)
+
+    def values(rows, low):
+        x, y, z = (torch.randint(-1, 2, (rows, k), generator=generator).float() for _ in range(3))
+        return x * (1 + y * 2.0 ** -9 + (z * 2.0 ** -18 if low else 0))
+
+    points = torch.zeros(k)
+    points[torch.randperm(k, generator=generator)[:24]] = 1.0
+    for low_a, low_b, middle in ((True, False, False), (False, True, False), (False, False, True)):
+        a = values(m, low_a) * points if low_a or middle else torch.randint(-1, 2, (m, k), generator=generator) * points
+        b = values(n, low_b) if low_b or middle else torch.randint(-1, 2, (n, k), generator=generator).float()
+        got = run(m, n, k, a_inner, b_inner, a, b, torch.zeros(n) if bias else None)
+        assert torch.equal(got.double(), a.double() @ b.double().t())
 
 
 @pytest.mark.gpu
@@ -155,17 +193,13 @@ def test_small_values_beside_others(m, n, k, tiles, case):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("a_inner,b_inner,bias", [(True, False, False), (True, True, True), (False, False, False), (False, True, True)])
-@pytest.mark.parametrize("m,n,k", [(1000, 1000, 1000), (254, 292, 1500), (655, 1031, 545), (2062, 1895, 768)])
-def test_sums_of_floats_themselves(m, n, k, a_inner, b_inner, bias):
+@pytest.mark.parametrize("m,n,k,order", [t for t in TAKEN if t[:3] in [(1000, 1000, 1000), (254, 292, 1500), (655, 1031, 545), (2062, 1895, 768)]])
+def test_sums_of_floats_themselves(m, n, k, order):
     """Blocks that compute again, with every order of the operands: an infinity and a NaN reach their row and column alone, also where the last step
     has fewer points, and denormal operands keep their sums."""
+    a_inner, b_inner, bias = ORDERS[order]
     generator = torch.Generator().manual_seed(4)
     a, b, c = (torch.randn(s, generator=generator) for s in ((m, k), (n, k), (n,)))
-    text, _ = tc.map_only(source(a_inner, b_inner, bias), "f", [ShapeOnly((m, k) if a_inner else (k, m)), ShapeOnly((n, k) if b_inner else (k, n))] +
-                          ([ShapeOnly((n,))] if bias else []), options(m, n))
-    if "__tc::SlicedProduct<" not in text.split('extern "C"')[-1]:
-        pytest.skip("the general pipeline is as fast for this order of the operands")
     for scale in (1.0, 2.0 ** -125):
         x, y = a * scale, b.clone()
         if scale == 1.0:

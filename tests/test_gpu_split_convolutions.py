@@ -94,9 +94,28 @@ def test_sums(sizes):
     ins = operands(sizes, lambda *s: torch.randn(s, generator=generator))
     got = run(source, sizes, ins).double()
     want, magnitudes = reference(sizes, ins)
-    # one rounding of 2^-24 a term and the bias, in whatever order, and 2^-26 of every product for the parts left out
+    # one rounding of 2^-24 a term and the bias, in whatever order, and up to 2^-24 of every product for the parts left out
     terms = sizes[2] * sizes[6][0] * sizes[6][1]
     assert ((got.reshape(want.shape) - want).abs() <= (terms + 2) * 2.0 ** -24 * magnitudes).all()
+    # Roundings do not add up like that: 0.5e-7 to 1.7e-7 here.  Without any one of the six products of parts it is 2.4e-6 or more.
+    assert (got.reshape(want.shape) - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", SIZES, ids=lambda s: "x".join(map(str, s[:6])))
+def test_every_product_of_parts(sizes):
+    """Sums of 24 bits, which are exact only with all six products of parts: values 1 + y 2^-9 + z 2^-18 (y, z of -1, 0, 1) in a few channels and places."""
+    source = DENSE if sizes[1] == 1 else GROUPS
+    generator = torch.Generator().manual_seed(sizes[2])
+    signs = lambda *s: torch.randint(-1, 2, s, generator=generator).float()  # noqa: E731
+    x, weights, bias = operands(sizes, signs)
+    places = torch.zeros(weights[0].numel() if sizes[1] == 1 else weights[0, 0].numel())
+    places[torch.randperm(places.numel(), generator=generator)[:24]] = 1.0
+    weights, bias = weights * places.view(weights.shape[-3:]), 0 * bias
+    middle = lambda t: t * (1 + signs(*t.shape) * 2.0 ** -9)  # noqa: E731
+    low = lambda t: t * (1 + signs(*t.shape) * 2.0 ** -9 + signs(*t.shape) * 2.0 ** -18)  # noqa: E731
+    for ins in ([low(x), weights, bias], [x, low(weights), bias], [middle(x), middle(weights), bias]):
+        assert torch.equal(run(source, sizes, ins).reshape(-1).double(), reference(sizes, ins)[0].reshape(-1))
 
 
 @pytest.mark.gpu
