@@ -5,13 +5,16 @@ namespace tc {
 namespace hip {
 
 // A float as the sum of three bf16 values: its nearest bf16, the nearest bf16 of what is left, and the rest, which
-// has at most 8 bits; the differences are exact, so the sum is the float.  A product of floats is six products of such parts
-// (high * high, the two of high * middle, middle * middle, the two of high * low); each is exact in float, and what
-// the other three would add is below 2^-26 of the product, less than half the rounding of one float addition.
+// has at most 8 bits; the differences are exact, so the sum is the float (Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence
+// Datatype For Higher-Precision Computations", ARITH 2019).  A product of floats is six products of such parts
+// (high * high, the two of high * middle, middle * middle, the two of high * low), each exact in float.  What the other three would
+// add is at most 2^-24 of the product (both factors just above a power of two, as 0x1.00ff8p0), a rounding of it; for normal deviates it is 6e-9 of a sum
+// of 1000 terms, a thirtieth of the roundings below.
 // v_mfma_f32_16x16x32_bf16 does 16 times the work of v_mfma_f32_16x16x4_f32 a cycle, so six of them still are 2.7
-// times as fast; an output's chain of additions gets shorter as well (32 products to an instruction), and the five small
-// products have an accumulator of their own, whose roundings are those of a sum 2^-8 as large.  Error against 64 bits, normal
-// deviates, 2-norm: 96, 992 and 4096 terms 0.6e-7, 1.8e-7, 3.9e-7 (float instruction 1.8e-7, 5.6e-7, 11.5e-7).
+// times as fast; an output's chain of additions gets shorter as well (32 products to an instruction), and in convolutions and in products of fewer than 16 tiles
+// a wavefront the five small products have an accumulator of their own, whose roundings are those of a sum 2^-8 as large.
+// Error against 64 bits, normal deviates, 2-norm: convolutions of 111, 576 and 837 terms 0.7e-7, 1.4e-7 and 1.7e-7; products of 1500 terms in eight slices 1.0e-7; with
+// one accumulator 1.6e-7 (1000 terms, eight slices) and 2.9e-7 (768 terms, two slices).  (Float instruction: 96, 992 and 4096 terms 1.8e-7, 5.6e-7, 11.5e-7.)
 //
 // What the parts cannot hold is computed again on the float instruction, block by block, from the same tiles (one infinity: 1000^3 16.5 -> 39.2 us,
 // the convolution below 30.3 -> 61.9):
