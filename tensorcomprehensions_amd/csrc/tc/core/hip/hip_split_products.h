@@ -28,7 +28,10 @@ namespace hip {
 //    looks at its sums beside the largest values of their row and column (of the window and the filters).  A sum that is still too small may be one
 //    of larger terms that cancelled, as the slices of a product and a few of the terms can tell, or of small values alone, whatever stands
 //    beside them: where that is left open the block looks its operands over for values other than zero below 2^-110.
-// The check costs half an instruction a value; one for every value's own exponent cost 1.5, and 1000^3 20.7 us for 17.4.
+// The check costs half an instruction a value; one for every value's own exponent cost 1.5, and 1000^3 20.7 us for 17.4.  What follows a doubt, 1000^3 and the
+// convolution below, 16.5 and 30 us: a row of zeros 18.3 and 29.6, all values 1e-20 18.9 and 30.0, a row of 1e10 18 and 29, an infinity 34.8 and 59.6, all values
+// 1e-40 33 and 62 (23 and 41 us in the general pipeline, whatever the values); 2048^3 with every 16th point of an operand of whole numbers other than zero looks its
+// operands over, 158 us for 103.
 constexpr const char* kDeviceSplitParts = R"HIP(
 namespace __tc {
 typedef __attribute__((address_space(3))) char ldschar;
@@ -109,12 +112,12 @@ __device__ __forceinline__ constexpr int splitPartB(int q) { return q == 2 ? 2 :
 // a weight's place in the window, in 16 bytes, three such planes.  A step of the matrix instruction multiplies
 // four of those: a lane group reads its eight channels of a pixel at its own place of the window, whatever place that
 // is.  WF x WP wavefronts divide the filters and the pixels; a lane ends up with four consecutive pixels of a filter.
-// Rows of pixels and of weights are an odd number of 16-byte units apart: no bank conflicts.
+// Rows of pixels and of weights are an odd number of 16-byte units apart, which leaves the conflicts between the lane groups of a read.
 //
 // What bounds it, at 16 x 64 x 57 x 57, 64 filters 3 x 3 (24 x 2 tiles, chunks of 16, 1 x 8 wavefronts, one block a compute
-// unit): 28 to 30 us (on the float instruction 41 to 44, whose matrix cores alone take 23): 14.4 us of matrix instructions (an eighth of them
-// for steps that do not exist: 18 places of eight channels in five steps), 9 of LDS reads, 3 of splitting, in turn at the
-// barriers of a chunk, one block being all that fits.  Two smaller blocks a compute unit instead 33 to 37 us, a chunk of 8
+// unit): 27 to 30 us (on the float instruction 41 to 44, whose matrix cores alone take 23), by counters 60 600 cycles: 23 000 of matrix
+// instructions (38 %; a tenth of them for steps that do not exist: 18 places of eight channels in five steps), 23 000 of LDS instructions and 11 400
+// of bank conflicts, 16 700 of vector instructions, in turn at the barriers of a chunk, one block being all that fits.  Two smaller blocks a compute unit instead 33 to 37 us, a chunk of 8
 // channels 33 (a third of its steps do not exist), four wavefronts 31 to 35, operands requested a step ahead by hand 32 and more (spills).
 constexpr const char* kDeviceSplitConvolution = R"HIP(
 namespace __tc {
@@ -399,9 +402,9 @@ template <bool Bias, int N, int G, int C, int F, int H, int W, int KH, int KW, i
 // columns is loaded and split once a block, and a sum is S short chains.  The partial tiles meet in LDS, are added and
 // stored in 256-byte runs.
 //
-// What bounds it at 1000^3 (64 x 64 outputs a block, 8 slices, one block a compute unit; 17.4 us, 23.4 in the general pipeline, whose matrix
-// cores alone take 13.3): the 11 us of splitting and multiplying, which one wavefront's instructions cannot overlap beyond two
-// vector instructions a multiplication, the first loads (2 us), the sums' way through LDS and the launch.
+// What bounds it at 1000^3 (64 x 64 outputs a block, 8 slices, one block a compute unit; 16.5 to 17 us, 23.4 in the general pipeline, whose matrix
+// cores alone take 13.3): by counters 35 100 cycles, 12 300 of matrix instructions (35 %) and 17 900 of vector instructions, which one wavefront's
+// instructions cannot overlap beyond two vector instructions a multiplication, the first loads (2 us), the sums' way through LDS and the launch.
 // Operands laid in LDS as parts and shared by the wavefronts of a block: 22.4 us there, 92 at 2048^3 (here 89, given tiles
 // 126.7): the same work behind barriers.  Parts through v_dot2_f32_bf16 save a third of the vector instructions, but it occupies the
 // matrix cores.  Steps two ahead in registers, parts of the next step made under the multiplications of this one: 18.2 to 25.

@@ -541,7 +541,7 @@ double givenConvolutionMicroseconds(const StagePlan& st, size_t rank, const Conv
 }
 
 void takeSplitConvolution(KernelPlan& k, StagePlan& st, const HipMappingOptions& o, int64_t waves, const DeviceLimits& limits, bool wide) {
-  // (its results are written through, which is a matter of useReadOnlyCache)
+  // (useReadOnlyCache: options without it keep the given tiles)
   if (k.stages.size() != 1 || wide || waves < 4 || !o.useSharedMemoryValue || !o.useReadOnlyCacheValue || st.atomic || st.stmts.size() > 2 || !st.stmts[0].init) return;
   const size_t rank = st.lhsSubs.size(); // n, (g,) f, h, w
   if ((rank != 4 && rank != 5) || st.numParallel != static_cast<int>(rank) || st.vars.size() != rank + 3) return;
@@ -641,8 +641,10 @@ void takeSplitConvolution(KernelPlan& k, StagePlan& st, const HipMappingOptions&
 // as before, 1250 x 208 x 1015 14.6 us for 10.8): 1000^3 22 -> 17 us, 45 x 2516 x 2699 27.1 -> 13.5, 1250 x 1015 x 208 14.5 -> 10.3,
 // 2048^3 126 -> 93 (rows, points, columns); 251 products drawn over these ranges and taken: 1.27 times as fast, the worst 6 % slower.
 // Tiles that were fitted to the device stay as they are, and are taken where the sliced form has their shape.  The general
-// pipeline keeps products of fewer than 1.06e8 multiplications or 128 reduction points and those whose tiles leave two compute units of three
-// idle.
+// pipeline keeps products of fewer than 1.06e8 multiplications (28 timed down to 2e7: 0.78 to 1.54 times as fast sliced, 0.99 on average, which the
+// estimate does not tell apart) or 128 reduction points (19 from 62 on: 0.80 to 1.25, 1.05), and those whose tiles leave two compute units of three
+// idle, which the estimate was not fitted to (20 timed since: 1.14 to 2.97 times as fast sliced, 1.65 on average; 138 x 9294 x 128 46 and 22 us).
+// Blocks of eight wavefronts and prefetchShared are what the stored options of such products say; others keep the given tiles.
 struct SlicedProductShape {
   int64_t rowTiles = 0, columnTiles = 0, rowWaves = 0, columnWaves = 0, slices = 0, lds = 0;
   double microseconds = 0;
@@ -693,7 +695,7 @@ void takeSlicedProduct(KernelPlan& k, StagePlan& st, const HipMappingOptions& o,
     if (bias.empty()) return;
   }
   const double multiplications = 1.0 * m.extent * n.extent * r.extent;
-  if (multiplications < 1.06e8 || r.extent < 128 || r.extent > 65536) return;  // (longer sums are not what isUnfitSum counts on)
+  if (multiplications < 1.06e8 || r.extent < 128 || r.extent > 65536) return;  // (longer sums are not what isUnsureSum counts on)
   // a block for every tile of these sizes?
   auto isOneBlockATile = [&](int64_t rows, int64_t columns) {
     int axis = 0;
